@@ -16,7 +16,7 @@ from pathlib import Path
 import torch  # noqa: F401  -- must be imported before the HIP library is loaded
 
 LIB_PATH = Path(__file__).resolve().parent / "libminiserve_amd.so"
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 # name -> (restype, argtypes); mirrors include/miniserve_amd.h.
 SIGNATURES: dict[str, tuple[object, list[object]]] = {
@@ -97,6 +97,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
     "msa_sample_workspace_size": (c_size_t, [c_int64, c_int64]),
     "msa_sample": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
+         c_void_p, c_size_t, c_void_p],
+    ),
+    "msa_sample_ranked": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
          c_void_p, c_size_t, c_void_p],

@@ -291,7 +291,24 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(SampArgs a) {
 //     ascending (masses in 2^-44 fixed point, exact 64-bit sums, as the whole-row path), and the
 //     exponential race over the final set -- noise read at the kept indices only. A row whose
 //     chunks held more than kCandCap candidates each (long runs of equal values), or whose top-k
-//     is outside (0, kTopKFast], takes the whole-row path instead.
+//     lies in (kTopKFast, vocab), takes the whole-row path instead.
+//
+// Rows without top-k (temperature alone, or top-p alone) are spread over the same chunks, with two
+// launches between those two. On the whole-row path such a row is read ten times by the one
+// workgroup that has it, and 32 of them among 64 kept the finishing kernel busy for 1,890 us
+// while most of the chip idled; the passes below take 65 us (17 + 10 + 22 + 17) for the same batch.
+//  1. sample_chunk_kernel writes the chunk's largest logit and, with top-p, a histogram of the
+//     softmax mass over kMassBins value bins (z falling in steps of 1 / kBinsPerUnit from the chunk
+//     maximum; masses exp(z - chunk max) in 2^-40 fixed point: exact sums, so atomics in any order).
+//  2. sample_cut_kernel, one workgroup per row: the row maximum, the chunks' histograms scaled to it
+//     and added in chunk order, and the bin where the mass at or below it passes (1 - p) of the total.
+//  3. sample_race_kernel, one workgroup per (row, chunk): every entry above that bin is kept and
+//     runs the race exp(z - m) / noise here; the entries inside the bin go to the chunk's
+//     candidate list. Logits and noise are each read once, coalesced.
+//  4. sample_finish_kernel decides the bin's entries one value at a time (mass at or below each in
+//     2^-40 fixed point, as the top-k rows) and joins their race with the chunks' winners.
+// A row with a NaN, without a finite maximum, with a temperature that is not positive, or with more
+// entries in the cut's bin than the lists hold takes the whole-row path.
 constexpr int kCandThreads = 256;
 constexpr int kCandPerThread = 40;
 constexpr int kCandChunk = kCandThreads * kCandPerThread;  // logits per chunk workgroup
@@ -299,6 +316,10 @@ constexpr int kTopKFast = 256;
 constexpr int kCandCap = 512;       // candidates kept per chunk
 constexpr int kFinishCap = 8192;    // candidates the finishing workgroup takes per row (LDS)
 constexpr int kMaxChunks = 64;      // chunks per row the finishing workgroup gathers (vocab <= 655,360)
+constexpr int kMassBins = 512;      // value bins of a chunk's mass histogram (the slot's list space holds it)
+constexpr float kBinsPerUnit = 16.f;  // bins per unit of z: 32 units below the maximum, past which e^-32 < 2^-40
+constexpr int kWideCap = kCandCap - 8;  // in-bin entries kept per chunk (the row's WideRow ends chunk 0's slot)
+constexpr int kCntWhole = -1, kCntOver = -2, kCntWide = -3;  // cand_cnt of a slot without a list
 constexpr int kFinishThreads = 256;  // (a row that falls back runs the whole-row path on these too)
 static_assert(kCandThreads == 256 && kFinishThreads == 256, "the bounds take the k-th largest of 256 thread maxima");
 static_assert(kMaxChunks == 64, "the finishing workgroup reads one chunk count per lane of a wavefront");
@@ -306,13 +327,33 @@ static_assert(kCandPerThread < 64, "a thread's candidate count fits six bits");
 
 struct CandArgs {
   SampArgs a;
-  int chunks;          // chunk workgroups per row
-  uint32_t* cand_key;  // [rows][chunks][kCandCap]
-  int32_t* cand_idx;   // [rows][chunks][kCandCap]
-  int32_t* cand_cnt;   // [rows][chunks]: candidates, or -1 (row not chunked) / -2 (over kCandCap)
-  float* arg_val;      // [rows][chunks]: greedy rows' chunk maximum
-  int32_t* arg_idx;    // [rows][chunks]: and its first index (0x7fffffff: none)
+  int chunks;         // chunk workgroups per row
+  int wide;           // rows without top-k run over the chunks too (else: the whole-row path)
+  uint32_t* cand;     // [rows][chunks] slots of kCandCap keys, then kCandCap indices
+  int32_t* cand_cnt;  // [rows][chunks]: candidates, or kCntWhole / kCntOver (over the cap) / kCntWide
+  float* arg_val;     // [rows][chunks]: chunk maximum of greedy rows and rows without top-k; the latter's best score
+  int32_t* arg_idx;   // [rows][chunks]: the first index with that maximum or score (0x7fffffff: none)
+
+  __device__ uint32_t* keys(int64_t slot) const { return cand + slot * (2 * kCandCap); }
+  __device__ int32_t* idxs(int64_t slot) const { return (int32_t*)(cand + slot * (2 * kCandCap) + kCandCap); }
+  __device__ unsigned long long* mass(int64_t slot) const { return (unsigned long long*)keys(slot); }
 };
+
+// What sample_cut_kernel found for a row without top-k, in the last 32 bytes of its chunk 0's slot
+// (written once the histogram there has been read; the lists of kWideCap entries end before it).
+enum { WIDE_NO = 0, WIDE_CUT = 1, WIDE_ALL = 2 };
+struct WideRow {
+  float m;    // the row's largest z
+  int state;  // WIDE_NO: the whole-row path; WIDE_ALL: every entry is kept
+  int cut;    // WIDE_CUT: bins below m's (0 = m's own) of the bin the cut lies in
+  int pad;
+  unsigned long long below;  // mass under that bin
+  double target;             // an entry is kept when the mass at or below it exceeds this
+};
+static_assert(sizeof(WideRow) == 4 * (kCandCap - kWideCap) && kMassBins * 8 == 2 * kCandCap * 4, "slot layout");
+__device__ __forceinline__ WideRow* wide_row(const CandArgs& c, int64_t row) {
+  return (WideRow*)(c.idxs(row * c.chunks) + kWideCap);
+}
 
 __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
@@ -332,6 +373,17 @@ __device__ __forceinline__ bool take_rows_chunked(const SampArgs& a, int64_t row
   const int64_t k = *(a.top_k ? a.top_k + row : &kDefaultTopK);
   *k_out = k;
   return k > 0 && k <= kTopKFast && k < a.vocab;
+}
+// Rows without top-k (k as take_rows_chunked returned it).
+__device__ __forceinline__ bool no_top_k(const SampArgs& a, int64_t k) { return k <= 0 || k >= a.vocab; }
+// The bin of z below the one of the row maximum (fbm = wide_bin of it); monotonic in z, so a bin holds
+// every entry of its values.
+__device__ __forceinline__ float wide_bin(float z) { return floorf(z * kBinsPerUnit); }
+// e in [0, 1] in 2^-40 fixed point, truncated: two exact 20-bit steps, cheaper than a 64-bit conversion.
+__device__ __forceinline__ unsigned long long mass_fixed(float e) {
+  const float a = e * 0x1p20f;
+  const uint32_t hi = (uint32_t)a;
+  return ((unsigned long long)hi << 20) + (uint32_t)((a - (float)hi) * 0x1p20f);
 }
 
 // Inclusive suffix sum over the lanes of a wavefront: lane l gets the sum over lanes >= l.
@@ -564,13 +616,58 @@ __device__ __forceinline__ uint32_t wg_prefix_small(uint32_t v, uint32_t* s_wave
   return before + ex;
 }
 
+// A chunk of a row without top-k: its largest logit and, with top-p, its mass histogram (s_hist:
+// kMassBins, cleared here).
+__device__ __forceinline__ void wide_chunk(const CandArgs& c, int64_t row, int64_t slot,
+                                           const float (&vals)[kCandPerThread], int n, unsigned long long* s_hist,
+                                           float* s_red, int* s_bad) {
+  const int tid = threadIdx.x;
+  const float t = row_temperature(c.a, row), p = row_top_p(c.a, row);
+  float mx = -INFINITY;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < kCandPerThread; ++i)
+    if (i * kCandThreads + tid < n) {
+      bad |= vals[i] != vals[i];
+      mx = fmaxf(mx, vals[i]);
+    }
+  mx = wave_max(mx);
+  const bool wbad = __any(bad);
+  if ((tid & 63) == 0) {
+    s_red[tid >> 6] = mx;
+    s_bad[tid >> 6] = wbad;
+  }
+  for (int b = tid; b < kMassBins; b += kCandThreads) s_hist[b] = 0ull;
+  __syncthreads();
+  mx = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+  const float mc = mx / t;
+  const bool ok = !(s_bad[0] | s_bad[1] | s_bad[2] | s_bad[3]) && t > 0.f &&
+                  (mx == -INFINITY || isfinite(mc * kBinsPerUnit));
+  if (tid == 0) {
+    c.arg_val[slot] = mx;
+    c.cand_cnt[slot] = ok ? kCntWide : kCntWhole;
+  }
+  if (!ok || !(p < 1.0f) || mx == -INFINITY) return;  // uniform
+  const float fbc = wide_bin(mc);
+#pragma unroll
+  for (int i = 0; i < kCandPerThread; ++i) {
+    const float z = vals[i] / t;
+    const unsigned long long w = mass_fixed(expf(z - mc));
+    if (i * kCandThreads + tid < n && w != 0ull)  // (z more than 32 below the maximum has no mass: no bin past the last)
+      atomicAdd(&s_hist[(int)fminf(fbc - wide_bin(z), (float)(kMassBins - 1))], w);
+  }
+  __syncthreads();
+  unsigned long long* h = c.mass(slot);
+  for (int b = tid; b < kMassBins; b += kCandThreads) h[b] = s_hist[b];
+}
+
 __global__ __launch_bounds__(kCandThreads) void sample_chunk_kernel(CandArgs c) {
   __shared__ __attribute__((aligned(16))) uint32_t s_tmax[kCandThreads];
   __shared__ uint32_t s_scan[kCandThreads / 64];
   __shared__ uint32_t s_sel[2];
   __shared__ float fred[kCandThreads / 64];
   __shared__ int ired[kCandThreads / 64];
-  __shared__ uint32_t s_ck[kCandThreads / 64][kCandCap];
+  __shared__ __attribute__((aligned(16))) uint32_t s_ck[kCandThreads / 64][kCandCap];
   __shared__ int32_t s_ci[kCandThreads / 64][kCandCap];
   const SampArgs& a = c.a;
   const int64_t row = blockIdx.y;
@@ -611,7 +708,8 @@ __global__ __launch_bounds__(kCandThreads) void sample_chunk_kernel(CandArgs c) 
   }
   int64_t k;
   if (!take_rows_chunked(a, row, &k)) {
-    if (tid == 0) c.cand_cnt[slot] = -1;
+    if (c.wide && no_top_k(a, k)) wide_chunk(c, row, slot, vals, n, (unsigned long long*)s_ck, fred, ired);
+    else if (tid == 0) c.cand_cnt[slot] = kCntWhole;
     return;
   }
   const float t = row_temperature(a, row);
@@ -661,12 +759,12 @@ __global__ __launch_bounds__(kCandThreads) void sample_chunk_kernel(CandArgs c) 
   __syncthreads();
   const uint32_t o1 = s_scan[0], o2 = o1 + s_scan[1], o3 = o2 + s_scan[2], all = o3 + s_scan[3];
   if (all > (uint32_t)kCandCap) {
-    if (tid == 0) c.cand_cnt[slot] = -2;
+    if (tid == 0) c.cand_cnt[slot] = kCntOver;
     return;
   }
   // The wavefronts' runs one after another, written out coalesced.
-  uint32_t* ck = c.cand_key + slot * kCandCap;
-  int32_t* ci = c.cand_idx + slot * kCandCap;
+  uint32_t* ck = c.keys(slot);
+  int32_t* ci = c.idxs(slot);
   for (uint32_t j = tid; j < all; j += kCandThreads) {
     const int src = j >= o3 ? 3 : j >= o2 ? 2 : j >= o1 ? 1 : 0;
     const uint32_t at = j - (src == 3 ? o3 : src == 2 ? o2 : src == 1 ? o1 : 0u);
@@ -674,6 +772,176 @@ __global__ __launch_bounds__(kCandThreads) void sample_chunk_kernel(CandArgs c) 
     ci[j] = s_ci[src][at];
   }
   if (tid == 0) c.cand_cnt[slot] = (int32_t)all;
+}
+
+// Row maximum and top-p cut bin of a row without top-k from its chunks' maxima and histograms.
+__global__ __launch_bounds__(kCandThreads) void sample_cut_kernel(CandArgs c) {
+  constexpr int NT = kCandThreads;
+  static_assert(kMassBins == 2 * NT, "two bins per thread");
+  __shared__ float s_red[4];
+  __shared__ int s_ok[4], s_off[NT];
+  __shared__ double s_scale[NT];
+  __shared__ unsigned long long s_wave[4], s_below;
+  __shared__ int s_cut;
+  const SampArgs& a = c.a;
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int64_t slot0 = row * c.chunks;
+  int64_t k;
+  if (take_rows_chunked(a, row, &k) || !no_top_k(a, k) || (a.greedy && a.greedy[row])) return;
+  const float t = row_temperature(a, row), p = row_top_p(a, row);
+  float mx = -INFINITY;
+  bool ok = true;
+  for (int ch = tid; ch < c.chunks; ch += NT) {
+    mx = fmaxf(mx, c.arg_val[slot0 + ch]);
+    ok &= c.cand_cnt[slot0 + ch] == kCntWide;
+  }
+  mx = wave_max(mx);
+  const bool wok = __all(ok);
+  if (lane == 0) {
+    s_red[w] = mx;
+    s_ok[w] = wok;
+  }
+  if (tid == 0) {
+    s_cut = 0;  // no bin passes the target (p <= 0): only the largest value is kept
+    s_below = 0ull;
+  }
+  __syncthreads();
+  mx = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+  const float m = mx / t;
+  WideRow* out = wide_row(c, row);
+  if (!(s_ok[0] & s_ok[1] & s_ok[2] & s_ok[3]) || !isfinite(m)) {
+    if (tid == 0) out->state = WIDE_NO;
+    return;
+  }
+  if (!(p < 1.0f)) {
+    if (tid == 0) {
+      out->m = m;
+      out->state = WIDE_ALL;
+    }
+    return;
+  }
+  const float fbm = wide_bin(m);
+  double sum[2] = {0.0, 0.0};
+  for (int c0 = 0; c0 < c.chunks; c0 += NT) {  // chunks in order: the sums are deterministic
+    const int nc = min(NT, c.chunks - c0);
+    __syncthreads();
+    if (tid < nc) {
+      const float cm = c.arg_val[slot0 + c0 + tid], mc = cm / t;
+      const bool live = cm != -INFINITY && fbm - wide_bin(mc) < (float)kMassBins;
+      s_off[tid] = live ? (int)(fbm - wide_bin(mc)) : kMassBins;
+      s_scale[tid] = live ? exp((double)mc - (double)m) : 0.0;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int q = 0; q < nc; ++q) {
+      const int off = s_off[q];
+      if (off >= kMassBins) continue;  // uniform
+      const unsigned long long* h = c.mass(slot0 + c0 + q);
+      const int b0 = 2 * tid - off, b1 = b0 + 1;
+      const unsigned long long h0 = h[max(b0, 0)], h1 = h[max(b1, 0)];
+      sum[0] += b0 >= 0 ? (double)h0 * s_scale[q] : 0.0;
+      sum[1] += b1 >= 0 ? (double)h1 * s_scale[q] : 0.0;
+    }
+  }
+  const unsigned long long v0 = (unsigned long long)sum[0], v1 = (unsigned long long)sum[1];
+  // Mass of the bins of later threads (lower values), then the bin where the running mass passes.
+  unsigned long long incl = v0 + v1;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const unsigned long long o = __shfl_down(incl, off);
+    incl += lane + off < 64 ? o : 0ull;
+  }
+  if (lane == 0) s_wave[w] = incl;
+  __syncthreads();  // (every histogram of the row has been read: chunk 0's slot may be written)
+  unsigned long long later = incl - v0 - v1, tot = 0ull;
+  for (int u = 0; u < 4; ++u) {
+    later += u > w ? s_wave[u] : 0ull;
+    tot += s_wave[u];
+  }
+  const double target = (1.0 - (double)p) * (double)tot;
+  const bool in0 = (double)(later + v1) <= target && (double)(later + v1 + v0) > target;
+  const bool in1 = (double)later <= target && (double)(later + v1) > target;
+  if (in0 || in1) {  // at most one thread: the running mass passes the target once
+    s_cut = 2 * tid + (in1 ? 1 : 0);
+    s_below = in1 ? later : later + v1;
+  }
+  __syncthreads();
+  if (tid == 0) *out = WideRow{m, WIDE_CUT, s_cut, 0, s_below, target};
+}
+
+// The exponential race over the entries of a chunk above the row's cut bin (all of them without
+// top-p), and the list of those inside it.
+__global__ __launch_bounds__(kCandThreads) void sample_race_kernel(CandArgs c) {
+  __shared__ uint32_t s_ck[kCandThreads / 64][kWideCap];
+  __shared__ int32_t s_ci[kCandThreads / 64][kWideCap];
+  __shared__ uint32_t s_scan[kCandThreads / 64];
+  __shared__ float s_v[kCandThreads / 64];
+  __shared__ int s_i[kCandThreads / 64];
+  const SampArgs& a = c.a;
+  const int64_t row = blockIdx.y;
+  const int chunk = blockIdx.x, tid = threadIdx.x, wv = tid >> 6;
+  int64_t k;
+  if (take_rows_chunked(a, row, &k) || !no_top_k(a, k) || (a.greedy && a.greedy[row])) return;
+  const WideRow wr = *wide_row(c, row);
+  if (wr.state == WIDE_NO) return;
+  const int64_t base = (int64_t)chunk * kCandChunk;
+  const int n = (int)min((int64_t)kCandChunk, a.vocab - base);
+  const float* lg = a.logits + row * a.ld + base;
+  const float* nz = a.noise + row * a.ldn + base;
+  float vals[kCandPerThread], noise[kCandPerThread];
+#pragma unroll
+  for (int i = 0; i < kCandPerThread; ++i) vals[i] = lg[min(i * kCandThreads + tid, n - 1)];
+#pragma unroll
+  for (int i = 0; i < kCandPerThread; ++i) noise[i] = __builtin_nontemporal_load(nz + min(i * kCandThreads + tid, n - 1));
+  const float t = row_temperature(a, row);
+  const bool all = wr.state == WIDE_ALL;
+  const float fbm = wide_bin(wr.m), cut = (float)wr.cut;
+  float bv = -1.f;
+  int bi = 0x7fffffff;
+  uint32_t wn = 0;  // the wavefront's in-bin entries so far
+#pragma unroll
+  for (int i = 0; i < kCandPerThread; ++i) {
+    const int e = i * kCandThreads + tid;
+    const float z = vals[i] / t;
+    const float r = fbm - wide_bin(z);
+    if (e < n && (all || r < cut)) {
+      const float s = expf(z - wr.m) / fmaxf(noise[i], 1.17549435e-38f);
+      if (s > bv) {  // ascending index: the first of equal scores stays
+        bv = s;
+        bi = (int)(base + e);
+      }
+    }
+    const bool in = !all && e < n && r == cut;
+    const unsigned long long mk = __ballot(in);
+    if (mk != 0ull) {
+      const uint32_t pos = wn + __builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u));
+      if (in && pos < (uint32_t)kWideCap) {
+        s_ck[wv][pos] = ord_key(vals[i]);
+        s_ci[wv][pos] = (int32_t)(base + e);
+      }
+      wn += (uint32_t)__popcll(mk);
+    }
+  }
+  if ((tid & 63) == 0) s_scan[wv] = wn;
+  const int id = wg_argmax(bv, bi, s_v, s_i);  // (its barrier also covers s_scan and the lists)
+  const int64_t slot = row * c.chunks + chunk;
+  const uint32_t o1 = s_scan[0], o2 = o1 + s_scan[1], o3 = o2 + s_scan[2], cnt = o3 + s_scan[3];
+  if (cnt <= (uint32_t)kWideCap) {
+    uint32_t* ck = c.keys(slot);
+    int32_t* ci = c.idxs(slot);
+    for (uint32_t j = tid; j < cnt; j += kCandThreads) {
+      const int src = j >= o3 ? 3 : j >= o2 ? 2 : j >= o1 ? 1 : 0;
+      const uint32_t at = j - (src == 3 ? o3 : src == 2 ? o2 : src == 1 ? o1 : 0u);
+      ck[j] = s_ck[src][at];
+      ci[j] = s_ci[src][at];
+    }
+  }
+  if (tid == 0) {
+    c.cand_cnt[slot] = cnt <= (uint32_t)kWideCap ? (int32_t)cnt : kCntOver;
+    c.arg_val[slot] = fmaxf(fmaxf(s_v[0], s_v[1]), fmaxf(s_v[2], s_v[3]));
+    c.arg_idx[slot] = id;
+  }
 }
 
 // LDS of the finishing workgroup's fast path.
@@ -803,8 +1071,8 @@ __device__ bool finish_regs(const CandArgs& c, int64_t row, uint32_t k, float t,
     cn[cc] = c.cand_cnt[sl];
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      rk[cc * 4 + b] = c.cand_key[sl * kCandCap + l + 64 * b];
-      ri[cc * 4 + b] = c.cand_idx[sl * kCandCap + l + 64 * b];
+      rk[cc * 4 + b] = c.keys(sl)[l + 64 * b];
+      ri[cc * 4 + b] = c.idxs(sl)[l + 64 * b];
     }
   }
   uint32_t tm = 0;
@@ -875,6 +1143,93 @@ __device__ int p_from_lds(const uint32_t* s_key, const int32_t* s_idx, int nc, u
   return (int)np;
 }
 
+// The finish of a row without top-k: the nc in-bin entries (z keys and indices in LDS) that the cut
+// keeps join the chunks' race winners. An entry is kept when the mass at or below its value
+// exceeds the target, or it equals the largest: up to one entry per thread each sums the list for
+// itself; more take a radix select on mass (four 8-bit digits of the key, 64-bit sums).
+__device__ void finish_wide(const CandArgs& c, int64_t row, const WideRow& wr, const uint32_t* s_key,
+                            const int32_t* s_idx, int nc, const float* nz, unsigned long long* s_mass,
+                            uint32_t* s_sel, SampShared& sh) {
+  constexpr int NT = kFinishThreads;
+  const int tid = threadIdx.x;
+  const int64_t slot0 = row * c.chunks;
+  const uint32_t mkey = ord_key(wr.m);
+  float bv = -1.f;
+  int bi = 0x7fffffff;
+  auto better = [&](float v, int i) {
+    if (v > bv || (v == bv && i < bi)) {
+      bv = v;
+      bi = i;
+    }
+  };
+  for (int ch = tid; ch < c.chunks; ch += NT) better(c.arg_val[slot0 + ch], c.arg_idx[slot0 + ch]);
+  if (nc > 0 && nc <= NT) {
+    uint32_t kv = 0;
+    float e = 0.f;
+    if (tid < nc) {
+      kv = s_key[tid];
+      e = expf(key_value(kv) - wr.m);
+    }
+    s_mass[tid] = tid < nc ? mass_fixed(e) : 0ull;
+    __syncthreads();
+    if (tid < nc) {
+      unsigned long long cum = wr.below;
+#pragma unroll 4
+      for (int j = 0; j < nc; ++j) cum += s_key[j] <= kv ? s_mass[j] : 0ull;
+      if ((double)cum > wr.target || kv == mkey) better(e / fmaxf(nz[s_idx[tid]], 1.17549435e-38f), s_idx[tid]);
+    }
+  } else if (nc > NT) {
+    uint32_t prefix = 0, pmask = 0;
+    unsigned long long below = wr.below;
+    bool found = true;
+    for (int shift = 24; shift >= 0; shift -= 8) {
+      s_mass[tid] = 0ull;
+      __syncthreads();
+      for (int i = tid; i < nc; i += NT) {
+        const uint32_t key = s_key[i];
+        if ((key & pmask) == prefix) atomicAdd(&s_mass[(key >> shift) & 255], mass_fixed(expf(key_value(key) - wr.m)));
+      }
+      __syncthreads();
+      if (tid < 64) {  // four digits per lane, ascending: the first whose running mass passes the target
+        unsigned long long h[4], own = 0ull;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) own += h[b] = s_mass[4 * tid + b];
+        unsigned long long incl = own;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const unsigned long long o = __shfl_up(incl, off);
+          incl += tid >= off ? o : 0ull;
+        }
+        unsigned long long cum = below + incl - own;
+        const bool hit = !((double)cum > wr.target) && (double)(below + incl) > wr.target;
+        if (tid == 0) s_sel[0] = 256u;
+        if (hit) {
+          int d = 0;
+          while (d < 3 && !((double)(cum + h[d]) > wr.target)) cum += h[d++];
+          s_sel[0] = (uint32_t)(4 * tid + d);
+          sh.bcast_ull = cum;
+        }
+      }
+      __syncthreads();
+      if (s_sel[0] == 256u) {  // rounding left no crossing: of these entries only the largest value
+        found = false;
+        break;
+      }
+      prefix |= s_sel[0] << shift;
+      pmask |= 255u << shift;
+      below = sh.bcast_ull;
+      __syncthreads();
+    }
+    for (int i = tid; i < nc; i += NT) {
+      const uint32_t key = s_key[i];
+      if ((found && key >= prefix) || key == mkey)
+        better(expf(key_value(key) - wr.m) / fmaxf(nz[s_idx[i]], 1.17549435e-38f), s_idx[i]);
+    }
+  }
+  const int id = block_argmax(bv, bi, sh);
+  if (tid == 0) c.a.ids[row] = id;
+}
+
 __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(CandArgs c) {
   __shared__ SampShared sh;
   __shared__ uint32_t s_key[kFinishCap];
@@ -907,11 +1262,18 @@ __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(CandArgs 
     return;
   }
   int64_t k;
-  take_rows_chunked(a, row, &k);  // (a row that was not chunked has a negative count below)
+  const bool ranked = take_rows_chunked(a, row, &k);  // (a row that was not chunked has a negative count below)
   const float t = row_temperature(a, row);
   const float p = row_top_p(a, row);
   const float* nz = a.noise + row * a.ldn;
-  if (c.chunks <= 16) {
+  WideRow wr{};
+  if (c.wide && !ranked && no_top_k(a, k)) {
+    wr = *wide_row(c, row);
+    if (wr.state == WIDE_ALL) {  // no lists: the chunks' winners
+      finish_wide(c, row, wr, s_key, s_idx, 0, nz, s_mass, s_sel, sh);
+      return;
+    }
+  } else if (c.chunks <= 16) {
     if (finish_regs<16>(c, row, (uint32_t)k, t, p, nz, fs)) return;
   } else if (c.chunks <= 32) {
     if (finish_regs<32>(c, row, (uint32_t)k, t, p, nz, fs)) return;
@@ -953,9 +1315,8 @@ __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(CandArgs 
         if (s_off[mid] <= j) lo = mid;
         else hi = mid - 1;
       }
-      const int64_t src = (slot0 + lo) * kCandCap + (j - s_off[lo]);
-      const uint32_t kv = c.cand_key[src];
-      const int32_t iv = c.cand_idx[src];
+      const uint32_t kv = c.keys(slot0 + lo)[j - s_off[lo]];
+      const int32_t iv = c.idxs(slot0 + lo)[j - s_off[lo]];
       if (j0 + tid < nc) {
         s_key[j] = ord_key(key_value(kv) / t);  // z = logits / temperature (IEEE division)
         s_idx[j] = iv;
@@ -963,6 +1324,10 @@ __global__ __launch_bounds__(kFinishThreads) void sample_finish_kernel(CandArgs 
     }
   }
   __syncthreads();
+  if (wr.state == WIDE_CUT) {
+    finish_wide(c, row, wr, s_key, s_idx, nc, nz, s_mass, s_sel, sh);
+    return;
+  }
   {
     uint32_t mkey;
     const int np = p_from_lds(s_key, s_idx, nc, (uint32_t)k, fs, &mkey);
@@ -1207,9 +1572,11 @@ extern "C" size_t msa_sample_workspace_size(int64_t rows, int64_t vocab) {
   return sample_ws_bytes(rows, vocab);
 }
 
-extern "C" int msa_sample(const float* logits, int64_t ld, int64_t rows, int64_t vocab, const float* temperature,
-                          const int32_t* top_k, const float* top_p, const uint8_t* greedy, const float* noise,
-                          int64_t ldn, int64_t* out_ids, void* workspace, size_t workspace_bytes, msa_stream_t stream) {
+// wide: the batch may hold rows without top-k; without it the two launches that serve them are
+// left out and such a row takes the whole-row path.
+static int sample_ids(const float* logits, int64_t ld, int64_t rows, int64_t vocab, const float* temperature,
+                      const int32_t* top_k, const float* top_p, const uint8_t* greedy, const float* noise, int64_t ldn,
+                      int64_t* out_ids, void* workspace, size_t workspace_bytes, bool wide, msa_stream_t stream) {
   if (!out_ids || !noise || ldn < vocab) return fail(MSA_ERR_INVALID, "msa_sample: bad noise / out_ids");
   SampArgs a{};
   a.logits = logits; a.ld = ld; a.vocab = vocab; a.temperature = temperature; a.top_k = top_k; a.top_p = top_p;
@@ -1224,15 +1591,35 @@ extern "C" int msa_sample(const float* logits, int64_t ld, int64_t rows, int64_t
   c.chunks = (int)sample_chunks(vocab);
   const size_t slots = (size_t)rows * c.chunks;
   char* w = (char*)workspace;
-  c.cand_key = (uint32_t*)w;
-  c.cand_idx = (int32_t*)(w + slots * kCandCap * sizeof(uint32_t));
+  c.wide = wide && (reinterpret_cast<uintptr_t>(w) & 7u) == 0;  // the histograms are 8-byte words
+  c.cand = (uint32_t*)w;
   c.cand_cnt = (int32_t*)(w + slots * kCandCap * 2 * sizeof(uint32_t));
   c.arg_val = (float*)(c.cand_cnt + slots);
   c.arg_idx = (int32_t*)(c.arg_val + slots);
   hipLaunchKernelGGL(sample_chunk_kernel, dim3((unsigned)c.chunks, (unsigned)rows), dim3(kCandThreads), 0,
                      (hipStream_t)stream, c);
+  if (c.wide) {
+    hipLaunchKernelGGL(sample_cut_kernel, dim3((unsigned)rows), dim3(kCandThreads), 0, (hipStream_t)stream, c);
+    hipLaunchKernelGGL(sample_race_kernel, dim3((unsigned)c.chunks, (unsigned)rows), dim3(kCandThreads), 0,
+                       (hipStream_t)stream, c);
+  }
   hipLaunchKernelGGL(sample_finish_kernel, dim3((unsigned)rows), dim3(kFinishThreads), 0, (hipStream_t)stream, c);
   return check_launch("msa_sample");
+}
+
+extern "C" int msa_sample(const float* logits, int64_t ld, int64_t rows, int64_t vocab, const float* temperature,
+                          const int32_t* top_k, const float* top_p, const uint8_t* greedy, const float* noise,
+                          int64_t ldn, int64_t* out_ids, void* workspace, size_t workspace_bytes, msa_stream_t stream) {
+  return sample_ids(logits, ld, rows, vocab, temperature, top_k, top_p, greedy, noise, ldn, out_ids, workspace,
+                    workspace_bytes, true, stream);
+}
+
+extern "C" int msa_sample_ranked(const float* logits, int64_t ld, int64_t rows, int64_t vocab, const float* temperature,
+                                 const int32_t* top_k, const float* top_p, const uint8_t* greedy, const float* noise,
+                                 int64_t ldn, int64_t* out_ids, void* workspace, size_t workspace_bytes,
+                                 msa_stream_t stream) {
+  return sample_ids(logits, ld, rows, vocab, temperature, top_k, top_p, greedy, noise, ldn, out_ids, workspace,
+                    workspace_bytes, false, stream);
 }
 
 extern "C" int msa_verify_greedy(const int64_t* target_ids, int64_t batch, int64_t k, const int64_t* drafts,

@@ -735,6 +735,8 @@ def lm_head_logits(
 
 # ---- sampling ---------------------------------------------------------------------------------------
 
+RANKED_MAX_TOP_K = 256  # largest top_k the sampling kernel takes from vocabulary chunks' candidates
+
 
 def _rows_f32(logits: Tensor, name: str) -> Tensor:
     _check(logits.dtype == torch.float32 and logits.dim() == 2 and logits.stride(-1) == 1, f"{name}: float32 [R, V] logits")
@@ -780,16 +782,20 @@ def sample_ids(
     top_p: Tensor | None,
     greedy: Tensor | None,
     noise: Tensor | None,
+    ranked: bool = False,
 ) -> Tensor:
     """Token id per row: the greedy argmax where ``greedy``, else argmax(probs / noise) with the
     probabilities of ``sampling_probs`` (runner/sampler.py:55-69). ``noise`` [R, V] float32 ~ Exp(1);
-    it may be None only when every row is greedy."""
+    it may be None only when every row is greedy. ``ranked``: the caller knows that every row is
+    greedy or has 0 < top_k <= 256, so the launches that serve other rows are left out (the same ids
+    either way: such a row would still be served, by one workgroup)."""
     _on_gpu(logits)
     _rows_f32(logits, "sample_ids")
     r, v = logits.shape
     if noise is None:
         _check(greedy is not None, "sample_ids: noise is required for sampled rows")
         noise = logits  # never read: every row is greedy
+        ranked = True
     _check(noise.dtype == torch.float32 and noise.dim() == 2 and noise.shape == (r, v) and noise.stride(-1) == 1,
            "sample_ids: noise [R, V] float32")
     out = torch.empty(r, dtype=torch.int64, device=logits.device)
@@ -797,11 +803,11 @@ def sample_ids(
     tk = _opt_param(top_k, torch.int32, r, "top_k")
     tp = _opt_param(top_p, torch.float32, r, "top_p")
     gr = _opt_param(greedy, torch.uint8, r, "greedy")
-    # Greedy rows and rows with 0 < top_k <= 256 run over vocabulary chunks (the workspace holds
-    # each chunk's candidates); the others fall back to a workgroup per row inside the same call.
+    # Greedy rows, rows with 0 < top_k <= 256 and rows without top-k run over vocabulary chunks (the
+    # workspace holds each chunk's candidates); the others take a workgroup per row in the same call.
     ws_bytes = _native.query("msa_sample_workspace_size", r, v)
     ws = workspaces.get("sample", logits.device, ws_bytes)
-    _native.call("msa_sample", _ptr(logits), logits.stride(0), r, v, _ptr(temps), _ptr(tk), _ptr(tp), _ptr(gr),
+    _native.call("msa_sample_ranked" if ranked else "msa_sample", _ptr(logits), logits.stride(0), r, v, _ptr(temps), _ptr(tk), _ptr(tp), _ptr(gr),
                  _ptr(noise), noise.stride(0), _ptr(out), _ptr(ws), ws.numel() if ws is not None else 0,
                  _stream(logits))
     return out

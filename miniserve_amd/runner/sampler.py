@@ -74,4 +74,5 @@ def sample(logits: Tensor, params: Sequence[Any], generators: Sequence[torch.Gen
     temps = to_device([max(p.temperature, 1e-5) for p in params], dev, torch.float32)
     top_k, top_p = _filters(params, vocab, dev)
     noise = exponential_noise((rows, vocab), generators, dev)
-    return kernels.sample_ids(logits, temps, top_k, top_p, greedy, noise)
+    ranked = all(p.greedy or 0 < p.top_k <= kernels.RANKED_MAX_TOP_K for p in params)
+    return kernels.sample_ids(logits, temps, top_k, top_p, greedy, noise, ranked)

@@ -206,3 +206,53 @@ def test_chunked_sampling_matches_the_whole_row_path(vocab):
             assert int(got[r]) == int(whole[r]), r
             checked += 1
     assert checked >= rows * 3 // 4
+
+
+@pytest.mark.parametrize("vocab", [64, 10240, 10241, 151936, 660000])
+def test_rows_without_top_k_over_chunks(vocab):
+    """Rows with temperature alone or top-p alone (mass histogram, cut bin, race over chunks)
+    against the whole-row path on the same logits and noise: identical ids wherever the best two
+    scores differ by more than 1e-5 relative (float32 scores, each within a few 2^-24 of exact).
+    Rows: dense and bf16-rounded logits (ties at the cut), a flat row and a row of few values (more
+    entries at the cut than the lists hold), a row with one dominating entry, rows with -inf
+    entries, with whole chunks of them and with a NaN, top-p near 0 and near 1, a temperature so
+    small that z leaves the range of whole numbers, a row stride that is not the vocabulary.
+    Vocabularies: less than a workgroup, one chunk, a one-entry last chunk, 15 chunks, and more
+    chunks than the finishing workgroup gathers."""
+    rows = 24
+    g = torch.Generator().manual_seed(vocab + 1)
+    logits = (torch.randn(rows, vocab + 3, generator=g) * 3)[:, :vocab]
+    logits[8:14] = logits[8:14].to(torch.bfloat16).float()
+    logits[14] = 0.5
+    logits[15] = torch.round(logits[15] / 4)
+    logits[16, vocab // 2] = 60.0
+    logits[17, ::2] = float("-inf")
+    logits[18, : vocab - 5] = float("-inf")
+    logits[19, 7] = float("nan")
+    p = (torch.rand(rows, generator=g) * 0.9 + 0.05).float()
+    p[::3] = 1.0
+    p[1], p[8], p[17], p[18] = 1e-7, 0.99999, 0.9, 0.7
+    temps = (torch.rand(rows, generator=g) * 1.2 + 0.3).float()
+    temps[20], temps[22] = 1e-5, 1e-5
+    k = torch.full((rows,), vocab, dtype=torch.int32)
+    k[2::5] = -1
+    greedy = torch.zeros(rows, dtype=torch.uint8)
+    greedy[5] = 1
+    noise = torch.empty(rows, vocab).exponential_(generator=g)
+    ld = torch.empty(rows, vocab + 3, device=DEV)[:, :vocab].copy_(logits)
+    td, kd, pd, gd, nd = (t.to(DEV) for t in (temps, k, p, greedy, noise))
+    got = kernels.sample_ids(ld, td, kd, pd, gd, nd).cpu()
+    assert torch.equal(got, kernels.sample_ids(ld, td, kd, pd, gd, nd).cpu())  # deterministic
+    assert torch.equal(got[greedy.bool()], logits.argmax(-1)[greedy.bool()])
+    whole = _whole_row_ids(ld, td, kd, pd, gd, nd).cpu()
+    scores = (kernels.sampling_probs(ld, td, kd, pd) / nd.clamp_min(1.17549435e-38)).double()
+    top2 = scores.topk(2).values.cpu()
+    checked = 0
+    for r in range(rows):
+        if r == 19 or float(top2[r, 0] - top2[r, 1]) > 1e-5 * float(top2[r, 0]):
+            assert int(got[r]) == int(whole[r]), r
+            checked += 1
+    assert checked >= rows - 2
+    none = kernels.sample_ids(ld, td, None, None, gd, nd).cpu()  # no filters at all: temperature alone
+    full = kernels.sample_ids(ld, td, kd, torch.ones_like(pd), gd, nd).cpu()
+    assert torch.equal(none, full)
