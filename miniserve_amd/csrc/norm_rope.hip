@@ -47,6 +47,56 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict
   }
 }
 
+// RMSNorm of rows of 2048 to 2048 NV elements: a workgroup per row, the row in registers between the
+// sum of squares and the normalization, every load (row and norm weight) issued before the first
+// use. A wavefront per row (above) walks a 4096-wide row in eight dependent steps, twice: 5.8 us
+// after an 8B-shaped o projection of 1 to 27 rows, latency alone, against 2.4 here (2.1-2.3 back to
+// back in a graph); 4096 rows (67 MB in and out) 15.7 against 11.2 us.
+template <int NV>
+__global__ __launch_bounds__(256) void rmsnorm_row_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                          const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
+                                                          int64_t ldo, int dim, float eps) {
+  __shared__ float red[4];
+  const int tid = threadIdx.x;
+  const uint16_t* xr = x + (int64_t)blockIdx.x * ldx;
+  uint16_t* orow = out + (int64_t)blockIdx.x * ldo;
+  uint4 v[NV], wv[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = min((tid + 256 * i) * 8, dim - 8);  // pieces past the row repeat its last one: not summed or stored
+    v[i] = *(const uint4*)(xr + c);
+    wv[i] = *(const uint4*)(w + c);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const uint32_t u[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+    if ((tid + 256 * i) * 8 < dim) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss += bf16lo(u[e]) * bf16lo(u[e]) + bf16hi(u[e]) * bf16hi(u[e]);
+    }
+  }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  ss = red[0] + red[1] + red[2] + red[3];
+  const float r = 1.0f / sqrtf(ss / (float)dim + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (tid + 256 * i) * 8;
+    if (c >= dim) continue;
+    const uint32_t u[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+    const uint32_t ww[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = round_bf16(bf16lo(u[e]) * r), b = round_bf16(bf16hi(u[e]) * r);
+      o[e] = pack_bf16x2(bf16lo(ww[e]) * a, bf16hi(ww[e]) * b);
+    }
+    *(uint4*)(orow + c) = uint4{o[0], o[1], o[2], o[3]};
+  }
+}
+
 __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const uint16_t* resid_in, const uint16_t* __restrict__ delta,
                                                           uint16_t* resid_out, const uint16_t* __restrict__ w,
                                                           uint16_t* __restrict__ out, int64_t rows, int dim, float eps) {
@@ -368,6 +418,14 @@ void launch_splitk_add_rmsnorm(const float* part, int k_split, int64_t rows, int
 
 void launch_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* w, uint16_t* out, int64_t ldo, int64_t rows, int dim,
                     float eps, hipStream_t s) {
+  // (out may be x: a workgroup has read its row before it writes it)
+  if (dim >= 2048 && dim <= 8192) {
+    const dim3 grid((unsigned)rows), block(256);
+    if (dim == 2048) hipLaunchKernelGGL(rmsnorm_row_kernel<1>, grid, block, 0, s, x, ldx, w, out, ldo, dim, eps);
+    else if (dim <= 4096) hipLaunchKernelGGL(rmsnorm_row_kernel<2>, grid, block, 0, s, x, ldx, w, out, ldo, dim, eps);
+    else hipLaunchKernelGGL(rmsnorm_row_kernel<4>, grid, block, 0, s, x, ldx, w, out, ldo, dim, eps);
+    return;
+  }
   hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, x, ldx, w, out, ldo, rows, dim,
                      eps);
 }
@@ -401,8 +459,8 @@ extern "C" int msa_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* weigh
   if (dim % 8 != 0 || ldx % 8 != 0 || ldo % 8 != 0 || !aligned16(x) || !aligned16(out) || !aligned16(weight))
     return fail(MSA_ERR_UNSUPPORTED, "msa_rmsnorm: dim and row strides must be multiples of 8, pointers 16-byte aligned");
   if (ldx < dim || ldo < dim) return fail(MSA_ERR_INVALID, "msa_rmsnorm: row stride smaller than dim");
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, (hipStream_t)stream, x, ldx,
-                     weight, out, ldo, rows, (int)dim, eps);
+  if (rows > 0x7fffffff) return fail(MSA_ERR_INVALID, "msa_rmsnorm: bad shape");
+  launch_rmsnorm(x, ldx, weight, out, ldo, rows, (int)dim, eps, (hipStream_t)stream);
   return check_launch("msa_rmsnorm");
 }
 

@@ -1,0 +1,29 @@
+"""GPU parity of RMSNorm over the row widths at which its kernels change: a wavefront per row (below
+2048 and above 8192), a workgroup per row with one, two or four 16-byte pieces per thread (2048, up to
+4096, up to 8192), ragged widths among them. Within rel-L2 2e-3 of the oracle: the order of the sum of
+squares moves the row factor by float32 roundings, which flip bf16 roundings of single elements."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+from helpers import rel_l2
+
+from miniserve_amd import kernels
+from oracle import layers as ol
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _bf16(shape, seed, std=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * std).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 2048), (3, 2056), (5, 4096), (2, 4104), (7, 8192), (3, 8200), (9, 1024)])
+def test_rmsnorm_row_widths(rows, dim):
+    x, w = _bf16((rows, dim), seed=dim, std=2.0), _bf16((dim,), seed=4, std=0.1) + 1
+    xd = x.to(DEV)
+    out = kernels.rmsnorm(xd, w.to(DEV), 1e-6)
+    assert rel_l2(out.cpu(), ol.rms_norm(x, w, 1e-6)) < 2e-3
+    assert torch.equal(kernels.rmsnorm(xd, w.to(DEV), 1e-6, out=xd), out)  # in place
