@@ -236,6 +236,25 @@ static void launch_skinny(const SkinnyPlan& p, SkinnyArgs& a, hipStream_t s) {
   }
 }
 
+// The merge of float32 partials [k_split][m][n] with the epilogue, one thread per output.
+static int launch_splitk_epilogue(const float* partial, int k_split, int64_t m, int64_t n, uint16_t* y, int64_t ldy,
+                                  int epilogue, const uint16_t* residual, int64_t ldr, hipStream_t s) {
+  const int64_t total = m * (epilogue == MSA_EPI_SILU_MUL ? n / 2 : n);
+  const dim3 grid((unsigned)((total + 255) / 256)), block(256);
+  switch (epilogue) {
+    case MSA_EPI_NONE:
+      hipLaunchKernelGGL(splitk_epilogue_kernel<MSA_EPI_NONE>, grid, block, 0, s, partial, k_split, m, (int)n, y, ldy, residual, ldr);
+      break;
+    case MSA_EPI_SILU_MUL:
+      hipLaunchKernelGGL(splitk_epilogue_kernel<MSA_EPI_SILU_MUL>, grid, block, 0, s, partial, k_split, m, (int)n, y, ldy, residual, ldr);
+      break;
+    default:
+      hipLaunchKernelGGL(splitk_epilogue_kernel<MSA_EPI_RESIDUAL>, grid, block, 0, s, partial, k_split, m, (int)n, y, ldy, residual, ldr);
+      break;
+  }
+  return check_launch("msa_int8_linear (split-K epilogue)");
+}
+
 static int check_linear_args(const char* fn, const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
                              const int8_t* qweight, const uint16_t* scale, int64_t n) {
   if (!x || !qweight || !scale) return fail(MSA_ERR_INVALID, std::string(fn) + ": null pointer");
@@ -250,11 +269,27 @@ static int check_linear_args(const char* fn, const uint16_t* x, int64_t m, int64
 
 }  // namespace msa
 
-// Batches of at least this many rows (with k % 64 == 0) go to the LDS-tiled GEMM (gemm_int8.hip).
+// Batches of at least this many rows (with k % 64 == 0) go to the LDS-tiled GEMM (gemm_int8.hip);
+// over weights of 12 MB and more already those past the wide decode kernel's 64: the kernels for
+// small batches read such weights once per 16 tokens (8B-shaped gate_up at 96 tokens 132 us, the GEMM
+// at 128 tokens 62).
 constexpr int64_t kGemmMinRows = 128;
+constexpr int64_t kGemmMinRowsWide = 65, kWideWeights = (int64_t)12 << 20;
+static bool takes_gemm(int64_t m, int64_t n, int64_t k) {
+  return k % 64 == 0 && (m >= kGemmMinRows || (m >= kGemmMinRowsWide && n * k >= kWideWeights));
+}
 
 namespace msa {
 bool dec_linear_supported(int64_t k);  // gemv_dec.hip: K in {1024, 2048, 3072, 4096}
+bool dec_stream_eligible(int64_t m, int64_t k, int64_t n, int epilogue);  // gemv_stream.hip
+// gemv_wide.hip: up to 64 tokens over weights of 12 MB and more
+bool dec_wide_eligible(int64_t m, int64_t k, int64_t n, int64_t ldx, int64_t ldy, int64_t ldr);
+int dec_wide_splits(int64_t m, int64_t n, int64_t k);
+int launch_dec_wide(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight, const uint16_t* scale,
+                    int64_t n, uint16_t* y, int64_t ldy, int epilogue, const uint16_t* residual, int64_t ldr,
+                    hipStream_t s);
+int launch_dec_wide_partials(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
+                             const uint16_t* scale, int64_t n, int splits, float* part, hipStream_t s);
 }  // namespace msa
 
 extern "C" int msa_int8_gemm(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
@@ -264,6 +299,16 @@ extern "C" int msa_int8_linear_rows(const uint16_t* x, int64_t ldx, int64_t m, i
                                     float eps, const int8_t* qweight, const uint16_t* scale, int64_t n, int epilogue,
                                     uint16_t* y, int64_t ldy, const uint16_t* residual, int64_t ldr,
                                     msa_stream_t stream);
+
+// msa_int8_linear_add_rmsnorm on the wide decode kernel: up to this many tokens the product and the
+// residual in one launch, then the norm; above, split-K partials that the norm's kernel merges (8B
+// down at 32 tokens: 22 us against 16.5, o 9.1 against 7.7; at 16 tokens 16.4 / 7.2 against 14.6 /
+// 6.7 with a dearer merge).
+constexpr int64_t kWideDirectTokens = 16;
+// msa_int8_linear there: a long K (8B down: 24.0 us at 32 tokens in one launch, 34.2 at 64) is split
+// too, merged by an epilogue kernel (about 20 and 23); o (K = 4096) takes 10.0 / 13.5 us in one
+// launch, which a merge would not beat.
+constexpr int64_t kWideSplitMinK = 8192;
 
 // Smaller batches whose activation tile fits in LDS go to the token-split kernels (gemv_rows.hip).
 static bool rows_fits(int64_t k) { return k % 64 == 0 && 16 * (k + 8) * 2 + 16 * 1024 <= 160 * 1024; }
@@ -283,7 +328,11 @@ void launch_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* w, uint16_t*
 
 extern "C" size_t msa_int8_linear_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  if (m >= kGemmMinRows && k % 64 == 0) return msa::gemm_workspace_size(m, n, k, MSA_EPI_NONE);  // split-K partials
+  if (takes_gemm(m, n, k)) return msa::gemm_workspace_size(m, n, k, MSA_EPI_NONE);  // split-K partials
+  if (msa::dec_wide_eligible(m, k, n, k, n, n)) {  // the partials of msa_int8_linear_add_rmsnorm
+    const int sp = msa::dec_wide_splits(m, n, k);
+    return sp > 1 && m > kWideDirectTokens ? (size_t)sp * m * n * sizeof(float) : 0;
+  }
   if (msa::dec_linear_supported(k) || rows_fits(k)) return 0;
   size_t best = 0;
   for (int epi = 0; epi < 3; ++epi) {
@@ -309,9 +358,21 @@ extern "C" int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t 
   if (ldy < out_cols) return fail(MSA_ERR_INVALID, "msa_int8_linear: ldy too small");
   if (epilogue == MSA_EPI_RESIDUAL && (!residual || ldr < n))
     return fail(MSA_ERR_INVALID, "msa_int8_linear: residual epilogue needs residual with ldr >= n");
-  if (m >= kGemmMinRows && k % 64 == 0)
+  if (takes_gemm(m, n, k))
     return gemm_run(x, m, k, ldx, qweight, scale, n, y, ldy, epilogue, residual, ldr, workspace, workspace_bytes,
                     (hipStream_t)stream);
+  // Large weights: the streaming kernel (up to 16 tokens, K of 2048 / 4096, enough rows; inside the
+  // decode entry point below), else the wide kernel.
+  if (!dec_stream_eligible(m, k, n, epilogue) &&
+      dec_wide_eligible(m, k, n, ldx, ldy, epilogue == MSA_EPI_RESIDUAL ? ldr : 0)) {
+    const int splits = m > kWideDirectTokens && k >= kWideSplitMinK && epilogue != MSA_EPI_SILU_MUL ? dec_wide_splits(m, n, k) : 1;
+    if (splits > 1 && workspace && workspace_bytes >= (size_t)splits * m * n * sizeof(float) && aligned16(workspace)) {
+      rc = launch_dec_wide_partials(x, m, k, ldx, qweight, scale, n, splits, (float*)workspace, (hipStream_t)stream);
+      if (rc != MSA_OK) return rc;
+      return launch_splitk_epilogue((const float*)workspace, splits, m, n, y, ldy, epilogue, residual, ldr, (hipStream_t)stream);
+    }
+    return launch_dec_wide(x, m, k, ldx, qweight, scale, n, y, ldy, epilogue, residual, ldr, (hipStream_t)stream);
+  }
   // Decode-sized batches: the decode kernel (all of a workgroup's loads in flight at once, the same
   // rounding points); other K that fit the LDS activation tile: the token-split rows kernel.
   if (dec_linear_supported(k))
@@ -337,23 +398,7 @@ extern "C" int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t 
     launch_skinny<kEpiPartial>(pp, a, s);
     rc = check_launch("msa_int8_linear (split-K pass)");
     if (rc != MSA_OK) return rc;
-    const int64_t total = m * out_cols;
-    const unsigned blocks = (unsigned)((total + 255) / 256);
-    switch (epilogue) {
-      case MSA_EPI_NONE:
-        hipLaunchKernelGGL(splitk_epilogue_kernel<MSA_EPI_NONE>, dim3(blocks), dim3(256), 0, s, a.partial, pp.k_split,
-                           m, (int)n, y, ldy, residual, ldr);
-        break;
-      case MSA_EPI_SILU_MUL:
-        hipLaunchKernelGGL(splitk_epilogue_kernel<MSA_EPI_SILU_MUL>, dim3(blocks), dim3(256), 0, s, a.partial,
-                           pp.k_split, m, (int)n, y, ldy, residual, ldr);
-        break;
-      default:
-        hipLaunchKernelGGL(splitk_epilogue_kernel<MSA_EPI_RESIDUAL>, dim3(blocks), dim3(256), 0, s, a.partial,
-                           pp.k_split, m, (int)n, y, ldy, residual, ldr);
-        break;
-    }
-    return check_launch("msa_int8_linear (split-K epilogue)");
+    return launch_splitk_epilogue(a.partial, pp.k_split, m, n, y, ldy, epilogue, residual, ldr, s);
   }
   switch (epilogue) {
     case MSA_EPI_NONE: launch_skinny<MSA_EPI_NONE>(p, a, s); break;
@@ -395,11 +440,20 @@ extern "C" int msa_int8_linear_add_rmsnorm(const uint16_t* x, int64_t m, int64_t
     return fail(MSA_ERR_UNSUPPORTED,
                 "msa_int8_linear_add_rmsnorm: n must be a multiple of 8 and residual / norm_w / out 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  if (m >= kGemmMinRows && k % 64 == 0) {
+  if (takes_gemm(m, n, k)) {
     const int splits = gemm_run_partials(x, m, k, ldx, qweight, scale, n, (float*)workspace, workspace_bytes, s);
     if (splits < 0) return MSA_ERR_LAUNCH;
     if (splits > 1) {
       rc = check_launch("msa_int8_linear_add_rmsnorm (split-K pass)");
+      if (rc != MSA_OK) return rc;
+      launch_splitk_add_rmsnorm((const float*)workspace, splits, m, (int)n, residual, residual, norm_w, out, eps, s);
+      return check_launch("msa_int8_linear_add_rmsnorm (merge + norm)");
+    }
+  }
+  if (m > kWideDirectTokens && dec_wide_eligible(m, k, n, ldx, n, n)) {
+    const int splits = dec_wide_splits(m, n, k);
+    if (splits > 1 && workspace && workspace_bytes >= (size_t)splits * m * n * sizeof(float) && aligned16(workspace)) {
+      rc = launch_dec_wide_partials(x, m, k, ldx, qweight, scale, n, splits, (float*)workspace, s);
       if (rc != MSA_OK) return rc;
       launch_splitk_add_rmsnorm((const float*)workspace, splits, m, (int)n, residual, residual, norm_w, out, eps, s);
       return check_launch("msa_int8_linear_add_rmsnorm (merge + norm)");

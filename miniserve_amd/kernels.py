@@ -574,6 +574,10 @@ def int8_linear_rows(
 DEC_MAX_TOKENS = 128  # decode-sized batches the pipeline sends to msa_int8_linear_dec
 
 
+WIDE_MIN_WEIGHTS = 12 << 20  # int8 weights of this many bytes: one launch streams for longer than it takes to start
+STREAM_MAX_TOKENS = 16  # tokens the streaming decode linear (RMSNorm prologue included) serves
+
+
 def dec_supported(k: int) -> bool:
     """Whether msa_int8_linear_dec takes this in_features (K split over 4-16 wavefronts of four
     64-wide chunks each)."""

@@ -164,6 +164,8 @@ class Qwen3ForCausalLM(nn.Module):
             residual = self._token_split_layers(input_ids, positions, kv_caches, meta)
             out: Tensor = self.norm(residual)
             return out
+        if self._wide_decode_ok(input_ids.numel(), meta):
+            return self._wide_decode_layers(input_ids, kv_caches, meta)
         x = self.embed_tokens(input_ids)
         cos, sin = self.rotary(positions)
         if self._all_int8():
@@ -216,6 +218,67 @@ class Qwen3ForCausalLM(nn.Module):
             and kernels.rows_supported(cfg.intermediate_size)
             and self._all_int8()
         )
+
+    def _wide_decode_ok(self, tokens: int, meta: AttentionMetadata) -> bool:
+        """Whether a batch takes the large-weight decode layers: decode rows only, up to
+        DEC_MAX_TOKENS, head_dim 128, int8 linears of WIDE_MIN_WEIGHTS and more (the 8B shape)."""
+        cfg = self.cfg
+        return (
+            meta.prefill is None
+            and meta.decode is not None
+            and 0 < tokens <= kernels.DEC_MAX_TOKENS
+            and cfg.head_dim == 128
+            and cfg.num_attention_heads // cfg.num_key_value_heads in (1, 2, 4, 8)
+            and self.decode_linears
+            and all(n * k >= kernels.WIDE_MIN_WEIGHTS and k % 64 == 0 for n, k in self._linear_shapes())
+            and self._all_int8()
+        )
+
+    def _linear_shapes(self) -> tuple[tuple[int, int], ...]:
+        """(out, in) features of a layer's qkv, o, gate_up and down projections."""
+        c = self.cfg
+        q, kv = c.num_attention_heads * c.head_dim, c.num_key_value_heads * c.head_dim
+        return ((q + 2 * kv, c.hidden_size), (c.hidden_size, q), (2 * c.intermediate_size, c.hidden_size),
+                (c.hidden_size, c.intermediate_size))
+
+    def _wide_decode_layers(
+        self, input_ids: Tensor, kv_caches: list[tuple[Tensor, Tensor]], meta: AttentionMetadata
+    ) -> Tensor:
+        """The decode layers of a model with large weights; returns the final-normed hidden states.
+        Per-head norms, RoPE and the cache write run inside the decode attention. Up to
+        STREAM_MAX_TOKENS tokens the RMSNorms run inside the qkv and gate_up linears (five launches a
+        layer); with more, each would be repeated by every workgroup, so they join the o and down
+        projections (whose split-K partials that kernel merges)."""
+        cfg, rot = self.cfg, self.rotary
+        t = input_ids.numel()
+        x = self.embed_tokens(input_ids.view(-1))  # the residual stream, updated in place
+        inside = t <= kernels.STREAM_MAX_TOKENS and kernels.dec_supported(cfg.hidden_size)
+        first = self.layers[0].input_layernorm
+        h = x if inside else kernels.rmsnorm(x, first.weight, first.eps)
+        for i, (k_cache, v_cache) in enumerate(kv_caches):
+            layer = self.layers[i]
+            attn, mlp = layer.self_attn, layer.mlp
+            qkv, o, gu, dn = attn.qkv_proj, attn.o_proj, mlp.gate_up_proj, mlp.down_proj
+            pre, post = layer.input_layernorm, layer.post_attention_layernorm
+            if inside:
+                rows = kernels.int8_linear_dec(x, qkv.qweight, qkv.kscale, norm_w=pre.weight, eps=pre.eps)
+            else:
+                rows = kernels.int8_linear(h, qkv.qweight, qkv.kscale)
+            a = attend_decode_qkv(
+                rows, attn.num_heads, attn.q_norm.weight, attn.k_norm.weight, attn.q_norm.eps, rot.cos, rot.sin,
+                k_cache, v_cache, meta, attn.scale,
+            ).view(t, attn.q_size)
+            if inside:
+                kernels.int8_linear(a, o.qweight, o.kscale, kernels.EPI_RESIDUAL, residual=x, out=x)
+                act = kernels.int8_linear_dec(x, gu.qweight, gu.kscale, kernels.EPI_SILU_MUL, norm_w=post.weight,
+                                              eps=post.eps)
+                kernels.int8_linear(act, dn.qweight, dn.kscale, kernels.EPI_RESIDUAL, residual=x, out=x)
+            else:
+                hn = kernels.int8_linear_add_rmsnorm(a, o.qweight, o.kscale, x, post.weight, post.eps)
+                act = kernels.int8_linear(hn, gu.qweight, gu.kscale, kernels.EPI_SILU_MUL)
+                nxt = self.layers[i + 1].input_layernorm if i + 1 < len(self.layers) else self.norm
+                h = kernels.int8_linear_add_rmsnorm(act, dn.qweight, dn.kscale, x, nxt.weight, nxt.eps)
+        return kernels.rmsnorm(x, self.norm.weight, self.norm.eps) if inside else h
 
     def _token_split_layers(
         self, input_ids: Tensor, positions: Tensor, kv_caches: list[tuple[Tensor, Tensor]], meta: AttentionMetadata

@@ -1,0 +1,118 @@
+"""GPU parity of the wide decode linear (gemv_wide.hip), which msa_int8_linear takes for up to 64 tokens
+over weights of 12 MB and more (and msa_int8_linear_add_rmsnorm with it, in one launch or merging
+split-K partials), against the CPU oracle on the same seeded inputs; and of the large-weight decode
+layers against the general layer loop.
+
+Same operands and rounding points as the oracle's bf16 product, float32 accumulation in another
+order: within rel-L2 2e-3 of the oracle and within one bf16 rounding (4e-3) of float64, as the other
+decode linears. Shapes take every unit width (1, 2, 3, 6 tiles) and token-tile count, ragged last
+units, K whose chunks do not deal evenly to the eight wavefronts, 1 and 64 tokens."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+from helpers import rel_l2
+
+from miniserve_amd import _native, kernels, workloads
+from miniserve_amd.quant.int8 import quantize_int8_
+from miniserve_amd.runner.model_runner import ModelRunner, ScheduledChunk
+from oracle import int8 as oi
+from oracle import layers as ol
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _bf16(shape, seed, std=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * std).to(torch.bfloat16)
+
+
+WIDE_SHAPES = [  # (m, n, k)
+    (1, 4090, 4160),  # one tile per unit, ragged n, 65 chunks
+    (16, 3072, 4160),
+    (5, 6150, 3136),  # two tiles, 49 chunks
+    (13, 12290, 1088),  # three tiles, 17 chunks
+    (17, 4096, 3136),
+    (32, 6144, 3136),
+    (20, 12280, 1088),
+    (32, 24560, 576),  # six tiles, 9 chunks
+    (33, 4096, 3136),
+    (47, 6150, 3136),
+    (48, 12290, 1088),
+    (49, 4090, 3136),
+    (64, 6144, 3136),
+    (63, 12290, 1088),
+    (32, 2048, 8256),  # split K, merged by the epilogue kernel
+    (64, 1600, 8256),
+]
+
+
+@pytest.mark.parametrize("m,n,k", WIDE_SHAPES)
+def test_wide_linear(m, n, k):
+    assert n * k >= kernels.WIDE_MIN_WEIGHTS
+    q, s = oi.quantize_int8(_bf16((n, k), seed=n + k, std=0.02))
+    x, r = _bf16((m, k), seed=m), _bf16((m, n), seed=m + 1)
+    xd, qd, sd, rd = (t.to(DEV) for t in (x, q, s, r))
+    y = kernels.int8_linear(xd, qd, sd)
+    assert torch.equal(y, kernels.int8_linear(xd, qd, sd))
+    exact = x.double() @ oi.dequantize(q, s, torch.bfloat16).double().T
+    assert rel_l2(y.cpu(), oi.int8_linear(x, q, s)) < 2e-3
+    assert rel_l2(y.cpu(), exact) < 4e-3
+    # without a workspace: one launch, K never split; strided x and y rows
+    xs = torch.zeros(m, k + 64, dtype=torch.bfloat16, device=DEV)
+    xs[:, :k] = xd
+    y2 = torch.zeros(m, n + 8, dtype=torch.bfloat16, device=DEV)
+    _native.call("msa_int8_linear", kernels._ptr(xs), m, k, k + 64, kernels._ptr(qd), kernels._ptr(sd), n,
+                 kernels._ptr(y2), n + 8, 0, None, 0, None, 0, kernels._stream(y2))
+    assert rel_l2(y2[:, :n].cpu(), exact) < 4e-3 and not y2[:, n:].any()
+    # residual added to the rounded product, in place
+    acc = rd.clone()
+    kernels.int8_linear(xd, qd, sd, kernels.EPI_RESIDUAL, residual=acc, out=acc)
+    assert torch.equal(acc, (rd.float() + y.float()).to(torch.bfloat16))
+    # silu(gate) * up of the two halves
+    gate, up = exact.to(torch.bfloat16).chunk(2, dim=-1)
+    act = kernels.int8_linear(xd, qd, sd, kernels.EPI_SILU_MUL)
+    assert rel_l2(act.cpu(), torch.nn.functional.silu(gate) * up) < 8e-3
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4096, 4160), (16, 2048, 8256), (17, 4096, 3136), (40, 2048, 8256), (64, 2568, 4992)])
+def test_wide_linear_add_rmsnorm(m, n, k):
+    q, s = oi.quantize_int8(_bf16((n, k), seed=n + k, std=0.02))
+    x, r, w = _bf16((m, k), seed=m), _bf16((m, n), seed=m + 1), _bf16((n,), seed=3, std=0.1) + 1
+    res = r.to(DEV)
+    out = kernels.int8_linear_add_rmsnorm(x.to(DEV), q.to(DEV), s.to(DEV), res, w.to(DEV), 1e-6)
+    ref = r + oi.int8_linear(x, q, s)
+    assert rel_l2(res.cpu(), ref) < 2e-3
+    assert rel_l2(out.cpu(), ol.rms_norm(res.cpu(), w, 1e-6)) < 2e-3  # of its own sum: the order of squares
+
+
+@pytest.mark.parametrize("batch", [1, 16, 17, 64, 70])
+def test_wide_decode_layers_match_the_layer_loop(batch, monkeypatch):
+    """The large-weight decode layers against the general loop on the same model and pool: the same
+    values but for the orders of float32 sums, amplified by bf16 roundings over two layers (each
+    route measures about 1.4e-2 from float64 on this shape)."""
+    cfg = {**workloads.QWEN3_8B, "num_hidden_layers": 2, "vocab_size": 512, "tie_word_embeddings": True}
+    model = workloads.build_model(cfg, workloads.random_weights(cfg, 5, norm_jitter=0.1, device="cuda"), DEV, 256)
+    quantize_int8_(model)
+    runner = ModelRunner(model, DEV, max_model_len=256)
+    ctx = [3 + (37 * i) % 200 for i in range(batch)]
+    blocks = [-(-c // 16) for c in ctx]
+    perm = torch.randperm(sum(blocks), generator=torch.Generator().manual_seed(1)).tolist()
+    tables, off = [], 0
+    for b in blocks:
+        tables.append(perm[off : off + b])
+        off += b
+    sched = [ScheduledChunk([(7 * i + j) % 512 for j in range(c)], c - 1, 1, t) for i, (c, t) in enumerate(zip(ctx, tables))]
+    got = []
+    for wide in (True, False):
+        if not wide:
+            monkeypatch.setattr(type(model), "_wide_decode_ok", lambda self, tokens, meta: False)
+        runner.allocate_kv_cache(sum(blocks))
+        workloads.fill_kv_pool_(runner.kv_cache, 9, on_device=True)
+        inp = runner.prepare(sched)
+        assert model._wide_decode_ok(batch, inp.attn) is wide
+        with torch.inference_mode():
+            got.append((model(inp.input_ids, inp.positions, runner.kv_caches, inp.attn), runner.kv_cache.clone()))
+    assert rel_l2(got[0][0].cpu(), got[1][0].cpu()) < 2e-2
+    assert rel_l2(got[0][1].cpu(), got[1][1].cpu()) < 5e-3
