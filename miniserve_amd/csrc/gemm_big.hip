@@ -1,27 +1,32 @@
-// Int8 weight-only linear for large prefill GEMMs: 256-token tiles, eight wavefronts per
-// workgroup (two per SIMD).
+// Int8 weight-only linear for large prefill GEMMs: 256-token tiles, eight or sixteen wavefronts per
+// workgroup (two or four per SIMD).
 //
 // y[m, n] = sum_k x[m, k] * bf16(q[n, k] * s[n]) with float32 accumulation, as Int8Linear.forward
 // (quant/int8.py:35-37) computes it -- the same operands and rounding points as the 128 x 128 GEMM
 // (gemm_int8.hip); only the tiling differs.
 //
 // Why a second tiling: a wavefront tile of TM x TN reads (TM + TN) x K operand bytes from LDS for
-// TM x TN x K MACs, so 128 x 64 wavefront tiles of 32 x 32 x 16 MFMAs read 3/4 of the LDS bytes
-// per flop of the 128 x 128 tiling's 64 x 64 ones, and a 256-token tile dequantizes each weight
-// once per 256 tokens instead of per 128. Two wavefronts per SIMD (their accumulators in ordinary
-// registers) let one issue MFMAs while the other waits on LDS or stages the next K step: against
-// four wavefronts of 128 x 128 quarters (one per SIMD) the 256 x 256 tile runs 18% faster at
-// M = 2048, K = 1024 and 13% faster at K = 4096.
+// TM x TN x K MACs, and a 256-token tile dequantizes each weight once per 256 tokens instead of per
+// 128.
 //
-//  * Workgroup = 8 wavefronts (WM x WN) over 256 tokens x BN weight rows: 256 x 256 (2 x 4
-//    wavefronts of 128 x 64), 256 x 192 (4 x 2 of 64 x 96) or 256 x 128 (4 x 2 of 64 x 64); the
-//    host picks the one that fills the most of the 256 CUs. Per 64-wide K step the workgroup stages
-//    the x tile (256 x 64 bf16, 32 KB) and the dequantized q tile (BN x 64 -> bf16) in LDS, double
-//    buffered, the next step's global loads in registers during the MFMAs, the staging into LDS
-//    split into four parts placed after the step's 16-wide K slices. On the 256 x 192 and
-//    256 x 128 tilings each slice's MFMA fragments are read from LDS before the previous slice's
-//    MFMAs issue (two fragment sets), and the step's barrier sits before its last slice, whose
-//    MFMAs cover the read of the next step's first slice.
+//  * Workgroup = WM x WN wavefronts over 256 tokens x BN weight rows: 256 x 256 (2 x 4 wavefronts of
+//    128 x 64), 256 x 192 (8 x 2 of 32 x 96) or 256 x 128 (4 x 4 of 64 x 32); the host picks the one
+//    that fills the most of the 256 CUs. Per 64-wide K step the workgroup stages the x tile (256 x 64
+//    bf16, 32 KB) and the dequantized q tile (BN x 64 -> bf16) in LDS, double buffered. A piece's
+//    registers are reloaded for the step after next right after they are stored, so every load has a
+//    whole step to arrive (8B-shaped gate_up at 4096 tokens 719 us with the loads at the step's end,
+//    704 with this).
+//    (256 x 128 with the residual epilogue: 4 x 2 of 64 x 64.)
+//  * What bounds it: no unit alone. Per step of a 256 x 128 tile (about 1 us) the MFMAs take 0.47 us
+//    of each SIMD, LDS reads 0.34 (1.75 ns per 1 KB read instruction) and writes 0.28 (5.8 ns each),
+//    dequantization 0.17; wavefronts that leave a barrier together do the same thing at the same time.
+//    Sixteen wavefronts with each slice's fragments read before the previous slice's MFMAs issue
+//    overlap them best on the narrow tiles (gate_up at 256 tokens 69.6 us with eight, 69.9 with
+//    sixteen that read their own slice's fragments, 65.2 with sixteen that read ahead; qkv at 4096
+//    212, 212, 200). On 256 x 256 tiles (128 accumulators a lane) eight wavefronts that read a slice's
+//    fragments just before its MFMAs are faster (4096 tokens: 704 us; sixteen 766; reading ahead
+//    747; the two wavefronts of a SIMD in alternate memory and MFMA phases 800-821; MFMAs at a raised
+//    wavefront priority 784).
 //  * Epilogues: bf16 store; residual add (in place allowed); silu(gate) * up with each
 //    wavefront's TN weight rows laid out as TN / 2 gate rows then their TN / 2 up rows. Results go
 //    through LDS so that each lane writes 16 contiguous bytes (gate and up meet there).
@@ -74,15 +79,16 @@ __device__ __forceinline__ int big_wrow(const BigGemmArgs& a, int nb, int r) {
   }
 }
 
-template <int BN, int WM, int EPI>
-__global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
-  constexpr int WN = 8 / WM;
+template <int BN, int WM, int WN, int EPI>
+__global__ __launch_bounds__(64 * WM * WN) void int8_gemm256_kernel(BigGemmArgs a) {
+  constexpr int NTH = 64 * WM * WN;     // threads
+  constexpr int AR = kBM * 8 / NTH;     // 16-byte x pieces per thread per K step
   constexpr int TM = kBM / WM, TN = BN / WN;  // wavefront tile
   constexpr int MT = TM / 32, NT = TN / 32;   // 32 x 32 accumulator tiles
-  static_assert(WM * WN == 8 && TM % 32 == 0 && TN % 32 == 0, "eight wavefronts of 32 x 32 tiles");
+  static_assert((NTH == 512 || NTH == 1024) && TM % 32 == 0 && TN % 32 == 0, "wavefronts of 32 x 32 tiles");
   static_assert(EPI != MSA_EPI_SILU_MUL || (TN / 2) % 8 == 0, "gate and up halves in 16-byte pieces");
-  constexpr int BCH = (BN * 4 + 511) / 512;  // 16-byte weight chunks per thread per K step
-  static_assert(BCH <= 2, "weight chunks fit parts 2 and 3");
+  constexpr int BCH = (BN * 4 + NTH - 1) / NTH;  // 16-byte weight chunks per thread per K step
+  static_assert(AR <= 4 && BCH <= 2, "two parts of x pieces, two of weight chunks");
   extern __shared__ __attribute__((aligned(16))) uint16_t bsm[];
   uint16_t* As = bsm;                   // [2][256][kBLd]
   uint16_t* Bs = bsm + 2 * kBM * kBLd;  // [2][BN][kBLd]
@@ -97,48 +103,48 @@ __global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
   const int m0 = mb * kBM;
   const uint32_t kbase = (uint32_t)ks * (uint32_t)a.k_per;  // this split's first K element
 
-  // Loader roles. A: rows tid / 8 + 64 i (i < 4), 8-element chunk tid % 8. B: chunk
-  // c = tid + 512 i (c < 4 BN): row c / 4, 16-byte piece c % 4.
+  // Loader roles. A: rows tid / 8 + NTH / 8 i (i < AR), 8-element chunk tid % 8. B: chunk
+  // c = tid + NTH i (c < 4 BN): row c / 4, 16-byte piece c % 4.
   const int ar = tid >> 3, ac = (tid & 7) * 8;
   // 32-bit byte offsets from the uniform base pointers (the caller checks that they fit): half the
   // registers of per-row 64-bit pointers.
-  uint32_t aoff[4];
+  uint32_t aoff[AR];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = min(m0 + ar + 64 * i, a.m - 1);  // rows past m repeat row m - 1; outputs dropped
+  for (int i = 0; i < AR; ++i) {
+    const int row = min(m0 + ar + NTH / 8 * i, a.m - 1);  // rows past m repeat row m - 1; outputs dropped
     aoff[i] = (uint32_t)(row * (uint32_t)a.ldx + ac + kbase) * 2u;
   }
   uint32_t boff[BCH];
   float bs[BCH];
 #pragma unroll
   for (int i = 0; i < BCH; ++i) {
-    const int c = min(tid + 512 * i, BN * 4 - 1);  // chunks past the tile reload the last one (not stored)
+    const int c = min(tid + NTH * i, BN * 4 - 1);  // chunks past the tile reload the last one (not stored)
     int row = big_wrow<BN, TN, EPI>(a, nb, c / 4);
     row = row < a.n ? row : a.n - 1;
     boff[i] = (uint32_t)row * (uint32_t)a.k + kbase + (c % 4) * 16;
     bs[i] = bf16_to_f32(a.scale[row]);
   }
-  // One register set: a step's global loads are issued at the end of the step before the one that
-  // stages them. (A second set, loads two steps ahead, exceeds the 256 registers of two
-  // wavefronts per SIMD.)
-  u32x4 ra[4], rb[BCH];  // native vectors: a struct-typed array stays in private memory
-  auto load_step = [&](int k0) {
+  // A step's global loads in registers, in four parts: p = 0, 1 the halves of the x pieces, p = 2, 3
+  // the weight chunks p - 2 (of BCH).
+  u32x4 ra[AR], rb[BCH];  // native vectors: a struct-typed array stays in private memory
+  auto load_part = [&](int k0, int p) {
+    if (p < 2) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ra[i] = *(const u32x4*)((const char*)a.x + aoff[i] + 2u * k0);
-#pragma unroll
-    for (int i = 0; i < BCH; ++i) rb[i] = *(const u32x4*)((const char*)a.w + boff[i] + k0);
+      for (int i = AR / 2 * p; i < AR / 2 * (p + 1); ++i) ra[i] = *(const u32x4*)((const char*)a.x + aoff[i] + 2u * k0);
+    } else if (p - 2 < BCH) {
+      rb[p - 2] = *(const u32x4*)((const char*)a.w + boff[p - 2] + k0);
+    }
   };
-  // Part p of the staged step into LDS buffer buf: p = 0, 1 the x rows 2p, 2p + 1 (of 4); p = 2, 3
-  // the weight chunk p - 2 (of BCH), dequantized.
+  // Part p into LDS buffer buf, the weights dequantized.
   auto store_part = [&](int buf, int p) {
     if (p < 2) {
       uint16_t* A_ = As + buf * kBM * kBLd + ar * kBLd + ac;
 #pragma unroll
-      for (int i = 2 * p; i < 2 * p + 2; ++i) *(u32x4*)(A_ + 64 * i * kBLd) = ra[i];
+      for (int i = AR / 2 * p; i < AR / 2 * (p + 1); ++i) *(u32x4*)(A_ + NTH / 8 * i * kBLd) = ra[i];
     } else if (p - 2 < BCH) {
       const int i = p - 2;
-      const int c = tid + 512 * i;
-      if (BN * 4 % 512 == 0 || c < BN * 4) {
+      const int c = tid + NTH * i;
+      if (BN * 4 % NTH == 0 || c < BN * 4) {  // (a whole wavefront takes one side)
         uint16_t* B_ = Bs + buf * BN * kBLd + (c / 4) * kBLd + (c % 4) * 16;
         // An empty asm redefines rb[i] here, so the compiler cannot start dequantizing the next
         // step's bytes before the barrier that ends the current one (a wait on loads just issued).
@@ -179,14 +185,15 @@ __global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
   // Top of step kt: LDS buffer kt & 1 holds step kt and the registers step kt + 1. Loads and
   // stores are unconditional (the last steps reload step nk - 1 and stage it into the idle
   // buffer: in bounds, never used) so the prefetch registers stay registers.
-  load_step(0);
 #pragma unroll
-  for (int p = 0; p < 4; ++p) store_part(0, p);
-  load_step(min(1, nk - 1) * kBK);
+  for (int p = 0; p < 4; ++p) load_part(0, p);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    store_part(0, p);
+    load_part(min(1, nk - 1) * kBK, p);
+  }
   __syncthreads();
   if constexpr (BN == 256) {
-    // 128 x 64 wavefront tiles: each slice's eight MFMAs cover its own fragment reads; a second
-    // fragment set would take these wavefronts to 242 registers and measured slower.
     for (int kt = 0; kt < nk; ++kt) {
       const int cur = kt & 1;
 #pragma unroll
@@ -195,17 +202,17 @@ __global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
         read_frags(cur, ks, af, bfr);
         mfmas(af, bfr);
         store_part(cur ^ 1, ks);  // step kt + 1 into the other buffer
+        load_part(min(kt + 2, nk - 1) * kBK, ks);
         __builtin_amdgcn_sched_barrier(0);  // keeps each slice's fragments and staging with its MFMAs
       }
-      load_step(min(kt + 2, nk - 1) * kBK);
       __syncthreads();
     }
   } else {
     // Two fragment sets: each slice's LDS reads are issued before the previous slice's MFMAs.
-    // Slices 0 and 1 stage step kt + 1 into the other buffer, then the registers take step
-    // kt + 2; the barrier before slice 3 publishes the staged step (and ends every read of the
-    // buffer the next step overwrites), and slice 3's MFMAs cover the read of the next step's
-    // first slice (at the last step a read of the idle buffer, not used).
+    // Slices 0 and 1 stage step kt + 1 into the other buffer and reload the registers; the barrier
+    // before slice 3 publishes the staged step (and ends every read of the buffer the next step
+    // overwrites), and slice 3's MFMAs cover the read of the next step's first slice (at the last
+    // step a read of the idle buffer, not used).
     bf16x8 af[2][MT], bfr[2][NT];
     read_frags(0, 0, af[0], bfr[0]);
     for (int kt = 0; kt < nk; ++kt) {
@@ -220,10 +227,12 @@ __global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
         }
         mfmas(af[ks & 1], bfr[ks & 1]);
         if (ks < 2) {
-          store_part(cur ^ 1, ks);
-          store_part(cur ^ 1, ks + 2);
+#pragma unroll
+          for (int p = 2 * ks; p < 2 * ks + 2; ++p) {
+            store_part(cur ^ 1, p);
+            load_part(min(kt + 2, nk - 1) * kBK, p);
+          }
         }
-        if (ks == 1) load_step(min(kt + 2, nk - 1) * kBK);
         __builtin_amdgcn_sched_barrier(0);  // keeps each slice's reads and staging with its MFMAs
       }
     }
@@ -265,7 +274,7 @@ __global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
         for (int nt = 0; nt < NT; ++nt) c[nt * 32] = f32_to_bf16(acc[mt][nt][i]);
       }
     __syncthreads();
-    qk_norm_rope_tile<512, kBM>(a.qk, bsm, kQLd, nb, m0, a.m, tid);
+    qk_norm_rope_tile<NTH, kBM>(a.qk, bsm, kQLd, nb, m0, a.m, tid);
     return;
   }
 
@@ -275,7 +284,7 @@ __global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
   // in tile (mt, nt) is token row mt*32 + 8(i/4) + 4h + i%4 and weight row nt*32 + r of the
   // wavefront's TN.
   constexpr int kCLd = TN + 8;
-  static_assert((size_t)8 * TM * kCLd * 2 <= big_lds_bytes<BN>(), "epilogue staging fits the tile buffers");
+  static_assert((size_t)WM * WN * TM * kCLd * 2 <= big_lds_bytes<BN>(), "epilogue staging fits the tile buffers");
   uint16_t* Cs = bsm + wave * TM * kCLd;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -332,15 +341,12 @@ __global__ __launch_bounds__(512) void int8_gemm256_kernel(BigGemmArgs a) {
 
 // ---- host side ----------------------------------------------------------------------------------
 
-struct BigTiling {
-  int bn, wm;  // weight rows per tile, wavefront rows (of 8 wavefronts)
-};
-// In order of preference when two fill the chip equally (larger wavefront tiles first).
-constexpr BigTiling kBigTilings[] = {{256, 2}, {192, 4}, {128, 4}};
+// Weight rows per tile, in order of preference when two fill the chip equally (larger tiles first).
+constexpr int kBigTilings[] = {256, 192, 128};
 constexpr int kBigTilingCount = 3;
 
 static int64_t big_n_blocks(int t, int64_t n, int epilogue) {
-  const int bn = kBigTilings[t].bn;
+  const int bn = kBigTilings[t];
   return epilogue == MSA_EPI_SILU_MUL ? (n / 2 + bn / 2 - 1) / (bn / 2) : (n + bn - 1) / bn;
 }
 
@@ -366,22 +372,24 @@ int gemm256_pick(int64_t m, int64_t n, int64_t k, int epilogue, int64_t* tiles) 
   return best;
 }
 
-template <int BN, int WM, int EPI>
+template <int BN, int WM, int WN, int EPI>
 static int launch_big(const BigGemmArgs& a, int blocks, hipStream_t s) {
   constexpr size_t lds = big_lds_bytes<BN>();
-  auto kernel = int8_gemm256_kernel<BN, WM, EPI>;
+  auto kernel = int8_gemm256_kernel<BN, WM, WN, EPI>;
   const int rc = allow_dynamic_lds((const void*)kernel, (int)lds, "int8_gemm256_kernel");
   if (rc != MSA_OK) return rc;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(512), lds, s, a);
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * WM * WN), lds, s, a);
   return check_launch("msa_int8_gemm (256-token tiles)");
 }
 
-template <int BN, int WM>
+template <int BN, int WM, int WN>
 static int launch_big_epi(const BigGemmArgs& a, int blocks, int epilogue, hipStream_t s) {
   switch (epilogue) {
-    case MSA_EPI_NONE: return launch_big<BN, WM, MSA_EPI_NONE>(a, blocks, s);
-    case MSA_EPI_SILU_MUL: return launch_big<BN, WM, MSA_EPI_SILU_MUL>(a, blocks, s);
-    default: return launch_big<BN, WM, MSA_EPI_RESIDUAL>(a, blocks, s);
+    case MSA_EPI_NONE: return launch_big<BN, WM, WN, MSA_EPI_NONE>(a, blocks, s);
+    case MSA_EPI_SILU_MUL: return launch_big<BN, WM, WN, MSA_EPI_SILU_MUL>(a, blocks, s);
+    default:
+      if constexpr (BN == 128) return fail(MSA_ERR_INVALID, "msa_int8_gemm: residual tiling");
+      else return launch_big<BN, WM, WN, MSA_EPI_RESIDUAL>(a, blocks, s);
   }
 }
 
@@ -400,9 +408,12 @@ int gemm256_run(int t, const uint16_t* x, int64_t m, int64_t k, int64_t ldx, con
   const int64_t blocks = (int64_t)((a.n_blocks + 7) / 8) * 8 * a.m_blocks;
   if (blocks > 0x7fffffff) return fail(MSA_ERR_INVALID, "msa_int8_gemm: too many tiles");
   switch (t) {
-    case 0: return launch_big_epi<256, 2>(a, (int)blocks, epilogue, s);
-    case 1: return launch_big_epi<192, 4>(a, (int)blocks, epilogue, s);
-    default: return launch_big_epi<128, 4>(a, (int)blocks, epilogue, s);
+    case 0: return launch_big_epi<256, 2, 4>(a, (int)blocks, epilogue, s);
+    case 1: return launch_big_epi<192, 8, 2>(a, (int)blocks, epilogue, s);
+    default:
+      // o / down: eight wavefronts (8B o at 2048 tokens 71.8 us, sixteen 74.3; down 209, 213)
+      if (epilogue == MSA_EPI_RESIDUAL) return launch_big<128, 4, 2, MSA_EPI_RESIDUAL>(a, (int)blocks, s);
+      return launch_big_epi<128, 4, 4>(a, (int)blocks, epilogue, s);
   }
 }
 
@@ -420,7 +431,7 @@ int gemm256_qk_norm_run(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, co
   a.qk = qk;
   const int64_t blocks = (int64_t)((a.n_blocks + 7) / 8) * 8 * a.m_blocks;
   if (blocks > 0x7fffffff) return fail(MSA_ERR_INVALID, "msa_int8_gemm_qk_norm_rope_cache: too many tiles");
-  return launch_big<128, 4, kEpiQkNorm>(a, (int)blocks, s);
+  return launch_big<128, 4, 4, kEpiQkNorm>(a, (int)blocks, s);
 }
 
 // Split-K on 256 x 128 tiles for shapes with too few output tiles to fill the chip unsplit and a
@@ -455,7 +466,7 @@ int gemm256_partials_run(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, c
   a.part = part;
   const int64_t blocks = (int64_t)((a.n_blocks + 7) / 8) * 8 * splits * a.m_blocks;
   if (blocks > 0x7fffffff) return fail(MSA_ERR_INVALID, "msa_int8_gemm: too many tiles");
-  return launch_big<128, 4, kBigEpiPartial>(a, (int)blocks, s);
+  return launch_big<128, 4, 4, kBigEpiPartial>(a, (int)blocks, s);
 }
 
 }  // namespace msa
