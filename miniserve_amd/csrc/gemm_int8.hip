@@ -311,21 +311,30 @@ static int splits256(int64_t m, int64_t n, int64_t k, int64_t ldx) {
   return gemm256_split_plan(m, n, k);
 }
 
+// Splits on the 256 x 128 tiles where their number is past what splits128 would split but leaves
+// much of the chip idle in one unsplit round (96 to 128 tiles on 256 CUs): two splits fill 192 to 256
+// of them in one round. 8B-shaped o at 768 / 1024 tokens 52 / 57 us unsplit, 48 / 56 in two splits
+// and their merge (with the next norm 56 / 61 and 45 / 51); down 140 / 151, 106 / 123.
+static int splits_mid(int64_t m, int64_t n, int64_t k, int epilogue) {
+  if (epilogue == MSA_EPI_SILU_MUL || m < 192) return 1;
+  const int64_t tiles = ((n + 127) / 128) * ((m + 255) / 256);
+  return tiles >= 96 && tiles <= 128 && gemm256_split_plan(m, n, k) == 2 ? 2 : 1;
+}
+
 // The split count of a GEMM that splits K (1: unsplit): the 256 x 128 tiles' plan where it applies
-// (eight wavefronts per workgroup, two per SIMD), else the 128 x 128 tiles' (four wavefronts).
+// (sixteen wavefronts per workgroup), else the 128 x 128 tiles' (four wavefronts).
 int gemm_splits(int64_t m, int64_t n, int64_t k, int epilogue) {
-  if (splits128(m, n, k, epilogue) <= 1) return 1;
+  const int s128 = splits128(m, n, k, epilogue);
+  if (s128 <= 1) return splits_mid(m, n, k, epilogue);
   const int s256 = gemm256_split_plan(m, n, k);
-  return s256 > 1 ? s256 : splits128(m, n, k, epilogue);
+  return s256 > 1 ? s256 : s128;
 }
 
 // Partials for either plan (the 128 x 128 one serves when x's pitch is too large for the 256-token
 // kernel's 32-bit offsets).
 size_t gemm_workspace_size(int64_t m, int64_t n, int64_t k, int epilogue) {
-  const int s128 = splits128(m, n, k, epilogue);
-  if (s128 <= 1) return 0;
-  const int s = std::max(s128, gemm256_split_plan(m, n, k));
-  return (size_t)s * m * n * sizeof(float);
+  const int splits = std::max(gemm_splits(m, n, k, epilogue), splits128(m, n, k, epilogue));
+  return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
 }
 
 // The 256-token tilings (gemm_big.hip): the best-filling one and its tile count, and the GEMM on it.
@@ -378,12 +387,16 @@ int gemm_run(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t*
   a.n_blocks = (int)(epilogue == MSA_EPI_SILU_MUL ? (n / 2 + 63) / 64 : (n + kGBN - 1) / kGBN);
   a.m_blocks = (int)((m + kGBM - 1) / kGBM);
   int splits = gemm_splits(m, n, k, epilogue);
-  const int big = splits == 1 ? use_gemm256(m, n, k, ldx, epilogue) : -1;
-  if (big >= 0) return gemm256_run(big, x, m, k, ldx, qweight, scale, n, y, ldy, epilogue, residual, ldr, s);
+  // The middle shapes' two splits pay without the fused norm only over a long K (0.6B o / down at 4096
+  // tokens, K = 2048 / 3072: 33 / 47 us unsplit, 42 / 53 split; with the norm 39 / 51 and 38 / 48).
+  if (splits > 1 && splits128(m, n, k, epilogue) <= 1 && k < 4096) splits = 1;
+  const bool unsplit_plan = splits == 1 || splits128(m, n, k, epilogue) <= 1;  // planned unsplit but for splits_mid
   if (splits > 1 && (!workspace || workspace_bytes < gemm_workspace_size(m, n, k, epilogue) || !aligned16(workspace)))
     splits = 1;
   const int s256 = splits > 1 ? splits256(m, n, k, ldx) : 0;
   if (splits > 1 && s256 <= 1) splits = splits128(m, n, k, epilogue);
+  const int big = splits == 1 && unsplit_plan ? use_gemm256(m, n, k, ldx, epilogue) : -1;
+  if (big >= 0) return gemm256_run(big, x, m, k, ldx, qweight, scale, n, y, ldy, epilogue, residual, ldr, s);
   a.k_per = (int)(k / splits);
   a.part = (float*)workspace;
   const int64_t blocks = (int64_t)a.n_blocks * a.m_blocks * splits;
@@ -423,6 +436,7 @@ int gemm_run_partials(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, cons
   const int s256 = splits256(m, n, k, ldx);
   if (s256 > 1) return gemm256_partials_run(x, m, k, ldx, qweight, scale, n, s256, part, s) == MSA_OK ? s256 : -1;
   const int splits = splits128(m, n, k, MSA_EPI_NONE);
+  if (splits <= 1) return 1;
   GemmArgs a{};
   a.x = x; a.ldx = ldx; a.w = qweight; a.scale = scale;
   a.m = (int)m; a.n = (int)n; a.k = (int)k;
