@@ -326,6 +326,13 @@ int msa_paged_attention_prefill(const uint16_t* q, int64_t ldq, const uint16_t* 
                                 int head_dim, int block_size, const int32_t* block_tables, int max_blocks,
                                 const int32_t* seq_info, const int32_t* work, int num_work, float scale,
                                 uint16_t* out, int64_t ldo, msa_stream_t stream);
+/* The same on query tiles of twice the tokens (work lists of 128 / (heads / kv_heads) tokens): for
+ * batches with enough tiles to fill the chip. */
+int msa_paged_attention_prefill_wide(const uint16_t* q, int64_t ldq, const uint16_t* k_cache,
+                                     const uint16_t* v_cache, int64_t num_slots, int heads, int kv_heads,
+                                     int head_dim, int block_size, const int32_t* block_tables, int max_blocks,
+                                     const int32_t* seq_info, const int32_t* work, int num_work, float scale,
+                                     uint16_t* out, int64_t ldo, msa_stream_t stream);
 
 /* ---- sampling (runner/sampler.py) ------------------------------------------------------------ */
 

@@ -29,6 +29,14 @@ from miniserve_amd.utils import upload_int32
 SHORT_QUERY = 8  # the reference's batched-path threshold (backends.py:32); kept for callers
 MAX_GATHER_TOKENS = 16384  # the reference's gather cap (backends.py:33); nothing is gathered here
 PREFILL_TILE = {1: 64, 2: 32, 4: 16}  # query tokens per prefill work item, by H / KVH
+# Tiles of twice the tokens (32-query wavefronts) when they give at least this many workgroups, three
+# for every two CUs: each key and value read from LDS then serves twice the queries (2000 tokens
+# after 6000 at 32 / 8 heads, 504 workgroups: 376 -> 272 us; 2 x 2048 fresh at 16 / 8 heads, 512:
+# 77 -> 56). With fewer, the longer chains of the larger tiles cost more than they save (1984 fresh
+# tokens at 16 / 8 heads, 248: 38 -> 42; 500 at 32 / 8, 128: 12.5 -> 16.3), and where the tokens do not
+# fill them they only double the padding (64 x 4 tokens: 58 -> 65).
+PREFILL_WIDE_MIN_WORKGROUPS = 384
+PREFILL_TILE_SIZES = tuple(sorted({f * t for t in PREFILL_TILE.values() for f in (1, 2)}))  # every plan's work lists
 
 
 @dataclass
@@ -138,7 +146,7 @@ def build_attention_metadata(
     if pre:
         add("p_info", np.array([[c.flat_start, c.num_new, c.num_cached] for c in pre], dtype=np.int32))
         add("p_tables", _padded_tables(pre, block_size))
-        for tile in sorted(set(PREFILL_TILE.values())):
+        for tile in PREFILL_TILE_SIZES:
             add(f"p_work{tile}", _prefill_work(pre, tile))
 
     flat = upload_int32(np.concatenate(parts), device) if parts else None
@@ -162,14 +170,11 @@ def metadata_from_parts(
         DecodePlan(views["d_rows"], views["d_ctx"], views["d_tables"], split_context) if "d_rows" in views else None
     )
     prefill = (
-        PrefillPlan(views["p_info"], views["p_tables"], {t: views[f"p_work{t}"] for t in set(PREFILL_TILE.values())})
+        PrefillPlan(views["p_info"], views["p_tables"], {t: views[f"p_work{t}"] for t in PREFILL_TILE_SIZES})
         if "p_info" in views
         else None
     )
     return AttentionMetadata(slot_mapping, block_size, decode, prefill)
-
-
-PREFILL_TILE_SIZES = tuple(sorted(set(PREFILL_TILE.values())))  # the work lists every plan carries
 
 
 _SIDE_STREAMS: dict[int, tuple[torch.cuda.Stream, torch.cuda.Event, torch.cuda.Event]] = {}
@@ -187,13 +192,22 @@ def _side_stream(device: torch.device) -> tuple[torch.cuda.Stream, torch.cuda.Ev
     return st
 
 
+def prefill_takes_wide(plan: PrefillPlan, tile: int, kv_heads: int) -> bool:
+    """Whether a prefill plan runs on tiles of 2 x ``tile`` tokens: enough of them, and well filled
+    (at most three for every four of the small ones)."""
+    work = plan.work.get(2 * tile)
+    return (work is not None and work.shape[0] * kv_heads >= PREFILL_WIDE_MIN_WORKGROUPS
+            and 4 * work.shape[0] <= 3 * plan.work[tile].shape[0])
+
+
 def attend(q: Tensor, k_cache: Tensor, v_cache: Tensor, meta: AttentionMetadata, scale: float) -> Tensor:
     """Attention of every new token over its cached context (the caches already hold this
     step's keys and values). q [T, H, D] -> [T, H, D].
 
     In a mixed batch the decode rows (HBM-bound) run on a second stream next to the prefill rows
     (MFMA-bound), in four-wavefront workgroups that fit on a CU beside a prefill workgroup; the two
-    write disjoint rows of the output, and the caller's stream waits for both."""
+    write disjoint rows of the output, and the caller's stream waits for both. The wide prefill
+    tiles' wavefronts leave no registers for a decode workgroup, so mixed batches keep the small ones."""
     out = torch.empty_like(q)
     heads, kv_heads = q.shape[1], k_cache.shape[1]
     side = cur = join = None
@@ -216,8 +230,9 @@ def attend(q: Tensor, k_cache: Tensor, v_cache: Tensor, meta: AttentionMetadata,
         tile = PREFILL_TILE.get(group)
         if tile is None:
             raise RuntimeError(f"prefill attention supports H/KVH in 1, 2, 4 (got {group})")
-        kernels.paged_attention_prefill(q, k_cache, v_cache, p.block_tables, p.seq_info, p.work[tile], scale, out,
-                                        meta.block_size)
+        wide = side is None and prefill_takes_wide(p, tile, kv_heads)  # (beside decode rows: see above)
+        kernels.paged_attention_prefill(q, k_cache, v_cache, p.block_tables, p.seq_info,
+                                        p.work[2 * tile if wide else tile], scale, out, meta.block_size, wide)
     if side is not None:
         join.record(side)
         cur.wait_event(join)

@@ -750,9 +750,241 @@ __global__ __launch_bounds__(256 * kKeyGroups) __attribute__((amdgpu_waves_per_e
   }
 }
 
+// The same attention on 32-query wavefront tiles (v_mfma_f32_32x32x16_bf16): every K and V^T fragment
+// read from LDS feeds twice the queries, and a query's keys lie in two lanes instead of four. The
+// 16-query kernel is bound by LDS and VALU (per 32-key tile and wavefront 41 ns of LDS reads, its share
+// of the stores and ~40 ns of softmax against 33 ns of MFMA); here the reads, the maxima and the tile's
+// bookkeeping serve two times the MFMAs: 2000 tokens after 6000 at 32 / 8 heads 376 -> 272 us (0.61 ->
+// 0.84 PFLOP/s), 2 x 2048 fresh tokens 152 -> 106. 163 registers: three wavefronts per SIMD and no room
+// for a decode wavefront beside them. Taken when it gives enough workgroups (the caller's rule).
+constexpr int kVsStride32 = kHeadDim + 32;  // 320 bytes: a transposing read's 4 rows x 64 bytes on distinct banks
+constexpr int kVsTile32 = kKeyTile * kVsStride32;
+constexpr int kXchFloats32 = 66 * 64;  // per wavefront at the merge: 64 accumulators, m, l per lane
+constexpr size_t kPrefillTiles32 = (size_t)kKeyGroups * 2 * (kKsTile + kVsTile32) * 2;
+constexpr size_t kPrefillXch32 = (size_t)4 * (kKeyGroups - 1) * kXchFloats32 * 4;
+constexpr size_t kPrefillLds32 = kPrefillTiles32 > kPrefillXch32 ? kPrefillTiles32 : kPrefillXch32;
+
+template <int G, bool OFF32>
+__global__ __launch_bounds__(256 * kKeyGroups) __attribute__((amdgpu_waves_per_eu(3, 3))) void paged_prefill32_kernel(PrefillArgs a) {
+  constexpr int kSub = 4 / G;       // 32-token query sub-tiles per workgroup
+  constexpr int kQTok = 32 * kSub;  // query tokens per workgroup
+  extern __shared__ __attribute__((aligned(16))) uint16_t psm[];
+  const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // key group
+  const int tg = threadIdx.x & 255;                                  // thread within the key group
+  uint16_t* Ks = psm + kg * 2 * (kKsTile + kVsTile32);  // [2][kKeyTile][kKsStride]
+  uint16_t* Vs = Ks + 2 * kKsTile;                       // [2][kKeyTile][kVsStride32]
+
+  const int lin = blockIdx.x + gridDim.x * blockIdx.y;  // KV head fastest, as in the 16-query kernel
+  const int kvh = lin % a.kv_heads, wi = lin / a.kv_heads;
+  const int seq = a.work[2 * wi], tstart = a.work[2 * wi + 1];
+  const int flat = a.seq_info[3 * seq], nnew = a.seq_info[3 * seq + 1], ncached = a.seq_info[3 * seq + 2];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(tg >> 6);  // wavefront within the key group
+  const int st = wave / G, head = kvh * G + wave % G;
+  const int qc = lane & 31, h = lane >> 5;  // this lane's query column; its half of each 16-wide K slice
+
+  const int qi = tstart + st * 32 + qc;
+  const bool qvalid = qi < nnew;
+  const int qi_c = qvalid ? qi : nnew - 1;
+  const int qpos = ncached + qi_c;
+  const int wave_last = ncached + min(tstart + st * 32 + 31, nnew - 1);
+  const int wave_first = ncached + min(tstart + st * 32, nnew - 1);
+
+  bf16x8 qfrag[8];  // Q^T, the B operand: dims 16 ks + 8h .. + 7 of query qc
+  {
+    const uint16_t* qp = a.q + (int64_t)(flat + qi_c) * a.ldq + (int64_t)head * kHeadDim + 8 * h;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qfrag[ks] = *(const bf16x8*)(qp + 16 * ks);
+  }
+
+  const int kend = ncached + min(tstart + kQTok, nnew);
+  const int ntiles = (kend + kKeyTile - 1) / kKeyTile;
+  const int niter = (ntiles + kKeyGroups - 1) / kKeyGroups;
+  const int32_t* btr = a.bt + (int64_t)seq * a.max_blocks;
+  const int64_t tok_stride = (int64_t)a.kv_heads * kHeadDim;
+
+  const int la = tg >> 4, lb = tg & 15;
+  const int64_t thread_off = (int64_t)(2 * (la % 8)) * tok_stride + (int64_t)kvh * kHeadDim + 8 * lb;
+  const uint32_t thread_off_b = (uint32_t)thread_off * 2u;
+  const uint32_t row_b = (uint32_t)tok_stride * 2u, block_b = (uint32_t)kBlock * row_b;
+  u32x4 kr[2], vr[2];
+  int dead_from = 2;
+  auto tile_of = [&](int i) { return kg + kKeyGroups * i; };
+  auto table_entry = [&](int tile) { return btr[min(tile * (kKeyTile / kBlock) + la / 8, a.max_blocks - 1)]; };
+  auto load_tile = [&](int tile, int phys) {
+    phys = ((uint32_t)phys < (uint64_t)a.num_blocks) ? phys : 0;
+    const int key = tile * kKeyTile + 2 * la;
+    const bool blk_ok = tile * (kKeyTile / kBlock) + la / 8 < a.max_blocks;
+    dead_from = !blk_ok || key >= kend ? 0 : (key + 1 >= kend ? 1 : 2);
+    if constexpr (OFF32) {
+      const uint32_t base = __umul24((unsigned)phys, block_b) + thread_off_b;
+      const uint32_t off0 = (blk_ok && key < kend) ? base : 0u;
+      const uint32_t off1 = (blk_ok && key + 1 < kend) ? base + row_b : 0u;
+      kr[0] = *(const u32x4*)((const char*)a.kc + off0);
+      vr[0] = *(const u32x4*)((const char*)a.vc + off0);
+      kr[1] = *(const u32x4*)((const char*)a.kc + off1);
+      vr[1] = *(const u32x4*)((const char*)a.vc + off1);
+    } else {
+      const int64_t base = (int64_t)phys * kBlock * tok_stride + thread_off;
+      const int64_t off0 = (blk_ok && key < kend) ? base : 0;
+      const int64_t off1 = (blk_ok && key + 1 < kend) ? base + tok_stride : 0;
+      kr[0] = *(const u32x4*)(a.kc + off0);
+      vr[0] = *(const u32x4*)(a.vc + off0);
+      kr[1] = *(const u32x4*)(a.kc + off1);
+      vr[1] = *(const u32x4*)(a.vc + off1);
+    }
+  };
+  auto store_tile = [&](int buf, bool last) {
+    uint16_t* K = Ks + buf * kKsTile;
+    uint16_t* V = Vs + buf * kVsTile32;
+    if (last) {
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr)
+        if (rr >= dead_from) vr[rr] = u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int rr = 0; rr < 2; ++rr) {
+      *(u32x4*)&K[(2 * la + rr) * kKsStride + 8 * lb] = kr[rr];
+      *(u32x4*)&V[(2 * la + rr) * kVsStride32 + 8 * lb] = vr[rr];
+    }
+  };
+  auto is_last = [&](int tile) { return (tile + 1) * kKeyTile > kend; };
+  // V^T fragments by the transposing read: in each 16-lane group, lane i names 4 dims of key row
+  // i / 4 of the group's 4 and lane c receives dim c of those 4 rows. Lane (h, d) of the A operand
+  // needs, for the 16-key slice s, keys 16s + 4h + 0..3 and 16s + 8 + 4h + 0..3 of dim d -- the keys
+  // whose probabilities the score accumulators leave in lane (h, query).
+  const int grp = lane >> 4, j = lane & 15;
+  const int vt_off = (4 * (grp >> 1) + (j >> 2)) * kVsStride32 + 16 * (grp & 1) + 4 * (j & 3);
+
+  f32x16 acc[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) acc[dt] = f32x16{};
+  float lsum = 0.f;  // this lane's part of the query's sum (its half of the keys)
+  float m = -INFINITY;
+
+  load_tile(tile_of(0), table_entry(tile_of(0)));
+  const int ph1 = table_entry(tile_of(1));
+  store_tile(0, is_last(tile_of(0)));
+  if (niter > 1) load_tile(tile_of(1), ph1);
+  int ph_next = table_entry(tile_of(2));
+  __syncthreads();
+  for (int i = 0; i < niter; ++i) {
+    const int buf = i & 1;
+    const int key0 = tile_of(i) * kKeyTile;
+    if (key0 <= wave_last) {
+      const uint16_t* K = Ks + buf * kKsTile;
+      const uint16_t* V = Vs + buf * kVsTile32;
+      f32x16 sT = f32x16{};
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) {
+        const bf16x8 kf = *(const bf16x8*)&K[qc * kKsStride + 16 * ks + 8 * h];
+        sT = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qfrag[ks], sT, 0, 0, 0);
+      }
+      // value i of this lane: key 8 (i / 4) + 4h + i % 4 of the tile, query qc
+      if (key0 + kKeyTile - 1 > wave_first) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (key0 + 8 * (e >> 2) + 4 * h + (e & 3) > qpos) sT[e] = -INFINITY;
+      }
+      float bm = fmaxf(sT[0], sT[1]);
+#pragma unroll
+      for (int e = 2; e < 16; e += 2) bm = fmaxf(fmaxf(sT[e], sT[e + 1]), bm);
+      bm = xor32_max(bm) * a.scale_log2;
+      const float mn = fmaxf(m, bm);
+      if (__builtin_amdgcn_ballot_w64(mn > m)) {
+        const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+        lsum *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[dt][e] *= alpha;
+      }
+      m = mn;
+      const float mb = mn == -INFINITY ? 0.0f : mn;
+      bf16x8 pb[2];
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        pb[e >> 3][e & 7] = (__bf16)__builtin_amdgcn_exp2f(__builtin_fmaf(sT[e], a.scale_log2, -mb));
+      // the sum of the rounded probabilities, the ones the product uses
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const u32x4 w = __builtin_bit_cast(u32x4, pb[s]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lsum = dot2_bf16(w[e], 0x3f803f80u, lsum);
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          const uint16_t* vp = V + vt_off + 16 * s * kVsStride32 + dt * 32;
+          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)vp);
+          const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + 8 * kVsStride32));
+          const bf16x8 va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[s], acc[dt], 0, 0, 0);
+        }
+    }
+    if (i + 1 < niter) {
+      store_tile(buf ^ 1, is_last(tile_of(i + 1)));
+      if (i + 2 < niter) load_tile(tile_of(i + 2), ph_next);
+      ph_next = table_entry(tile_of(i + 3));
+    }
+    __syncthreads();
+  }
+  float l = xor32_sum(lsum);
+
+  // Merge of the key groups, as in the 16-query kernel.
+  if (kg > 0) {
+    float* xw = (float*)psm + ((kg - 1) * 4 + wave) * kXchFloats32;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) xw[(dt * 16 + e) * 64 + lane] = acc[dt][e];
+    xw[64 * 64 + lane] = m;
+    xw[65 * 64 + lane] = l;
+  }
+  __syncthreads();
+  if (kg > 0) return;
+  float mm = m;  // finite: group 0 saw key 0
+#pragma unroll
+  for (int o = 1; o < kKeyGroups; ++o) mm = fmaxf(mm, ((float*)psm + ((o - 1) * 4 + wave) * kXchFloats32)[64 * 64 + lane]);
+  const float f0 = __builtin_amdgcn_exp2f(m - mm);
+  float fo[kKeyGroups];
+  l = l * f0;
+#pragma unroll
+  for (int o = 1; o < kKeyGroups; ++o) {
+    const float* xw = (float*)psm + ((o - 1) * 4 + wave) * kXchFloats32;
+    const float mo = xw[64 * 64 + lane];
+    fo[o] = mo == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - mm);
+    l += xw[65 * 64 + lane] * fo[o];
+  }
+  if (!qvalid) return;
+  const float inv = 1.0f / l;
+  uint16_t* orow = a.out + (int64_t)(flat + qi) * a.ldo + (int64_t)head * kHeadDim;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      float o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = acc[dt][4 * b + r] * f0;
+#pragma unroll
+        for (int oo = 1; oo < kKeyGroups; ++oo)
+          v += ((float*)psm + ((oo - 1) * 4 + wave) * kXchFloats32)[(dt * 16 + 4 * b + r) * 64 + lane] * fo[oo];
+        o[r] = v * inv;
+      }
+      *(uint2*)(orow + dt * 32 + 8 * b + 4 * h) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+    }
+}
+
 // The key groups' K / V buffers exceed the 64 KB static LDS limit: dynamic LDS, attribute set once.
 template <int G, bool OFF32>
-static int launch_prefill_kernel(const PrefillArgs& a, dim3 grid, hipStream_t s) {
+static int launch_prefill_kernel(const PrefillArgs& a, dim3 grid, bool wide, hipStream_t s) {
+  if (wide) {
+    const int rc = allow_dynamic_lds((const void*)paged_prefill32_kernel<G, OFF32>, (int)kPrefillLds32, "paged_prefill32_kernel");
+    if (rc != MSA_OK) return rc;
+    hipLaunchKernelGGL((paged_prefill32_kernel<G, OFF32>), grid, dim3(256 * kKeyGroups), kPrefillLds32, s, a);
+    return MSA_OK;
+  }
   const int rc = allow_dynamic_lds((const void*)paged_prefill_kernel<G, OFF32>, (int)kPrefillLds, "paged_prefill_kernel");
   if (rc != MSA_OK) return rc;
   hipLaunchKernelGGL((paged_prefill_kernel<G, OFF32>), grid, dim3(256 * kKeyGroups), kPrefillLds, s, a);
@@ -762,11 +994,11 @@ static int launch_prefill_kernel(const PrefillArgs& a, dim3 grid, hipStream_t s)
 // 32-bit byte offsets when every block of the cache lies within 4 GB of its base (and a block's
 // byte size and index both fit __umul24's 24-bit operands).
 template <int G>
-static int launch_prefill(const PrefillArgs& a, dim3 grid, hipStream_t s) {
+static int launch_prefill(const PrefillArgs& a, dim3 grid, bool wide, hipStream_t s) {
   const int64_t block_bytes = (int64_t)kBlock * a.kv_heads * kHeadDim * 2;
   const bool off32 = a.num_blocks * block_bytes < ((int64_t)1 << 32) && block_bytes < (1 << 24) &&
                      a.num_blocks <= (1 << 24);
-  return off32 ? launch_prefill_kernel<G, true>(a, grid, s) : launch_prefill_kernel<G, false>(a, grid, s);
+  return off32 ? launch_prefill_kernel<G, true>(a, grid, wide, s) : launch_prefill_kernel<G, false>(a, grid, wide, s);
 }
 
 }  // namespace msa
@@ -1010,34 +1242,54 @@ extern "C" int msa_paged_attention_decode_qkv(const uint16_t* qkv, int64_t ldqkv
   return check_launch("msa_paged_attention_decode_qkv (split merge)");
 }
 
-extern "C" int msa_paged_attention_prefill(const uint16_t* q, int64_t ldq, const uint16_t* k_cache,
-                                           const uint16_t* v_cache, int64_t num_slots, int heads, int kv_heads,
-                                           int head_dim, int block_size, const int32_t* block_tables, int max_blocks,
-                                           const int32_t* seq_info, const int32_t* work, int num_work, float scale,
-                                           uint16_t* out, int64_t ldo, msa_stream_t stream) {
-  using namespace msa;
+namespace msa {
+static int prefill_entry(const char* who, bool wide, const uint16_t* q, int64_t ldq, const uint16_t* k_cache,
+                         const uint16_t* v_cache, int64_t num_slots, int heads, int kv_heads, int head_dim,
+                         int block_size, const int32_t* block_tables, int max_blocks, const int32_t* seq_info,
+                         const int32_t* work, int num_work, float scale, uint16_t* out, int64_t ldo, hipStream_t s) {
   if (num_work == 0) return MSA_OK;
   if (!q || !k_cache || !v_cache || !block_tables || !seq_info || !work || !out)
-    return fail(MSA_ERR_INVALID, "msa_paged_attention_prefill: null pointer");
-  if (head_dim != kHeadDim) return fail(MSA_ERR_UNSUPPORTED, "msa_paged_attention_prefill: head_dim must be 128");
-  if (block_size != kBlock) return fail(MSA_ERR_UNSUPPORTED, "msa_paged_attention_prefill: block_size must be 16");
+    return fail(MSA_ERR_INVALID, std::string(who) + ": null pointer");
+  if (head_dim != kHeadDim) return fail(MSA_ERR_UNSUPPORTED, std::string(who) + ": head_dim must be 128");
+  if (block_size != kBlock) return fail(MSA_ERR_UNSUPPORTED, std::string(who) + ": block_size must be 16");
   if (num_work < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || max_blocks <= 0)
-    return fail(MSA_ERR_INVALID, "msa_paged_attention_prefill: bad shape");
+    return fail(MSA_ERR_INVALID, std::string(who) + ": bad shape");
   if (ldq % 8 != 0 || ldo % 4 != 0 || !aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out))
-    return fail(MSA_ERR_INVALID, "msa_paged_attention_prefill: q/out/caches must be 16-byte aligned");
+    return fail(MSA_ERR_INVALID, std::string(who) + ": q/out/caches must be 16-byte aligned");
   PrefillArgs a{};
   a.q = q; a.ldq = ldq; a.kc = k_cache; a.vc = v_cache; a.num_blocks = num_slots / kBlock;
   a.heads = heads; a.kv_heads = kv_heads; a.bt = block_tables; a.max_blocks = max_blocks;
   a.seq_info = seq_info; a.work = work; a.scale_log2 = scale * kLog2e; a.out = out; a.ldo = ldo;
   const dim3 grid(num_work, kv_heads);
-  hipStream_t s = (hipStream_t)stream;
   int rc;
   switch (heads / kv_heads) {
-    case 1: rc = launch_prefill<1>(a, grid, s); break;
-    case 2: rc = launch_prefill<2>(a, grid, s); break;
-    case 4: rc = launch_prefill<4>(a, grid, s); break;
-    default: return fail(MSA_ERR_UNSUPPORTED, "msa_paged_attention_prefill: heads / kv_heads must be 1, 2 or 4");
+    case 1: rc = launch_prefill<1>(a, grid, wide, s); break;
+    case 2: rc = launch_prefill<2>(a, grid, wide, s); break;
+    case 4: rc = launch_prefill<4>(a, grid, wide, s); break;
+    default: return fail(MSA_ERR_UNSUPPORTED, std::string(who) + ": heads / kv_heads must be 1, 2 or 4");
   }
   if (rc != MSA_OK) return rc;
-  return check_launch("msa_paged_attention_prefill");
+  return check_launch(who);
+}
+}  // namespace msa
+
+extern "C" int msa_paged_attention_prefill(const uint16_t* q, int64_t ldq, const uint16_t* k_cache,
+                                           const uint16_t* v_cache, int64_t num_slots, int heads, int kv_heads,
+                                           int head_dim, int block_size, const int32_t* block_tables, int max_blocks,
+                                           const int32_t* seq_info, const int32_t* work, int num_work, float scale,
+                                           uint16_t* out, int64_t ldo, msa_stream_t stream) {
+  return msa::prefill_entry("msa_paged_attention_prefill", false, q, ldq, k_cache, v_cache, num_slots, heads, kv_heads,
+                            head_dim, block_size, block_tables, max_blocks, seq_info, work, num_work, scale, out, ldo,
+                            (hipStream_t)stream);
+}
+
+extern "C" int msa_paged_attention_prefill_wide(const uint16_t* q, int64_t ldq, const uint16_t* k_cache,
+                                                const uint16_t* v_cache, int64_t num_slots, int heads, int kv_heads,
+                                                int head_dim, int block_size, const int32_t* block_tables,
+                                                int max_blocks, const int32_t* seq_info, const int32_t* work,
+                                                int num_work, float scale, uint16_t* out, int64_t ldo,
+                                                msa_stream_t stream) {
+  return msa::prefill_entry("msa_paged_attention_prefill_wide", true, q, ldq, k_cache, v_cache, num_slots, heads,
+                            kv_heads, head_dim, block_size, block_tables, max_blocks, seq_info, work, num_work, scale,
+                            out, ldo, (hipStream_t)stream);
 }

@@ -508,14 +508,16 @@ def paged_attention_prefill(
     scale: float,
     out: Tensor,
     block_size: int = 16,
+    wide: bool = False,
 ) -> Tensor:
+    """``work`` lists query tiles of 64 / (H / KVH) tokens (``wide``: of 128 / (H / KVH))."""
     _on_gpu(q, k_cache, v_cache, block_tables, seq_info, work, out)
     _, heads, d = q.shape
     kvh = k_cache.shape[1]
     _check(seq_info.dtype == torch.int32 and work.dtype == torch.int32 and block_tables.dtype == torch.int32,
            "paged_attention_prefill: int32 metadata")
     _native.call(
-        "msa_paged_attention_prefill", _ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], heads,
+        "msa_paged_attention_prefill_wide" if wide else "msa_paged_attention_prefill", _ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], heads,
         kvh, d, block_size, _ptr(block_tables), block_tables.shape[1], _ptr(seq_info), _ptr(work), work.shape[0],
         float(scale), _ptr(out), out.stride(0), _stream(q),
     )
