@@ -218,8 +218,8 @@ def attend(q: Tensor, k_cache: Tensor, v_cache: Tensor, meta: AttentionMetadata,
         side.wait_event(fork)
     if meta.decode is not None:
         d = meta.decode
-        ptok, parts = kernels.decode_splits(d.num_seqs, kv_heads, d.block_tables.shape[1], heads // kv_heads,
-                                        d.split_context)
+        ptok, parts = kernels.decode_plan(d.num_seqs, kv_heads, d.block_tables.shape[1], heads // kv_heads,
+                                      d.split_context)
         kernels.paged_attention_decode(
             q, k_cache, v_cache, d.block_tables, d.context_lens, d.q_rows, ptok, parts, scale, out, meta.block_size,
             narrow=side is not None, stream=side,
@@ -260,8 +260,8 @@ def attend_decode_qkv(
     d = meta.decode
     kv_heads, dim = k_cache.shape[1], k_cache.shape[2]
     out = torch.empty(qkv.shape[0], heads, dim, dtype=qkv.dtype, device=qkv.device)
-    ptok, parts = kernels.decode_splits(d.num_seqs, kv_heads, d.block_tables.shape[1], heads // kv_heads,
-                                        d.split_context)
+    ptok, parts = kernels.decode_plan(d.num_seqs, kv_heads, d.block_tables.shape[1], heads // kv_heads,
+                                      d.split_context)
     kernels.paged_attention_decode_qkv(
         qkv, heads, q_norm_w, k_norm_w, qk_eps, cos_table, sin_table, meta.slot_mapping, k_cache, v_cache, d.block_tables,
         d.context_lens, d.q_rows, ptok, parts, scale, out, meta.block_size,
