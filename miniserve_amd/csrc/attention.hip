@@ -445,7 +445,8 @@ __global__ __launch_bounds__(64 * W) void paged_decode_kernel(DecodeArgs a) {
 // Merge of the workgroup-level splits of each (sequence, query head): one thread per dim. Every load
 // -- the context, lane p's (maximum, sum) of split p, the splits' partial values -- is issued at once,
 // unconditionally (slots past the sequence's splits hold anything and are not used), so the kernel
-// waits for memory once instead of four times in a row: XXX us against YYY for 3 sequences of 15 splits.
+// waits for memory once instead of four times in a row: 7.8 -> 4.8 us for one sequence of 18
+// splits at 32 heads, 6.7 -> 4.7 for three of 15 (traced durations).
 constexpr int kReduceSplits = 64;  // a wavefront's lanes
 template <int CH>
 __global__ __launch_bounds__(kHeadDim) void paged_decode_reduce_kernel(DecodeArgs a) {
