@@ -16,6 +16,7 @@ from __future__ import annotations
 
 from typing import Any, Sequence
 
+import numpy as np
 import torch
 from torch import Tensor
 
@@ -56,11 +57,31 @@ def exponential_noise(
 ) -> Tensor:
     """Exp(1) noise per row; rows with their own generator (a seeded request) use it
     (sampler.py:43-52)."""
+    noise = _raw_noise(shape, generators, device)
+    return noise.clamp_(min=torch.finfo(noise.dtype).tiny)
+
+
+def _raw_noise(
+    shape: tuple[int, int], generators: Sequence[torch.Generator | None], device: torch.device
+) -> Tensor:
     noise = torch.empty(shape, device=device).exponential_()
     for i, g in enumerate(generators):
         if g is not None:
             noise[i].exponential_(generator=g)
-    return noise.clamp_(min=torch.finfo(noise.dtype).tiny)
+    return noise
+
+
+def _settings(params: Sequence[Any], vocab: int, dev: torch.device) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+    """(temperature, top_k, top_p, greedy) of every row on the device, in one upload."""
+    r = len(params)
+    host = np.zeros((4, r), dtype=np.float32)
+    host[0] = [max(p.temperature, 1e-5) for p in params]
+    host[1].view(np.int32)[:] = [p.top_k if 0 < p.top_k < vocab else vocab for p in params]
+    host[2] = [p.top_p for p in params]
+    host[3].view(np.uint8)[:r] = [1 if p.greedy else 0 for p in params]
+    t = torch.from_numpy(host)
+    d = t.to(dev) if dev.type != "cuda" else t.pin_memory().to(dev, non_blocking=True)
+    return d[0], d[1].view(torch.int32), d[2], d[3].view(torch.uint8)[:r]
 
 
 def sample(logits: Tensor, params: Sequence[Any], generators: Sequence[torch.Generator | None]) -> Tensor:
@@ -68,11 +89,14 @@ def sample(logits: Tensor, params: Sequence[Any], generators: Sequence[torch.Gen
     logits = logits.float().contiguous()
     dev = logits.device
     rows, vocab = logits.shape
-    greedy = to_device([1 if p.greedy else 0 for p in params], dev, torch.uint8)
     if all(p.greedy for p in params):
+        greedy = to_device([1] * len(params), dev, torch.uint8)
         return kernels.sample_ids(logits, None, None, None, greedy, None)
-    temps = to_device([max(p.temperature, 1e-5) for p in params], dev, torch.float32)
-    top_k, top_p = _filters(params, vocab, dev)
-    noise = exponential_noise((rows, vocab), generators, dev)
+    temps, top_k, top_p, greedy = _settings(params, vocab, dev)
+    if not any(0 < p.top_k < vocab or p.top_p < 1.0 for p in params):
+        top_k = top_p = None
+    # The race clamps the noise it reads (to the smallest normal float32, as exponential_noise does), so
+    # the pass over [R, V] that would clamp it in memory is left out.
+    noise = _raw_noise((rows, vocab), generators, dev)
     ranked = all(p.greedy or 0 < p.top_k <= kernels.RANKED_MAX_TOP_K for p in params)
     return kernels.sample_ids(logits, temps, top_k, top_p, greedy, noise, ranked)
