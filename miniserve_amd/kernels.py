@@ -112,32 +112,44 @@ def int8_linear(
     x [..., in] bf16. EPI_SILU_MUL treats the rows as [gate | up] and returns silu(g) * u
     [..., out/2]; EPI_RESIDUAL returns residual + y.
     """
-    _on_gpu(x, qweight, scale)
-    _check(x.dtype == torch.bfloat16, "int8_linear: activations must be bf16")
-    _check(qweight.dtype == torch.int8 and qweight.dim() == 2 and qweight.is_contiguous(), "int8_linear: bad qweight")
-    _check(scale.dtype == torch.bfloat16 and scale.numel() == qweight.shape[0], "int8_linear: bad scale")
-    n, k = qweight.shape
-    _check(x.shape[-1] == k, f"int8_linear: x has {x.shape[-1]} features, weight expects {k}")
-    lead = x.shape[:-1]
-    x2 = x.reshape(-1, k)
-    if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
+    dev = x.get_device()  # -1 for a CPU tensor
+    if dev < 0 or qweight.get_device() != dev or scale.get_device() != dev:
+        _on_gpu(x, qweight, scale)
+    if x.dtype != torch.bfloat16:
+        raise RuntimeError("int8_linear: activations must be bf16")
+    wshape, xshape = qweight.shape, x.shape
+    if qweight.dtype != torch.int8 or len(wshape) != 2 or not qweight.is_contiguous():
+        raise RuntimeError("int8_linear: bad qweight")
+    n, k = wshape
+    if scale.dtype != torch.bfloat16 or scale.numel() != n:
+        raise RuntimeError("int8_linear: bad scale")
+    if xshape[-1] != k:
+        raise RuntimeError(f"int8_linear: x has {xshape[-1]} features, weight expects {k}")
+    x2 = x if len(xshape) == 2 else x.reshape(-1, k)
+    ldx, unit = x2.stride()
+    px = x2.data_ptr()
+    if unit != 1 or ldx % 8 != 0 or px % 16 != 0:
         x2 = x2.contiguous()
+        ldx, px = x2.stride(0), x2.data_ptr()
     m = x2.shape[0]
     cols = n // 2 if epilogue == EPI_SILU_MUL else n
     if out is None:
-        out = torch.empty(*lead, cols, dtype=torch.bfloat16, device=x.device)
-    _check(out.shape[-1] == cols and out.is_contiguous(), "int8_linear: bad out")
-    r2 = None
+        out = torch.empty((*xshape[:-1], cols), dtype=torch.bfloat16, device=x.device)
+    elif out.shape[-1] != cols or not out.is_contiguous():
+        raise RuntimeError("int8_linear: bad out")
+    pr, ldr = None, 0
     if epilogue == EPI_RESIDUAL:
         _check(residual is not None and residual.shape[-1] == n, "int8_linear: residual epilogue needs residual")
         r2 = residual.reshape(-1, n)
         _check(r2.stride(-1) == 1 and r2.dtype == torch.bfloat16, "int8_linear: residual must be row-major bf16")
+        pr, ldr = r2.data_ptr(), r2.stride(0)
+    pw, nw = None, 0
     ws_bytes = _native.query("msa_int8_linear_workspace_size", m, n, k) if m else 0
-    ws = workspaces.get("linear", x.device, ws_bytes)
-    _native.call(
-        "msa_int8_linear", _ptr(x2), m, k, x2.stride(0), _ptr(qweight), _ptr(scale), n, _ptr(out), cols, epilogue,
-        _ptr(r2), r2.stride(0) if r2 is not None else 0, _ptr(ws), ws.numel() if ws is not None else 0, _stream(x),
-    )
+    if ws_bytes:
+        ws = workspaces.get("linear", x.device, ws_bytes)
+        pw, nw = ws.data_ptr(), ws.numel()
+    _native.call("msa_int8_linear", px, m, k, ldx, qweight.data_ptr(), scale.data_ptr(), n, out.data_ptr(), cols,
+                 epilogue, pr, ldr, pw, nw, _raw_stream(dev))
     return out
 
 

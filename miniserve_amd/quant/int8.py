@@ -80,7 +80,10 @@ class Int8Linear(nn.Module):
         """y = x @ bf16(qweight * scale)^T; ``epilogue`` fuses SwiGLU's silu(gate) * up or a
         residual add into the same kernel (used by this package's Qwen3 layers)."""
         if x.dtype == torch.bfloat16:
-            return kernels.int8_linear(x, self.qweight, self.kscale, epilogue, residual)
+            scale = self.scale
+            if scale.dtype != torch.bfloat16:
+                scale = self.kscale
+            return kernels.int8_linear(x, self.qweight, scale, epilogue, residual)
         r = residual.to(torch.bfloat16) if residual is not None else None
         y = kernels.int8_linear(x.to(torch.bfloat16), self.qweight, self.kscale, epilogue, r)
         return y.to(x.dtype)
