@@ -161,11 +161,11 @@ def metadata_from_parts(
     ((name, shape) pairs) back to back -- d_rows, d_ctx, d_tables for the decode sequences, p_info,
     p_tables and p_work<tile> for the prefill ones, each group present only when it has rows."""
     views: dict[str, Tensor] = {}
-    off = 0
-    for name, shape in layout:
-        size = shape[0] * shape[1] if len(shape) == 2 else shape[0]
-        views[name] = flat[off : off + size].view(*shape)
-        off += size
+    off = flat.storage_offset() if flat is not None else 0
+    for name, shape in layout:  # (one view each: a slice and its reshape would be two)
+        two = len(shape) == 2
+        views[name] = flat.as_strided(shape, (shape[1], 1) if two else (1,), off)
+        off += shape[0] * shape[1] if two else shape[0]
     decode = (
         DecodePlan(views["d_rows"], views["d_ctx"], views["d_tables"], split_context) if "d_rows" in views else None
     )
@@ -230,9 +230,13 @@ def attend(q: Tensor, k_cache: Tensor, v_cache: Tensor, meta: AttentionMetadata,
         tile = PREFILL_TILE.get(group)
         if tile is None:
             raise RuntimeError(f"prefill attention supports H/KVH in 1, 2, 4 (got {group})")
-        wide = side is None and prefill_takes_wide(p, tile, kv_heads)  # (beside decode rows: see above)
-        kernels.paged_attention_prefill(q, k_cache, v_cache, p.block_tables, p.seq_info,
-                                        p.work[2 * tile if wide else tile], scale, out, meta.block_size, wide)
+        work = p.work[tile]
+        wide = (side is None and 3 * work.shape[0] * kv_heads >= 4 * PREFILL_WIDE_MIN_WORKGROUPS
+                and prefill_takes_wide(p, tile, kv_heads))  # (beside decode rows: see above)
+        if wide:
+            work = p.work[2 * tile]
+        kernels.paged_attention_prefill(q, k_cache, v_cache, p.block_tables, p.seq_info, work, scale, out,
+                                        meta.block_size, wide)
     if side is not None:
         join.record(side)
         cur.wait_event(join)

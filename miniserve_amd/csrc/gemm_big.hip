@@ -16,7 +16,7 @@
 //    registers are reloaded for the step after next right after they are stored, so every load has a
 //    whole step to arrive (8B-shaped gate_up at 4096 tokens 719 us with the loads at the step's end,
 //    704 with this).
-//    (256 x 128 with the residual epilogue: 4 x 2 of 64 x 64.)
+//    (256 x 128 in one round of workgroups or with the residual epilogue: 4 x 2 of 64 x 64.)
 //  * What bounds it: no unit alone. Per step of a 256 x 128 tile (about 1 us) the MFMAs take 0.47 us
 //    of each SIMD, LDS reads 0.34 (1.75 ns per 1 KB read instruction) and writes 0.28 (5.8 ns each),
 //    dequantization 0.17; wavefronts that leave a barrier together do the same thing at the same time.
@@ -226,11 +226,20 @@ __global__ __launch_bounds__(64 * WM * WN) void int8_gemm256_kernel(BigGemmArgs 
           read_frags(cur ^ 1, 0, af[0], bfr[0]);
         }
         mfmas(af[ks & 1], bfr[ks & 1]);
-        if (ks < 2) {
+        if (NTH == 1024 && ks < 2) {
 #pragma unroll
           for (int p = 2 * ks; p < 2 * ks + 2; ++p) {
             store_part(cur ^ 1, p);
             load_part(min(kt + 2, nk - 1) * kBK, p);
+          }
+        } else if (ks < 2) {
+          // Eight wavefronts: a step's loads together, behind its last store (apart they measured 1%
+          // slower over a short K: 0.6B qkv at 900 tokens 17.2 -> 17.4 us).
+          store_part(cur ^ 1, ks);
+          store_part(cur ^ 1, ks + 2);
+          if (ks == 1) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) load_part(min(kt + 2, nk - 1) * kBK, p);
           }
         }
         __builtin_amdgcn_sched_barrier(0);  // keeps each slice's reads and staging with its MFMAs
@@ -411,8 +420,12 @@ int gemm256_run(int t, const uint16_t* x, int64_t m, int64_t k, int64_t ldx, con
     case 0: return launch_big_epi<256, 2, 4>(a, (int)blocks, epilogue, s);
     case 1: return launch_big_epi<192, 8, 2>(a, (int)blocks, epilogue, s);
     default:
-      // o / down: eight wavefronts (8B o at 2048 tokens 71.8 us, sixteen 74.3; down 209, 213)
+      // One round of workgroups, and the residual epilogue: eight wavefronts (8B o at 1300 tokens 57.9 us,
+      // sixteen 60.1; at 2048 with the residual 71.8, 74.3; 0.6B gate_up-sized rows at 1000 tokens 19.0,
+      // 19.4). More rounds: sixteen (8B qkv at 1300 / 2048 tokens 80 / 97, eight 90 / 104).
       if (epilogue == MSA_EPI_RESIDUAL) return launch_big<128, 4, 2, MSA_EPI_RESIDUAL>(a, (int)blocks, s);
+      if (epilogue == MSA_EPI_NONE && (int64_t)a.n_blocks * a.m_blocks <= 256)
+        return launch_big<128, 4, 2, MSA_EPI_NONE>(a, (int)blocks, s);
       return launch_big_epi<128, 4, 4>(a, (int)blocks, epilogue, s);
   }
 }

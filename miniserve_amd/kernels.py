@@ -373,10 +373,13 @@ def reshape_and_cache(k: Tensor, v: Tensor, k_cache: Tensor, v_cache: Tensor, sl
     """k_cache[slot_mapping] = k; v_cache[slot_mapping] = v (attention/backends.py:159-160)."""
     _on_gpu(k, v, k_cache, v_cache, slot_mapping)
     t, kvh, d = k.shape
-    _check(v.shape == k.shape and k_cache.shape[-2:] == (kvh, d), "reshape_and_cache: shapes")
-    _check(slot_mapping.dtype == torch.int64 and slot_mapping.numel() == t, "reshape_and_cache: slot_mapping")
-    k2 = k if k.stride(-1) == 1 and k.stride(-2) == d else k.contiguous()
-    v2 = v if v.stride(-1) == 1 and v.stride(-2) == d else v.contiguous()
+    if v.shape != k.shape or k_cache.shape[-2:] != (kvh, d):
+        raise RuntimeError("reshape_and_cache: shapes")
+    if slot_mapping.dtype != torch.int64 or slot_mapping.numel() != t:
+        raise RuntimeError("reshape_and_cache: slot_mapping")
+    ks, vs = k.stride(), v.stride()
+    k2 = k if ks[2] == 1 and ks[1] == d else k.contiguous()
+    v2 = v if vs[2] == 1 and vs[1] == d else v.contiguous()
     _native.call("msa_reshape_and_cache", _ptr(k2), k2.stride(0), _ptr(v2), v2.stride(0), t, kvh, d,
                  _ptr(slot_mapping), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], _stream(k))
 
