@@ -451,9 +451,9 @@ int gemm256_qk_norm_run(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, co
 // long K (the 8B-shaped qkv and down at 256 tokens, the 0.6B down at 2048): the fewest splits
 // whose workgroups fill 192-320 of the 256 CUs in one round, each split 16+ whole 64-wide K steps;
 // 0 when none does or the tiling does not apply (under 192 tokens, K not a multiple of 64). With
-// shorter splits the float32 partials (and the merge that reads them) cost more than the eight
-// wavefronts gain: the 8B-shaped o at 256 tokens in eight 512-wide splits 26.6 us against 25.9 on
-// 128 x 128 tiles in four; qkv in four 1024-wide splits 30.6 against 33.7, down 47.9 against 50.2.
+// shorter splits the float32 partials (and the merge that reads them) cost more than the tiling
+// gains: the 8B-shaped o at 256 tokens in eight 512-wide splits 26.6 us against 25.9 on 128 x 128
+// tiles in four; qkv in four 1024-wide splits 29.9 against 33.7, down 44.2 against 50.2.
 int gemm256_split_plan(int64_t m, int64_t n, int64_t k) {
   if (m < 192 || k % kBK != 0) return 0;
   const int64_t tiles = ((n + 127) / 128) * ((m + kBM - 1) / kBM);

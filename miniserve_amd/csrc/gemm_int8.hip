@@ -365,7 +365,7 @@ int gemm256_qk_norm_run(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, co
                         const uint16_t* scale, const QkNormOut& qk, hipStream_t s);
 
 // The qkv projection with its q/k-norm epilogue on 256 x 128 tiles (one head slot each, one
-// workgroup of eight wavefronts per CU) when they fill at least as much of the chip as the 128 x 128
+// workgroup of sixteen wavefronts per CU) when they fill at least as much of the chip as the 128 x 128
 // tiles (two workgroups per CU).
 static bool use_qk_norm256(int64_t m, int64_t k, int64_t ldx, int head_slots) {
   const int64_t n = (int64_t)head_slots * 128;

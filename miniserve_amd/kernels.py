@@ -9,6 +9,7 @@ demand and reserved before any graph capture); kernels never need them zeroed.
 from __future__ import annotations
 
 import contextlib
+import functools
 
 import torch
 from torch import Tensor
@@ -423,6 +424,7 @@ def decode_splits(
     return part, max(1, -(-max_blocks * 16 // part))
 
 
+@functools.lru_cache(maxsize=1024)  # plain arithmetic of five whole numbers, asked once a layer
 def decode_plan(
     num_seqs: int, kv_heads: int, max_blocks: int, group: int, split_context: int | None = None
 ) -> tuple[int, int]:
