@@ -730,7 +730,7 @@ def bench_prefill(args) -> dict:
     log(f"prefill attention (1984-token causal chunk): {asecs * 1e6:.1f} us, {aflops / asecs / 1e12:.1f} TFLOP/s")
     out["roofline"] = roofline("paged_prefill_kernel<2, true> (1984-token causal chunk, 16 q / 8 KV heads)", "mfma",
                                aflops / asecs / 1e12, aflops, asecs)
-    out["roofline_gemm"] = roofline("int8_gemm256_kernel<192, 4, 1> (gate_up + silu*up, M=2048, 256x192 tiles)", "mfma",
+    out["roofline_gemm"] = roofline("int8_gemm256_kernel<192, 8, 2, 1> (gate_up + silu*up, M=2048, 256x192 tiles)", "mfma",
                                     flops / secs / 1e12, flops, secs)
     if not args.no_cpu_baseline:
         from oracle import model as om

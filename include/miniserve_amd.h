@@ -60,10 +60,12 @@ size_t msa_int8_linear_workspace_size(int64_t m, int64_t n, int64_t k);
  * aligned. y has n columns (n/2 for MSA_EPI_SILU_MUL) with row stride ldy; residual (row stride
  * ldr) is read only for MSA_EPI_RESIDUAL and may alias y. When K is split across workgroups the
  * splits meet in the workspace and a second kernel sums them in a fixed order (deterministic).
- * Batches of 128 or more rows with k % 64 == 0 run msa_int8_gemm; smaller ones with k in {1024,
- * 2048, 3072, 4096} run msa_int8_linear_dec (no norm prologue), other smaller ones whose activation
- * tile fits in LDS (k % 64 == 0, k <= 4416) msa_int8_linear_rows; none of these uses the
- * workspace. */
+ * Batches of 128 or more rows with k % 64 == 0 run msa_int8_gemm (its split-K partials in the
+ * workspace). Over weights of n * k >= 12 MiB with k % 64 == 0, batches of 65 or more rows do too, and
+ * smaller ones read the weights once for all their rows (split-K partials in the workspace from 17 rows
+ * and k >= 8192 on). Other batches with k in {1024, 2048, 3072, 4096} run msa_int8_linear_dec (no norm
+ * prologue), and those whose activation tile fits in LDS (k % 64 == 0, k <= 4416) msa_int8_linear_rows;
+ * neither uses the workspace. Without a workspace nothing is split. */
 int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                     const uint16_t* scale, int64_t n, uint16_t* y, int64_t ldy, int epilogue,
                     const uint16_t* residual, int64_t ldr, void* workspace, size_t workspace_bytes,
@@ -73,7 +75,7 @@ int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const 
  * 128-token x 128-row tiles; each int8 weight tile is dequantized once per token tile to the same
  * bf16(q * s) value as the reference, float32 accumulation, then the epilogue of msa_int8_linear
  * (MSA_EPI_RESIDUAL may write y in place over residual). k % 64 == 0; x, qweight 16-byte aligned.
- * msa_int8_linear routes batches of 128 or more rows here. */
+ * msa_int8_linear routes batches of 128 or more rows here (65 or more over large weights). */
 int msa_int8_gemm(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                   const uint16_t* scale, int64_t n, uint16_t* y, int64_t ldy, int epilogue,
                   const uint16_t* residual, int64_t ldr, msa_stream_t stream);
