@@ -297,6 +297,17 @@ int msa_paged_attention_decode_qkv(const uint16_t* qkv, int64_t ldqkv, const uin
                                    const int32_t* context_lens, const int32_t* q_rows, int num_seqs,
                                    int partition_tokens, int max_partitions, float scale, uint16_t* out,
                                    int64_t ldo, void* workspace, size_t workspace_bytes, msa_stream_t stream);
+/* The same with the rotary rows gathered by the caller: sequence i is rotated by row q_rows[i] of the
+ * float32 [rows, 128] cos_rows / sin_rows (one per row of qkv), whatever its context length. */
+int msa_paged_attention_decode_qkv_rows(const uint16_t* qkv, int64_t ldqkv, const uint16_t* q_norm_w,
+                                        const uint16_t* k_norm_w, float qk_eps, const float* cos_rows,
+                                        const float* sin_rows, int64_t rows, const int64_t* slot_mapping,
+                                        uint16_t* k_cache,
+                                        uint16_t* v_cache, int64_t num_slots, int heads, int kv_heads, int head_dim,
+                                        int block_size, const int32_t* block_tables, int max_blocks,
+                                        const int32_t* context_lens, const int32_t* q_rows, int num_seqs,
+                                        int partition_tokens, int max_partitions, float scale, uint16_t* out,
+                                        int64_t ldo, void* workspace, size_t workspace_bytes, msa_stream_t stream);
 
 /* The qkv projection of a prefill-sized batch with the per-head q/k RMSNorm, RoPE and KV-cache
  * write of msa_qk_norm_rope_cache in its epilogue (model/qwen3.py:94-98, then the cache write of

@@ -255,10 +255,13 @@ def attend_decode_qkv(
     v_cache: Tensor,
     meta: AttentionMetadata,
     scale: float,
+    rope_rows: bool = False,
 ) -> Tensor:
     """A pure-decode step's attention from the qkv projection rows (model/qwen3.py:94-99): per-head
-    q/k RMSNorm, RoPE at each sequence's new position, the new keys and values written into the
-    caches at slot_mapping (negative slots are skipped) and attention, in one kernel. qkv [T, (H + 2 KVH) * D] -> [T, H, D]."""
+    q/k RMSNorm, RoPE at each sequence's new position (context length - 1, or with ``rope_rows`` by
+    the row of cos_table / sin_table [T, D] of each row of qkv), the new keys and values written into
+    the caches at slot_mapping (negative slots are skipped) and attention, in one kernel.
+    qkv [T, (H + 2 KVH) * D] -> [T, H, D]."""
     if meta.decode is None or meta.prefill is not None:
         raise RuntimeError("attend_decode_qkv serves batches of decode rows only")
     d = meta.decode
@@ -268,7 +271,7 @@ def attend_decode_qkv(
                                       d.split_context)
     kernels.paged_attention_decode_qkv(
         qkv, heads, q_norm_w, k_norm_w, qk_eps, cos_table, sin_table, meta.slot_mapping, k_cache, v_cache, d.block_tables,
-        d.context_lens, d.q_rows, ptok, parts, scale, out, meta.block_size,
+        d.context_lens, d.q_rows, ptok, parts, scale, out, meta.block_size, rope_rows,
     )
     return out
 

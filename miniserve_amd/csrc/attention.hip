@@ -53,7 +53,7 @@ struct DecodeArgs {
   const uint16_t* qn_w;
   const uint16_t* kn_w;
   float qk_eps;
-  const float* cos_t;  // [max_pos, 128] float32
+  const float* cos_t;  // [max_pos, 128] float32, a row per position (ROWS: per row of q)
   const float* sin_t;
   int64_t max_pos;
   const int64_t* slots;  // [T] cache slot of each row's new token (< 0: not written)
@@ -146,7 +146,8 @@ __device__ __forceinline__ void norm_rope16(uint32_t (&v)[8], const uint4& wlo, 
   for (int e = 0; e < 8; ++e) v[e] = pack_bf16x2(o[2 * (e & 3) + 8 * (e >> 2)], o[2 * (e & 3) + 1 + 8 * (e >> 2)]);
 }
 
-template <int G, int W, bool QKV>
+// ROWS (of QKV): the new token's rotary row is its own of rows the caller gathered, not position ctx - 1's.
+template <int G, int W, bool QKV, bool ROWS = false>
 __global__ __launch_bounds__(64 * W) void paged_decode_kernel(DecodeArgs a) {
   __shared__ float s_acc[W][G][kHeadDim];
   __shared__ float s_ml[W][G][2];
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(64 * W) void paged_decode_kernel(DecodeArgs a) {
     // the G + 1 is done by the row-pair group rp == v (of its round), then every lane gathers
     // all of them from those groups' lanes with the same dims.
     load8(qrow_p + (int64_t)(a.heads + a.kv_heads + kvh) * kHeadDim + 8 * dg, vn);
-    int64_t pos = (int64_t)ctx - 1;
+    int64_t pos = ROWS ? qrow : (int64_t)ctx - 1;
     pos = pos < 0 ? 0 : (pos >= a.max_pos ? a.max_pos - 1 : pos);  // memory safety only
     float c[16], sn[16];
 #pragma unroll
@@ -1072,7 +1073,7 @@ constexpr int kDecodeWideTokens = 1024;
 // sequences at contexts U[128, 2048]: 53.8 against 49.6 us) and keep the plan's order.
 constexpr int kDecodeSerpentineRows = 64;
 
-template <int G, bool QKV = false>
+template <int G, bool QKV = false, bool ROWS = false>
 static void launch_decode(DecodeArgs a, int num_seqs, hipStream_t s, bool narrow = false) {
   a.serpentine = QKV && a.kv_heads == 8 && a.splits == 1 && num_seqs <= kDecodeSerpentineRows;
   // Split-major grid: every sequence's first split, then the second splits, ... The splits past a
@@ -1087,7 +1088,7 @@ static void launch_decode(DecodeArgs a, int num_seqs, hipStream_t s, bool narrow
       return;
     }
   }
-  hipLaunchKernelGGL((paged_decode_kernel<G, kDecodeW, QKV>), grid, dim3(64 * kDecodeW), 0, s, a);
+  hipLaunchKernelGGL((paged_decode_kernel<G, kDecodeW, QKV, ROWS>), grid, dim3(64 * kDecodeW), 0, s, a);
 }
 
 // Shared checks and workspace binding of the two decode entry points.
@@ -1242,44 +1243,72 @@ extern "C" int msa_paged_attention_decode_noalloc(const uint16_t* q, int64_t ldq
                       max_partitions, scale, out, ldo, ws, need > 0 ? kDecodeScratchBytes : 0, (hipStream_t)stream);
 }
 
+namespace msa {
+template <bool ROWS>
+static int decode_qkv_entry(const char* who, const uint16_t* qkv, int64_t ldqkv, const uint16_t* q_norm_w,
+                            const uint16_t* k_norm_w, float qk_eps, const float* cos_table, const float* sin_table,
+                            int64_t max_positions, const int64_t* slot_mapping, uint16_t* k_cache, uint16_t* v_cache,
+                            int64_t num_slots, int heads, int kv_heads, int head_dim, int block_size,
+                            const int32_t* block_tables, int max_blocks, const int32_t* context_lens,
+                            const int32_t* q_rows, int num_seqs, int partition_tokens, int max_partitions, float scale,
+                            uint16_t* out, int64_t ldo, void* workspace, size_t workspace_bytes, hipStream_t s) {
+  if (num_seqs == 0) return MSA_OK;
+  DecodeArgs a;
+  int rc = decode_args(who, qkv, ldqkv, k_cache, v_cache, num_slots, heads, kv_heads, head_dim, block_size, block_tables,
+                       max_blocks, context_lens, q_rows, num_seqs, partition_tokens, max_partitions, scale, out, ldo,
+                       workspace, workspace_bytes, a);
+  if (rc != MSA_OK) return rc;
+  if (!q_norm_w || !k_norm_w || !cos_table || !sin_table || !slot_mapping || max_positions <= 0)
+    return fail(MSA_ERR_INVALID, std::string(who) + ": null norm weight / rotary table / slot_mapping");
+  if (!aligned16(q_norm_w) || !aligned16(k_norm_w) || !aligned16(cos_table) || !aligned16(sin_table))
+    return fail(MSA_ERR_INVALID, std::string(who) + ": norm weights / rotary tables must be 16-byte aligned");
+  if (ldqkv < (int64_t)(heads + 2 * kv_heads) * kHeadDim)
+    return fail(MSA_ERR_INVALID, std::string(who) + ": ldqkv smaller than (heads + 2 kv_heads) * 128");
+  a.qn_w = q_norm_w; a.kn_w = k_norm_w; a.qk_eps = qk_eps; a.cos_t = cos_table; a.sin_t = sin_table;
+  a.max_pos = max_positions;
+  a.slots = slot_mapping;
+  switch (heads / kv_heads) {
+    case 1: launch_decode<1, true, ROWS>(a, num_seqs, s); break;
+    case 2: launch_decode<2, true, ROWS>(a, num_seqs, s); break;
+    case 4: launch_decode<4, true, ROWS>(a, num_seqs, s); break;
+    case 8: launch_decode<8, true, ROWS>(a, num_seqs, s); break;
+    default: return fail(MSA_ERR_UNSUPPORTED, std::string(who) + ": heads / kv_heads must be 1, 2, 4 or 8");
+  }
+  rc = check_launch(who);
+  if (rc != MSA_OK || max_partitions == 1) return rc;
+  launch_reduce(a, num_seqs, s);
+  return check_launch("msa_paged_attention_decode_qkv (split merge)");
+}
+}  // namespace msa
+
 extern "C" int msa_paged_attention_decode_qkv(const uint16_t* qkv, int64_t ldqkv, const uint16_t* q_norm_w,
                                               const uint16_t* k_norm_w, float qk_eps, const float* cos_table,
-                                              const float* sin_table, int64_t max_positions,
-                                              const int64_t* slot_mapping, uint16_t* k_cache,
-                                              uint16_t* v_cache, int64_t num_slots, int heads, int kv_heads,
-                                              int head_dim, int block_size, const int32_t* block_tables,
+                                              const float* sin_table, int64_t max_positions, const int64_t* slot_mapping,
+                                              uint16_t* k_cache, uint16_t* v_cache, int64_t num_slots, int heads,
+                                              int kv_heads, int head_dim, int block_size, const int32_t* block_tables,
                                               int max_blocks, const int32_t* context_lens, const int32_t* q_rows,
                                               int num_seqs, int partition_tokens, int max_partitions, float scale,
                                               uint16_t* out, int64_t ldo, void* workspace, size_t workspace_bytes,
                                               msa_stream_t stream) {
-  using namespace msa;
-  if (num_seqs == 0) return MSA_OK;
-  DecodeArgs a;
-  int rc = decode_args("msa_paged_attention_decode_qkv", qkv, ldqkv, k_cache, v_cache, num_slots, heads, kv_heads,
-                       head_dim, block_size, block_tables, max_blocks, context_lens, q_rows, num_seqs, partition_tokens,
-                       max_partitions, scale, out, ldo, workspace, workspace_bytes, a);
-  if (rc != MSA_OK) return rc;
-  if (!q_norm_w || !k_norm_w || !cos_table || !sin_table || !slot_mapping || max_positions <= 0)
-    return fail(MSA_ERR_INVALID, "msa_paged_attention_decode_qkv: null norm weight / rotary table / slot_mapping");
-  if (!aligned16(q_norm_w) || !aligned16(k_norm_w) || !aligned16(cos_table) || !aligned16(sin_table))
-    return fail(MSA_ERR_INVALID, "msa_paged_attention_decode_qkv: norm weights / rotary tables must be 16-byte aligned");
-  if (ldqkv < (int64_t)(heads + 2 * kv_heads) * kHeadDim)
-    return fail(MSA_ERR_INVALID, "msa_paged_attention_decode_qkv: ldqkv smaller than (heads + 2 kv_heads) * 128");
-  a.qn_w = q_norm_w; a.kn_w = k_norm_w; a.qk_eps = qk_eps; a.cos_t = cos_table; a.sin_t = sin_table;
-  a.max_pos = max_positions;
-  a.slots = slot_mapping;
-  hipStream_t s = (hipStream_t)stream;
-  switch (heads / kv_heads) {
-    case 1: launch_decode<1, true>(a, num_seqs, s); break;
-    case 2: launch_decode<2, true>(a, num_seqs, s); break;
-    case 4: launch_decode<4, true>(a, num_seqs, s); break;
-    case 8: launch_decode<8, true>(a, num_seqs, s); break;
-    default: return fail(MSA_ERR_UNSUPPORTED, "msa_paged_attention_decode_qkv: heads / kv_heads must be 1, 2, 4 or 8");
-  }
-  rc = check_launch("msa_paged_attention_decode_qkv");
-  if (rc != MSA_OK || max_partitions == 1) return rc;
-  launch_reduce(a, num_seqs, s);
-  return check_launch("msa_paged_attention_decode_qkv (split merge)");
+  return msa::decode_qkv_entry<false>("msa_paged_attention_decode_qkv", qkv, ldqkv, q_norm_w, k_norm_w, qk_eps, cos_table,
+                               sin_table, max_positions, slot_mapping, k_cache, v_cache, num_slots, heads, kv_heads, head_dim,
+                               block_size, block_tables, max_blocks, context_lens, q_rows, num_seqs, partition_tokens,
+                               max_partitions, scale, out, ldo, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+extern "C" int msa_paged_attention_decode_qkv_rows(const uint16_t* qkv, int64_t ldqkv, const uint16_t* q_norm_w,
+                                                   const uint16_t* k_norm_w, float qk_eps, const float* cos_rows,
+                                                   const float* sin_rows, int64_t rows, const int64_t* slot_mapping,
+                                                   uint16_t* k_cache, uint16_t* v_cache, int64_t num_slots, int heads,
+                                                   int kv_heads, int head_dim, int block_size, const int32_t* block_tables,
+                                                   int max_blocks, const int32_t* context_lens, const int32_t* q_rows,
+                                                   int num_seqs, int partition_tokens, int max_partitions, float scale,
+                                                   uint16_t* out, int64_t ldo, void* workspace, size_t workspace_bytes,
+                                                   msa_stream_t stream) {
+  return msa::decode_qkv_entry<true>("msa_paged_attention_decode_qkv_rows", qkv, ldqkv, q_norm_w, k_norm_w, qk_eps, cos_rows,
+                               sin_rows, rows, slot_mapping, k_cache, v_cache, num_slots, heads, kv_heads, head_dim,
+                               block_size, block_tables, max_blocks, context_lens, q_rows, num_seqs, partition_tokens,
+                               max_partitions, scale, out, ldo, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 namespace msa {

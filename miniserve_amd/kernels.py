@@ -506,11 +506,13 @@ def paged_attention_decode_qkv(
     scale: float,
     out: Tensor,
     block_size: int = 16,
+    rope_rows: bool = False,
 ) -> Tensor:
     """Decode attention from the qkv projection rows [q | k | v] (msa_paged_attention_decode_qkv):
     per-head q/k RMSNorm and RoPE at position context_len - 1, the new key and value written into
     the caches at slot_mapping (negative slots are skipped), attention over the cached keys plus
-    the new one. out [T, heads, head_dim]."""
+    the new one. out [T, heads, head_dim]. ``rope_rows``: cos_table / sin_table hold one row per row
+    of qkv, gathered by the caller (msa_paged_attention_decode_qkv_rows)."""
     _on_gpu(qkv, q_norm_w, k_norm_w, cos_table, sin_table, slot_mapping, k_cache, v_cache, block_tables, context_lens,
             q_rows, out)
     _check(slot_mapping.dtype == torch.int64 and slot_mapping.numel() == qkv.shape[0], "paged_attention_decode_qkv: slots")
@@ -519,6 +521,7 @@ def paged_attention_decode_qkv(
            and qkv.shape[1] == (heads + 2 * kvh) * d, "paged_attention_decode_qkv: qkv [T, (H + 2 KVH) * D]")
     _check(cos_table.dtype == torch.float32 and cos_table.is_contiguous() and cos_table.shape[-1] == d
            and sin_table.shape == cos_table.shape and sin_table.is_contiguous(), "paged_attention_decode_qkv: rotary")
+    _check(not rope_rows or cos_table.shape[0] == qkv.shape[0], "paged_attention_decode_qkv: a rotary row per qkv row")
     _check(k_cache.is_contiguous() and v_cache.is_contiguous(), "paged_attention_decode_qkv: caches")
     num = context_lens.numel()
     _check(block_tables.dtype == torch.int32 and block_tables.is_contiguous() and block_tables.shape[0] == num,
@@ -528,7 +531,8 @@ def paged_attention_decode_qkv(
     ws = workspaces.get("attention", qkv.device, ws_bytes)
     o2 = out.view(out.shape[0], -1)
     _native.call(
-        "msa_paged_attention_decode_qkv", _ptr(qkv), qkv.stride(0), _ptr(q_norm_w), _ptr(k_norm_w), float(qk_eps),
+        "msa_paged_attention_decode_qkv_rows" if rope_rows else "msa_paged_attention_decode_qkv", _ptr(qkv),
+        qkv.stride(0), _ptr(q_norm_w), _ptr(k_norm_w), float(qk_eps),
         _ptr(cos_table), _ptr(sin_table), cos_table.shape[0], _ptr(slot_mapping), _ptr(k_cache), _ptr(v_cache),
         k_cache.shape[0], heads,
         kvh, d, block_size, _ptr(block_tables), block_tables.shape[1], _ptr(context_lens), _ptr(q_rows), num,

@@ -157,7 +157,9 @@ class Qwen3ForCausalLM(nn.Module):
         kv_caches: list[tuple[Tensor, Tensor]],
         meta: AttentionMetadata,
     ) -> Tensor:
-        """input_ids, positions: [T]. Returns final hidden states [T, hidden] (qwen3.py:140-153)."""
+        """input_ids, positions: [T]. Returns final hidden states [T, hidden] (qwen3.py:140-153).
+        (Decode batches whose linears are all within the token-split kernels take each row's position
+        from its plan, context length - 1.)"""
         if len(kv_caches) != len(self.layers):
             raise ValueError(f"{len(kv_caches)} KV caches for {len(self.layers)} layers")
         if self._token_split_ok(input_ids.numel()):
@@ -165,7 +167,7 @@ class Qwen3ForCausalLM(nn.Module):
             out: Tensor = self.norm(residual)
             return out
         if self._wide_decode_ok(input_ids.numel(), meta):
-            return self._wide_decode_layers(input_ids, kv_caches, meta)
+            return self._wide_decode_layers(input_ids, positions, kv_caches, meta)
         x = self.embed_tokens(input_ids)
         cos, sin = self.rotary(positions)
         if self._all_int8():
@@ -242,16 +244,17 @@ class Qwen3ForCausalLM(nn.Module):
                 (c.hidden_size, c.intermediate_size))
 
     def _wide_decode_layers(
-        self, input_ids: Tensor, kv_caches: list[tuple[Tensor, Tensor]], meta: AttentionMetadata
+        self, input_ids: Tensor, positions: Tensor, kv_caches: list[tuple[Tensor, Tensor]], meta: AttentionMetadata
     ) -> Tensor:
         """The decode layers of a model with large weights; returns the final-normed hidden states.
-        Per-head norms, RoPE and the cache write run inside the decode attention. Up to
+        Per-head norms, RoPE (by ``positions``) and the cache write run inside the decode attention. Up to
         STREAM_MAX_TOKENS tokens the RMSNorms run inside the qkv and gate_up linears (five launches a
         layer); with more, each would be repeated by every workgroup, so they join the o and down
         projections (whose split-K partials that kernel merges)."""
-        cfg, rot = self.cfg, self.rotary
+        cfg = self.cfg
         t = input_ids.numel()
-        x = self.embed_tokens(input_ids.view(-1))  # the residual stream, updated in place
+        x = self.embed_tokens(input_ids)  # the residual stream, updated in place
+        cos, sin = self.rotary(positions)
         inside = t <= kernels.STREAM_MAX_TOKENS and kernels.dec_supported(cfg.hidden_size)
         first = self.layers[0].input_layernorm
         h = x if inside else kernels.rmsnorm(x, first.weight, first.eps)
@@ -265,8 +268,8 @@ class Qwen3ForCausalLM(nn.Module):
             else:
                 rows = kernels.int8_linear(h, qkv.qweight, qkv.kscale)
             a = attend_decode_qkv(
-                rows, attn.num_heads, attn.q_norm.weight, attn.k_norm.weight, attn.q_norm.eps, rot.cos, rot.sin,
-                k_cache, v_cache, meta, attn.scale,
+                rows, attn.num_heads, attn.q_norm.weight, attn.k_norm.weight, attn.q_norm.eps, cos, sin, k_cache,
+                v_cache, meta, attn.scale, rope_rows=True,
             ).view(t, attn.q_size)
             if inside:
                 kernels.int8_linear(a, o.qweight, o.kscale, kernels.EPI_RESIDUAL, residual=x, out=x)

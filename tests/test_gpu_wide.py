@@ -116,3 +116,47 @@ def test_wide_decode_layers_match_the_layer_loop(batch, monkeypatch):
             got.append((model(inp.input_ids, inp.positions, runner.kv_caches, inp.attn), runner.kv_cache.clone()))
     assert rel_l2(got[0][0].cpu(), got[1][0].cpu()) < 2e-2
     assert rel_l2(got[0][1].cpu(), got[1][1].cpu()) < 5e-3
+
+
+# One layer whose linears all reach WIDE_MIN_WEIGHTS and whose down projection is past the token-split kernels.
+LARGE = {**workloads.QWEN3_8B, "num_hidden_layers": 1, "intermediate_size": 4608, "vocab_size": 512,
+         "tie_word_embeddings": True}
+
+
+def _decode_step(cfg, batch, blocks_each=4, seed=5):
+    """(runner, scheduled decode rows of 3 to 60 tokens): a seeded int8 model, each sequence in blocks of
+    its own."""
+    model = workloads.build_model(cfg, workloads.random_weights(cfg, seed, norm_jitter=0.1, device="cuda"), DEV, 256)
+    quantize_int8_(model)
+    runner = ModelRunner(model, DEV, max_model_len=256)
+    ctx = [3 + (37 * i) % (16 * blocks_each - 6) for i in range(batch)]
+    perm = torch.randperm(batch * blocks_each, generator=torch.Generator().manual_seed(1)).tolist()
+    return runner, [ScheduledChunk([(7 * i + j) % cfg["vocab_size"] for j in range(c)], c - 1, 1,
+                                   perm[blocks_each * i : blocks_each * (i + 1)]) for i, c in enumerate(ctx)]
+
+
+def _forward(runner, inp, blocks, positions=None):
+    """(hidden states, KV pool) of one forward over a freshly filled pool."""
+    runner.allocate_kv_cache(blocks)
+    workloads.fill_kv_pool_(runner.kv_cache, 9, on_device=True)
+    with torch.inference_mode():
+        out = runner.model(inp.input_ids, inp.positions if positions is None else positions, runner.kv_caches, inp.attn)
+    return out.cpu(), runner.kv_cache.cpu()
+
+
+@pytest.mark.parametrize("batch", [3, 20])
+def test_wide_decode_layers_rotate_by_the_given_positions(batch, monkeypatch):
+    """forward(input_ids, positions, ...) with positions other than the contexts' last ones (a shifted
+    window, say): the large-weight decode layers rotate by them as the general loop does, and write
+    the keys so rotated (bars as in the test above; another rotation is off by 0.1 and more)."""
+    runner, sched = _decode_step(LARGE, batch)
+    inp = runner.prepare(sched)
+    positions = (inp.positions * 3 + 41) % 256
+    assert not runner.model._token_split_ok(batch) and runner.model._wide_decode_ok(batch, inp.attn)
+    own, got = _forward(runner, inp, 4 * batch), _forward(runner, inp, 4 * batch, positions)
+    monkeypatch.setattr(type(runner.model), "_wide_decode_ok", lambda self, tokens, meta: False)
+    want = _forward(runner, inp, 4 * batch, positions)
+    assert rel_l2(got[0], want[0]) < 2e-2 and rel_l2(got[1], want[1]) < 5e-3
+    slots = inp.attn.slot_mapping.cpu()
+    assert rel_l2(got[1][0, 0, slots], want[1][0, 0, slots]) < 1e-2
+    assert rel_l2(own[1][0, 0, slots], want[1][0, 0, slots]) > 0.1
