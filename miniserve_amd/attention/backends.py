@@ -23,6 +23,10 @@ import numpy as np
 import torch
 from torch import Tensor
 
+try:
+    from miniserve_amd import _hostprep
+except ImportError as e:  # the in-tree CPython extension built with the HIP library
+    raise ImportError("miniserve_amd/_hostprep is not built: run `python -m miniserve_amd.build`") from e
 from miniserve_amd import kernels
 from miniserve_amd.utils import upload_int32
 
@@ -59,6 +63,11 @@ class DecodePlan:
     context_lens: Tensor  # [B] int32
     block_tables: Tensor  # [B, max_blocks] int32, padded with block 0
     split_context: int = 0  # longest context the key splits are planned for (0: the table width)
+    # Whether the slot of each row's new token is its table's slot of its last position and no other position
+    # of any row's context. True: known from the packing that made the slots; False: known from the
+    # tables not to be (the same sequence twice, say); None: slots made elsewhere. Attention that
+    # writes the new keys in the launch that reads the contexts would race where this fails.
+    own_slots: bool | None = None
 
     @property
     def num_seqs(self) -> int:
@@ -139,10 +148,14 @@ def build_attention_metadata(
         parts.append(np.ascontiguousarray(arr, dtype=np.int32).ravel())
         layout.append((name, arr.shape))
 
+    own_slots = None  # the slots are the caller's, on the device
     if dec:
+        ctx, tables = np.array([c.context_len for c in dec], dtype=np.int32), _padded_tables(dec, block_size)
+        if not _hostprep.rows_own_slots(tables, ctx, block_size):
+            own_slots = False
         add("d_rows", np.array([c.flat_start for c in dec], dtype=np.int32))
-        add("d_ctx", np.array([c.context_len for c in dec], dtype=np.int32))
-        add("d_tables", _padded_tables(dec, block_size))
+        add("d_ctx", ctx)
+        add("d_tables", tables)
     if pre:
         add("p_info", np.array([[c.flat_start, c.num_new, c.num_cached] for c in pre], dtype=np.int32))
         add("p_tables", _padded_tables(pre, block_size))
@@ -150,12 +163,12 @@ def build_attention_metadata(
             add(f"p_work{tile}", _prefill_work(pre, tile))
 
     flat = upload_int32(np.concatenate(parts), device) if parts else None
-    return metadata_from_parts(flat, layout, slot_mapping, block_size, split_context)
+    return metadata_from_parts(flat, layout, slot_mapping, block_size, split_context, own_slots)
 
 
 def metadata_from_parts(
     flat: Tensor | None, layout: list[tuple[str, tuple[int, ...]]], slot_mapping: Tensor, block_size: int,
-    split_context: int = 0,
+    split_context: int = 0, own_slots: bool | None = None,
 ) -> AttentionMetadata:
     """The plan from its uploaded int32 parts: ``flat`` holds the parts named in ``layout``
     ((name, shape) pairs) back to back -- d_rows, d_ctx, d_tables for the decode sequences, p_info,
@@ -167,7 +180,9 @@ def metadata_from_parts(
         views[name] = flat.as_strided(shape, (shape[1], 1) if two else (1,), off)
         off += shape[0] * shape[1] if two else shape[0]
     decode = (
-        DecodePlan(views["d_rows"], views["d_ctx"], views["d_tables"], split_context) if "d_rows" in views else None
+        DecodePlan(views["d_rows"], views["d_ctx"], views["d_tables"], split_context, own_slots)
+        if "d_rows" in views
+        else None
     )
     prefill = (
         PrefillPlan(views["p_info"], views["p_tables"], {t: views[f"p_work{t}"] for t in PREFILL_TILE_SIZES})
@@ -260,7 +275,8 @@ def attend_decode_qkv(
     """A pure-decode step's attention from the qkv projection rows (model/qwen3.py:94-99): per-head
     q/k RMSNorm, RoPE at each sequence's new position (context length - 1, or with ``rope_rows`` by
     the row of cos_table / sin_table [T, D] of each row of qkv), the new keys and values written into
-    the caches at slot_mapping (negative slots are skipped) and attention, in one kernel.
+    the caches at slot_mapping (negative slots are skipped) and attention, in one kernel. The rows have
+    to own their slots (DecodePlan.own_slots): keys are written in the launch that reads the contexts.
     qkv [T, (H + 2 KVH) * D] -> [T, H, D]."""
     if meta.decode is None or meta.prefill is not None:
         raise RuntimeError("attend_decode_qkv serves batches of decode rows only")

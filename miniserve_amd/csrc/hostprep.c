@@ -7,7 +7,7 @@
  * ScheduledChunk carries (the reference builds the same per-token ids, positions and slots in
  * runner/model_runner.py:162-205).
  *
- *   pack_decode(chunks, block_size, limit, host_i64, host_meta, host_tables, max_blocks) -> int
+ *   pack_decode(chunks, block_size, limit, host_i64, host_meta, host_tables, max_blocks, own_slots=False) -> int
  *
  * chunks: the step's scheduled sequences (objects with token_ids, num_computed, num_new,
  * block_table, params). Returns -1 when the step is not a pure greedy decode step within `limit`
@@ -20,9 +20,18 @@
  * and returns 1 when some table row changed, 0 when every row already held its prefix (the host
  * table buffer mirrors the device copy, so unchanged rows need no upload). Every check runs before
  * anything is written: a block table shorter than its context raises RuntimeError, an entry out of
- * int32 range OverflowError, and the buffers are left as they were.
+ * int32 range OverflowError, and the buffers are left as they were. With own_slots, a step whose rows do
+ * not own their slots (below) returns -1 as well.
  *
- *   pack_step(chunks, block_size, tiles) -> (data, total, sample_idx, layout)
+ *   rows_own_slots(tables, context_lens, block_size) -> bool
+ *
+ * Decode rows (int32 tables [rows, width], int32 context lengths [rows]) own their slots when the
+ * slot of each row's new token, its table's slot of position context - 1, is no other position of any
+ * row's context, its own included. Attention that writes the new keys in the launch that reads
+ * the contexts needs this; the same sequence twice in a batch, or a block that is still written
+ * to in two tables, breaks it. (Blocks shared as a full prefix do not.)
+ *
+ *   pack_step(chunks, block_size, tiles, own_rows=0) -> (data, total, sample_idx, layout[, own])
  *
  * Any step (prefill chunks, decodes, both): the flat batch of runner/model_runner.py:162-205 and
  * the attention plan of attention/backends.py:80-98 in one host buffer. `data` (a bytearray) holds
@@ -36,6 +45,8 @@
  *   p_work<t> [W, 2] for each tile size t in `tiles`: (prefill sequence, first new token) of every
  *     t-token query tile, the tiles with the most keys (cached + causal) first, ties in sequence
  *     then token order.
+ * With own_rows > 0 a fifth item says whether the rows of a step of up to that many decode sequences and
+ * no others own their slots (None for other steps).
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -77,6 +88,85 @@ static int by_position(const void *a, const void *b) {
   return x->idx < y->idx ? -1 : (x->idx > y->idx);        /* ties in batch order (a stable sort) */
 }
 
+/* Whether n decode rows own their slots (see above); -1 without memory. A small open-addressing
+ * table maps each row's last block to the row, so the check is one lookup per table entry (64 rows
+ * of up to 24 entries: 2.5 us; 256 of up to 250: 65). Negative entries are read as block 0, and not
+ * written. */
+typedef struct {
+  const int32_t *tab;
+  int64_t ctx;
+} DecRow;
+
+static int own_slots(const DecRow *rows, int64_t n, int64_t bs) {
+  uint32_t size = 16, mask;
+  while ((int64_t)size < 4 * n) size <<= 1;
+  mask = size - 1;
+  int32_t *keys = (int32_t *)PyMem_Malloc(2 * (size_t)size * sizeof(int32_t));
+  if (keys == NULL) return -1;
+  int32_t *who = keys + size;
+  memset(keys, 0xff, (size_t)size * sizeof(int32_t)); /* -1: no block */
+  int own = 1;
+  for (int64_t r = 0; r < n && own; ++r) {
+    if (rows[r].ctx < 1) continue;
+    const int32_t blk = rows[r].tab[(rows[r].ctx - 1) / bs];
+    uint32_t h = ((uint32_t)blk * 2654435761u) & mask;
+    while (blk >= 0 && keys[h] >= 0 && keys[h] != blk) h = (h + 1) & mask;
+    if (blk < 0 || keys[h] == blk) own = 0; /* (two rows in one last block: the later one reads the earlier's slot) */
+    keys[h] = blk;
+    who[h] = (int32_t)r;
+  }
+  for (int64_t r = 0; r < n && own; ++r) {
+    const int64_t ctx = rows[r].ctx, need = (ctx + bs - 1) / bs;
+    for (int64_t e = 0; e < need; ++e) {
+      const int32_t blk = rows[r].tab[e] < 0 ? 0 : rows[r].tab[e];
+      uint32_t h = ((uint32_t)blk * 2654435761u) & mask;
+      while (keys[h] >= 0 && keys[h] != blk) h = (h + 1) & mask;
+      if (keys[h] != blk || (who[h] == r && e == need - 1)) continue;
+      if (e * bs + (rows[who[h]].ctx - 1) % bs < ctx) {
+        own = 0;
+        break;
+      }
+    }
+  }
+  PyMem_Free(keys);
+  return own;
+}
+
+static PyObject *rows_own_slots(PyObject *self, PyObject *args) {
+  Py_buffer bt = {0}, bc = {0};
+  long long bs_ll;
+  if (!PyArg_ParseTuple(args, "y*y*L", &bt, &bc, &bs_ll)) return NULL;
+  PyObject *result = NULL;
+  DecRow *rows = NULL;
+  const int64_t bs = bs_ll, n = (int64_t)(bc.len / sizeof(int32_t));
+  const int64_t width = n ? (int64_t)(bt.len / sizeof(int32_t)) / n : 0;
+  const int32_t *ctx = (const int32_t *)bc.buf;
+  if (bs <= 0 || n * width * (int64_t)sizeof(int32_t) != (int64_t)bt.len) {
+    PyErr_SetString(PyExc_ValueError, "rows_own_slots: a positive block_size and tables [rows, width]");
+    goto done;
+  }
+  if ((rows = (DecRow *)PyMem_Malloc((n > 0 ? n : 1) * sizeof(DecRow))) == NULL) {
+    PyErr_NoMemory();
+    goto done;
+  }
+  for (int64_t r = 0; r < n; ++r) {
+    rows[r].tab = (const int32_t *)bt.buf + r * width;
+    rows[r].ctx = ctx[r];
+    if (rows[r].ctx > width * bs) {
+      PyErr_SetString(PyExc_ValueError, "rows_own_slots: a context is longer than its table row");
+      goto done;
+    }
+  }
+  const int own = own_slots(rows, n, bs);
+  if (own < 0) PyErr_NoMemory();
+  else result = PyBool_FromLong(own);
+done:
+  PyMem_Free(rows);
+  PyBuffer_Release(&bt);
+  PyBuffer_Release(&bc);
+  return result;
+}
+
 typedef struct {
   PyObject *toks, *tab;  /* new references */
   int64_t pos;
@@ -87,7 +177,8 @@ static PyObject *pack_decode(PyObject *self, PyObject *args) {
   PyObject *chunks;
   long long bs_ll, limit_ll, mb_ll;
   Py_buffer bi = {0}, bm = {0}, bt = {0};
-  if (!PyArg_ParseTuple(args, "OLLw*w*w*L", &chunks, &bs_ll, &limit_ll, &bi, &bm, &bt, &mb_ll)) return NULL;
+  int check_own = 0;
+  if (!PyArg_ParseTuple(args, "OLLw*w*w*L|p", &chunks, &bs_ll, &limit_ll, &bi, &bm, &bt, &mb_ll, &check_own)) return NULL;
   PyObject *result = NULL;
   PyObject *fast = NULL;
   Seq *seqs = NULL;
@@ -216,6 +307,18 @@ static PyObject *pack_decode(PyObject *self, PyObject *args) {
     }
     slots[i] = (int64_t)vrow[p / bs] * bs + p % bs;
   }
+  if (check_own) {
+    DecRow *dr = (DecRow *)PyMem_Malloc((b > 0 ? b : 1) * sizeof(DecRow));
+    for (Py_ssize_t i = 0; dr != NULL && i < b; ++i) {
+      dr[i].tab = vals + seqs[i].first;
+      dr[i].ctx = seqs[i].pos + 1;
+    }
+    const int own = dr != NULL ? own_slots(dr, b, bs) : -1;
+    PyMem_Free(dr);
+    if (own < 0) PyErr_NoMemory();
+    else if (!own) result = PyLong_FromLong(-1);
+    if (own <= 0) goto fail_ids;
+  }
 
   /* Pass 2: the writes. */
   qsort(rows, (size_t)b, sizeof(Row), by_position);
@@ -312,7 +415,9 @@ static PyObject *shape2(Py_ssize_t a, Py_ssize_t b) { return Py_BuildValue("(nn)
 static PyObject *pack_step(PyObject *self, PyObject *args) {
   PyObject *chunks, *tiles_obj;
   long long bs_ll;
-  if (!PyArg_ParseTuple(args, "OLO", &chunks, &bs_ll, &tiles_obj)) return NULL;
+  long long own_rows = 0;
+  int own = -1; /* not looked at */
+  if (!PyArg_ParseTuple(args, "OLO|L", &chunks, &bs_ll, &tiles_obj, &own_rows)) return NULL;
   const int64_t bs = bs_ll;
   PyObject *result = NULL, *fast = NULL, *tiles = NULL, *data = NULL, *sample = NULL, *layout = NULL;
   Chunk *c = NULL;
@@ -475,6 +580,19 @@ static PyObject *pack_step(PyObject *self, PyObject *args) {
     w32 += ndec;
     if (fill_tables(c, dec, ndec, bs, nb_d, w32) < 0) goto done;
     ADD_PART("d_tables", shape2(ndec, (Py_ssize_t)nb_d));
+    if (npre == 0 && ndec <= own_rows) {
+      DecRow *dr = (DecRow *)PyMem_Malloc((size_t)ndec * sizeof(DecRow));
+      for (Py_ssize_t r = 0; dr != NULL && r < ndec; ++r) {
+        dr[r].tab = w32 + r * nb_d;
+        dr[r].ctx = c[dec[r]].start + 1;
+      }
+      own = dr != NULL ? own_slots(dr, ndec, bs) : -1;
+      PyMem_Free(dr);
+      if (own < 0) {
+        PyErr_NoMemory();
+        goto done;
+      }
+    }
     w32 += ndec * nb_d;
   }
   if (npre) {
@@ -527,7 +645,9 @@ static PyObject *pack_step(PyObject *self, PyObject *args) {
     }
   }
 #undef ADD_PART
-  result = Py_BuildValue("(OLOO)", data, (long long)total, sample, layout);
+  result = own_rows > 0 ? Py_BuildValue("(OLOOO)", data, (long long)total, sample, layout,
+                                        own < 0 ? Py_None : own ? Py_True : Py_False)
+                        : Py_BuildValue("(OLOO)", data, (long long)total, sample, layout);
 done:
   if (c != NULL) {
     for (Py_ssize_t i = 0; i < made; ++i) {
@@ -551,8 +671,10 @@ done:
 
 static PyMethodDef methods[] = {
     {"pack_decode", pack_decode, METH_VARARGS,
-     "pack_decode(chunks, block_size, limit, host_i64, host_meta, host_tables, max_blocks) -> -1 | 0 | 1"},
-    {"pack_step", pack_step, METH_VARARGS, "pack_step(chunks, block_size, tiles) -> (data, total, sample_idx, layout)"},
+     "pack_decode(chunks, block_size, limit, host_i64, host_meta, host_tables, max_blocks, own_slots=False) -> -1 | 0 | 1"},
+    {"pack_step", pack_step, METH_VARARGS,
+     "pack_step(chunks, block_size, tiles, own_rows=0) -> (data, total, sample_idx, layout[, own])"},
+    {"rows_own_slots", rows_own_slots, METH_VARARGS, "rows_own_slots(tables, context_lens, block_size) -> bool"},
     {NULL, NULL, 0, NULL}};
 
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hostprep", "Decode-step input packing.", -1, methods};

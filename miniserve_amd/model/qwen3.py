@@ -223,12 +223,16 @@ class Qwen3ForCausalLM(nn.Module):
 
     def _wide_decode_ok(self, tokens: int, meta: AttentionMetadata) -> bool:
         """Whether a batch takes the large-weight decode layers: decode rows only, up to
-        DEC_MAX_TOKENS, head_dim 128, int8 linears of WIDE_MIN_WEIGHTS and more (the 8B shape)."""
+        DEC_MAX_TOKENS, head_dim 128, int8 linears of WIDE_MIN_WEIGHTS and more (the 8B shape). Their
+        attention writes the new keys itself and attends to them from registers, which is the layer
+        loop's write followed by its read only when every token is a plan row known to own its slot."""
         cfg = self.cfg
         return (
             meta.prefill is None
             and meta.decode is not None
+            and meta.decode.own_slots is True
             and 0 < tokens <= kernels.DEC_MAX_TOKENS
+            and meta.decode.num_seqs == tokens
             and cfg.head_dim == 128
             and cfg.num_attention_heads // cfg.num_key_value_heads in (1, 2, 4, 8)
             and self.decode_linears
@@ -312,7 +316,8 @@ class Qwen3ForCausalLM(nn.Module):
           KV write)] -> paged attention -> [int8 o + residual add]
           -> [post-attention RMSNorm + int8 gate_up + silu * up] -> [int8 down + residual add]
         A pure-decode batch of up to DEC_MAX_TOKENS tokens runs the qkv projection as a plain decode
-        linear and the per-head norms, RoPE and KV write inside the decode attention kernel."""
+        linear and the per-head norms, RoPE and KV write inside the decode attention kernel (rows known
+        not to own their slots are written by the qkv kernel, before any row attends)."""
         cfg = self.cfg
         t = residual.shape[0]
         rot = self.rotary
@@ -329,8 +334,8 @@ class Qwen3ForCausalLM(nn.Module):
             return kernels.int8_linear_rows
 
         fused_decode = (
-            meta.prefill is None and meta.decode is not None and t <= kernels.DEC_MAX_TOKENS
-            and kernels.dec_supported(cfg.hidden_size) and self.decode_linears
+            meta.prefill is None and meta.decode is not None and meta.decode.own_slots is not False
+            and t <= kernels.DEC_MAX_TOKENS and kernels.dec_supported(cfg.hidden_size) and self.decode_linears
         )
         first = input_ids is not None
         src = self.embed_tokens.weight if first else residual

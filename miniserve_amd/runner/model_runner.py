@@ -33,6 +33,7 @@ try:
 except ImportError as e:  # the in-tree CPython extension built with the HIP library
     raise ImportError("miniserve_amd/_hostprep is not built: run `python -m miniserve_amd.build`") from e
 from miniserve_amd.attention.backends import PREFILL_TILE_SIZES, AttentionMetadata, DecodePlan, metadata_from_parts
+from miniserve_amd.kernels import DEC_MAX_TOKENS
 from miniserve_amd.model.qwen3 import Qwen3ForCausalLM
 from miniserve_amd.runner.sampler import sample
 
@@ -92,7 +93,8 @@ class CapturedDecode:
         self.rows = torch.arange(b, dtype=torch.int64, device=dev)  # every row is sampled
         self.ids, self.pos, self.slots = self.dev[:b], self.dev[b : 2 * b], self.dev[2 * b : 3 * b]
         meta32 = self.dev[3 * b :].view(torch.int32)  # q_rows | context_lens, as int32
-        plan = DecodePlan(meta32[:b], meta32[b : 2 * b], self.dev_tab.view(b, max_blocks), runner.split_context)
+        # own_slots: run() checks every step (larger batches write the keys before they attend)
+        plan = DecodePlan(meta32[:b], meta32[b : 2 * b], self.dev_tab.view(b, max_blocks), runner.split_context, True)
         self.meta = AttentionMetadata(self.slots, runner.block_size, plan, None)
         self.host_meta = self.host[3 * b :].view(torch.int32).numpy()
         self.host_i64 = self.host[: 3 * b].numpy()
@@ -120,7 +122,7 @@ class CapturedDecode:
 
     def run(self, scheduled: list[ScheduledChunk], block_size: int, limit: int) -> list[int] | None:
         """Replay the step for ``scheduled``; None (nothing replayed) when it is not a pure greedy
-        decode step within ``limit`` positions.
+        decode step within ``limit`` positions (whose rows own their slots, where that is needed).
 
         ``_hostprep.pack_decode`` writes the ids, positions and slots, the attention plan rows
         (longest context first, each keeping its own q row, as build_attention_metadata orders
@@ -128,7 +130,7 @@ class CapturedDecode:
         buffers. The host table buffer mirrors the device copy, so it is uploaded only when some
         row changed (most decode steps append no block)."""
         rc = _hostprep.pack_decode(scheduled, block_size, limit, self.host_i64, self.host_meta, self.host_tables,
-                                   self.max_blocks)
+                                   self.max_blocks, self.batch <= DEC_MAX_TOKENS)
         if rc < 0:
             return None
         if rc:
@@ -187,7 +189,7 @@ class ModelRunner:
         plan (build_attention_metadata's parts) in one host buffer, uploaded with one pinned,
         non-blocking copy."""
         bs = self.block_size
-        data, total, sample_idx, layout = _hostprep.pack_step(scheduled, bs, PREFILL_TILE_SIZES)
+        data, total, sample_idx, layout, own = _hostprep.pack_step(scheduled, bs, PREFILL_TILE_SIZES, DEC_MAX_TOKENS)
         n64 = 3 * total + len(sample_idx)
         host = torch.frombuffer(data, dtype=torch.uint8) if len(data) else torch.empty(0, dtype=torch.uint8)
         dev = host.to(self.device) if self.device.type != "cuda" else host.pin_memory().to(self.device, non_blocking=True)
@@ -196,7 +198,7 @@ class ModelRunner:
         return StepInputs(
             input_ids=i64[:total],
             positions=i64[total : 2 * total],
-            attn=metadata_from_parts(dev[8 * n64 :].view(torch.int32), layout, slot_mapping, bs, self.split_context),
+            attn=metadata_from_parts(dev[8 * n64 :].view(torch.int32), layout, slot_mapping, bs, self.split_context, own),
             logits_rows=i64[3 * total :],
             sample_idx=sample_idx,
         )

@@ -13,8 +13,11 @@ from __future__ import annotations
 import pytest
 import torch
 from helpers import rel_l2
+from model_helpers import copy_pool_to_oracle, oracle_step, pair
 
 from miniserve_amd import _native, kernels, workloads
+from miniserve_amd.attention import backends
+from miniserve_amd.model import qwen3
 from miniserve_amd.quant.int8 import quantize_int8_
 from miniserve_amd.runner.model_runner import ModelRunner, ScheduledChunk
 from oracle import int8 as oi
@@ -160,3 +163,55 @@ def test_wide_decode_layers_rotate_by_the_given_positions(batch, monkeypatch):
     slots = inp.attn.slot_mapping.cpu()
     assert rel_l2(got[1][0, 0, slots], want[1][0, 0, slots]) < 1e-2
     assert rel_l2(own[1][0, 0, slots], want[1][0, 0, slots]) > 0.1
+
+
+def _twice(sched):
+    """The batch with its first sequence in it again, one token further (a verify as single rows, say)."""
+    s = sched[0]
+    return [*sched, ScheduledChunk([*s.token_ids, 11], s.num_computed + 1, 1, s.block_table)]
+
+
+def test_large_model_rows_that_share_a_slot_take_the_layer_loop(monkeypatch):
+    """Two rows of one sequence: the later attends to the key that the earlier writes in this step. The
+    large-weight decode layers write keys inside the attention launch, so such a batch, and one whose
+    slots the plan's builder did not make, takes the general loop, which writes every key first."""
+    runner, sched = _decode_step(LARGE, 3)
+    inp = runner.prepare(sched)
+    seqs = [backends.SeqChunk(i, 1, s.num_computed, s.block_table) for i, s in enumerate(sched)]
+    assert runner.model._wide_decode_ok(3, inp.attn)
+    assert not runner.model._wide_decode_ok(3, backends.build_attention_metadata(seqs, inp.attn.slot_mapping, 16))
+    inp = runner.prepare(_twice(sched))
+    assert not runner.model._wide_decode_ok(4, inp.attn)
+    got = _forward(runner, inp, 12)
+    monkeypatch.setattr(type(runner.model), "_wide_decode_ok", lambda self, tokens, meta: False)
+    want = _forward(runner, inp, 12)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_small_model_rows_that_share_a_slot(monkeypatch):
+    """The same batch on the token-split pipeline, eager and where a graph of its size is captured: keys
+    written before any row attends, logits as the oracle's (which writes, then attends)."""
+    cfg = {**workloads.QWEN3_0_6B, "num_hidden_layers": 1, "vocab_size": 1024}
+    runner, ocfg, ow, okv, tables = pair(cfg, seed=3, max_positions=256, num_blocks=16)
+    workloads.fill_kv_pool_(runner.kv_cache, seed=4)
+    copy_pool_to_oracle(runner, okv)
+    runner.use_graphs, runner.max_model_len = True, 256
+    ctx = [20, 33, 7]
+    sched = [ScheduledChunk([(5 * i + j) % 1024 for j in range(c)], c - 1, 1, list(range(4 * i, 4 * i + 4)))
+             for i, c in enumerate(ctx)]
+    before = runner.kv_cache.clone()
+    runner.execute([*sched, ScheduledChunk([1, 2], 1, 1, [13])])  # captures a graph of four rows
+    assert list(runner.graphs) == [4]
+    runner.kv_cache.copy_(before)
+    shared = _twice(sched)
+    logits, ids = oracle_step(ocfg, ow, okv, tables, shared)
+
+    def never(*args, **kwargs):
+        raise AssertionError("attention that writes the keys itself")
+
+    monkeypatch.setattr(qwen3, "attend_decode_qkv", never)
+    assert rel_l2(runner.forward_logits(runner.prepare(shared)).cpu(), logits) < 1e-2
+    runner.kv_cache.copy_(before)
+    assert [r[0] for r in runner.execute(shared)] == runner.forward_greedy(runner.prepare(shared)).tolist()
+    slots = runner.prepare(shared).attn.slot_mapping.cpu()
+    assert rel_l2(runner.kv_caches[0][0].cpu()[slots], okv[0][0][slots]) < 1e-2

@@ -238,3 +238,61 @@ def test_pack_step_errors():
     chunks[2].block_table[0] = -(2**31) - 1
     with pytest.raises(OverflowError):
         _hostprep.pack_step(chunks, BS, PREFILL_TILE_SIZES)
+
+
+# ---- which decode rows own the slot they write -----------------------------------------------------
+
+
+def owns_by_positions(chunks):
+    """Every (block, offset) of every row's context against every row's new slot."""
+    new = [(c.block_table[c.num_computed // BS], c.num_computed % BS) for c in chunks]
+    for r, c in enumerate(chunks):
+        for p in range(c.num_computed + 1):
+            at = (c.block_table[p // BS], p % BS)
+            if any(at == s and not (r == w and p == c.num_computed) for w, s in enumerate(new)):
+                return False
+    return True
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_rows_own_slots_matches_every_position(seed):
+    """Random batches over few blocks (own, shared as full prefixes, shared where they are written, the
+    same block twice in one table), through every entry point that answers."""
+    rng = random.Random(500 + seed)
+    chunks = batch(rng, rng.choice([1, 2, 7, 40]), hi=rng.choice([20, 200]))
+    fresh = iter(range(1, 10_000))  # (block 0 is what an unused table entry holds)
+    for c in chunks:
+        c.block_table = [next(fresh) for _ in c.block_table]
+    for _ in range(rng.choice([0, 1, 3])):
+        a, b = rng.choice(chunks), rng.choice(chunks)
+        n = rng.randint(0, min(len(a.block_table), len(b.block_table)))
+        if rng.random() < 0.5:
+            a.block_table[:n] = b.block_table[:n]
+        else:
+            a.block_table[rng.randrange(len(a.block_table))] = rng.choice(b.block_table)
+    want = owns_by_positions(chunks)
+    assert _hostprep.pack_step(chunks, BS, PREFILL_TILE_SIZES, 128)[4] is want
+    assert _hostprep.pack_step(chunks, BS, PREFILL_TILE_SIZES, len(chunks) - 1 or -1)[4:] in ((), (None,))
+    hi, hm, ht = buffers(len(chunks))
+    rc = _hostprep.pack_decode(chunks, BS, LIMIT, hi, hm, ht, MB, True)
+    assert (rc == 1) is want and (want or not (hi.any() or hm.any() or ht.any()))
+    assert runner_cpu().prepare(chunks).attn.decode.own_slots is want
+    seqs = [SeqChunk(i, 1, c.num_computed, c.block_table) for i, c in enumerate(chunks)]
+    meta = build_attention_metadata(seqs, torch.zeros(len(chunks), dtype=torch.int64), BS)
+    assert meta.decode.own_slots is (None if want else False)  # the slots themselves are not known there
+
+
+def test_rows_own_slots_cases():
+    def owns(tables, ctx):
+        return _hostprep.rows_own_slots(np.array(tables, np.int32), np.array(ctx, np.int32), BS)
+
+    assert owns([[3, 4], [3, 5]], [20, 32])  # a full prefix block shared
+    assert not owns([[3, 4], [3, 4]], [20, 21])  # the same sequence at two lengths
+    assert not owns([[3, 4], [3, 4]], [20, 20])
+    assert not owns([[3, 4], [4, 9]], [20, 17])  # row 0 writes into row 1's first block
+    assert owns([[3, 4], [9, 4]], [16, 32])  # row 0 does not reach its second entry
+    assert not owns([[3, 3]], [17])  # its own first block
+    assert not owns([[-1, 0]], [5])  # read as block 0, never written
+    assert owns([], []) and owns([[0, 0]], [0])
+    with pytest.raises(ValueError):
+        owns([[3, 4]], [33])
