@@ -127,12 +127,14 @@ def int8_linear(
     if xshape[-1] != k:
         raise RuntimeError(f"int8_linear: x has {xshape[-1]} features, weight expects {k}")
     x2 = x if len(xshape) == 2 else x.reshape(-1, k)
+    m = x2.shape[0]
     ldx, unit = x2.stride()
+    if m == 1:
+        ldx = k  # one row has no pitch, whatever stride its view carries
     px = x2.data_ptr()
     if unit != 1 or ldx % 8 != 0 or px % 16 != 0:
         x2 = x2.contiguous()
-        ldx, px = x2.stride(0), x2.data_ptr()
-    m = x2.shape[0]
+        ldx, px = k, x2.data_ptr()
     cols = n // 2 if epilogue == EPI_SILU_MUL else n
     if out is None:
         out = torch.empty((*xshape[:-1], cols), dtype=torch.bfloat16, device=x.device)

@@ -16,6 +16,7 @@ from helpers import rel_l2
 
 from miniserve_amd import kernels
 from miniserve_amd.attention import backends as hb
+from miniserve_amd.quant.int8 import Int8Linear
 from oracle import attention as oa
 from oracle import int8 as oi
 from oracle import layers as ol
@@ -90,6 +91,27 @@ def test_linear_parity(m, n, k):
     assert torch.equal(y, y2)
     assert rel_l2(y.cpu(), ref) < 1e-2
     assert rel_l2(y.cpu(), exact) < 4e-3
+
+
+@pytest.mark.parametrize("n,k", [(3072, 1024), (512, 2000), (4096, 4096)])
+def test_linear_one_row_of_any_pitch(n, k):
+    """A single activation row is taken whatever stride its view carries for the row dimension: a slice
+    of a wider buffer, a transposed column, an expanded row, a leading dimension of one; also every
+    second element of a row (copied)."""
+    _, q, s = _linear_inputs(1, n, k, seed=n)
+    row = _bf16((k,), seed=k).to(DEV)
+    lin = Int8Linear(torch.ones(n, k, dtype=torch.bfloat16, device=DEV))
+    lin.qweight.copy_(q)
+    lin.scale.copy_(s)
+    want = lin(row.view(1, k))
+    wide = torch.zeros(8, k + 4, dtype=torch.bfloat16, device=DEV)
+    wide[:, :k] = row
+    spread = torch.zeros(1, 2 * k, dtype=torch.bfloat16, device=DEV)
+    spread[:, ::2] = row
+    for x in (wide[:1, :k], row.view(k, 1).t(), row.expand(4, k)[:1], spread[:, ::2]):
+        assert x.shape == (1, k) and x.stride() != (k, 1)
+        assert torch.equal(lin(x), want)
+    assert torch.equal(lin(wide[:1, None, :k]), want.view(1, 1, n)) and torch.equal(lin(row), want[0])
 
 
 @pytest.mark.parametrize("m", [1, 16, 64, 77])
