@@ -299,14 +299,15 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(SampArgs a) {
 // while most of the chip idled; the passes below take 65 us (17 + 10 + 22 + 17) for the same batch.
 //  1. sample_chunk_kernel writes the chunk's largest logit and, with top-p, a histogram of the
 //     softmax mass over kMassBins value bins (z falling in steps of 1 / kBinsPerUnit from the chunk
-//     maximum; masses exp(z - chunk max) in 2^-40 fixed point: exact sums, so atomics in any order).
+//     maximum; masses exp(z - chunk max) in 2^-44 fixed point: exact sums, so atomics in any order).
 //  2. sample_cut_kernel, one workgroup per row: the row maximum, the chunks' histograms scaled to it
 //     and added in chunk order, and the bin where the mass at or below it passes (1 - p) of the total.
 //  3. sample_race_kernel, one workgroup per (row, chunk): every entry above that bin is kept and
 //     runs the race exp(z - m) / noise here; the entries inside the bin go to the chunk's
 //     candidate list. Logits and noise are each read once, coalesced.
 //  4. sample_finish_kernel decides the bin's entries one value at a time (mass at or below each in
-//     2^-40 fixed point, as the top-k rows) and joins their race with the chunks' winners.
+//     2^-44 fixed point of the largest entry, as finely as the whole-row path's of the total) and joins
+//     their race with the chunks' winners.
 // A row with a NaN, without a finite maximum, with a temperature that is not positive, or with more
 // entries in the cut's bin than the lists hold takes the whole-row path.
 constexpr int kCandThreads = 256;
@@ -317,7 +318,7 @@ constexpr int kCandCap = 512;       // candidates kept per chunk
 constexpr int kFinishCap = 8192;    // candidates the finishing workgroup takes per row (LDS)
 constexpr int kMaxChunks = 64;      // chunks per row the finishing workgroup gathers (vocab <= 655,360)
 constexpr int kMassBins = 512;      // value bins of a chunk's mass histogram (the slot's list space holds it)
-constexpr float kBinsPerUnit = 16.f;  // bins per unit of z: 32 units below the maximum, past which e^-32 < 2^-40
+constexpr float kBinsPerUnit = 16.f;  // bins per unit of z: 32 units below the maximum, past which e^-32 < 2^-44
 constexpr int kWideCap = kCandCap - 8;  // in-bin entries kept per chunk (the row's WideRow ends chunk 0's slot)
 constexpr int kCntWhole = -1, kCntOver = -2, kCntWide = -3;  // cand_cnt of a slot without a list
 constexpr int kFinishThreads = 256;  // (a row that falls back runs the whole-row path on these too)
@@ -379,12 +380,14 @@ __device__ __forceinline__ bool no_top_k(const SampArgs& a, int64_t k) { return 
 // The bin of z below the one of the row maximum (fbm = wide_bin of it); monotonic in z, so a bin holds
 // every entry of its values.
 __device__ __forceinline__ float wide_bin(float z) { return floorf(z * kBinsPerUnit); }
-// e in [0, 1] in 2^-40 fixed point, truncated: two exact 20-bit steps, cheaper than a 64-bit conversion.
+// e in [0, 1] in 2^-44 fixed point, truncated: two exact steps of 20 and 24 bits, cheaper than a 64-bit
+// conversion. The kMaxChunks * kCandChunk entries of the largest row that uses the sums fit 64 bits.
 __device__ __forceinline__ unsigned long long mass_fixed(float e) {
   const float a = e * 0x1p20f;
   const uint32_t hi = (uint32_t)a;
-  return ((unsigned long long)hi << 20) + (uint32_t)((a - (float)hi) * 0x1p20f);
+  return ((unsigned long long)hi << 24) + (uint32_t)((a - (float)hi) * 0x1p24f);
 }
+static_assert((int64_t)kMaxChunks * kCandChunk < 1 << 20, "a row's masses sum to less than 2^64");
 
 // Inclusive suffix sum over the lanes of a wavefront: lane l gets the sum over lanes >= l.
 __device__ __forceinline__ uint32_t wave_suffix_sum(uint32_t v) {
@@ -653,7 +656,7 @@ __device__ __forceinline__ void wide_chunk(const CandArgs& c, int64_t row, int64
   for (int i = 0; i < kCandPerThread; ++i) {
     const float z = vals[i] / t;
     const unsigned long long w = mass_fixed(expf(z - mc));
-    if (i * kCandThreads + tid < n && w != 0ull)  // (z more than 32 below the maximum has no mass: no bin past the last)
+    if (i * kCandThreads + tid < n && w != 0ull)  // (z 32 or more below the maximum has no mass: no bin past the last)
       atomicAdd(&s_hist[(int)fminf(fbc - wide_bin(z), (float)(kMassBins - 1))], w);
   }
   __syncthreads();

@@ -256,3 +256,40 @@ def test_rows_without_top_k_over_chunks(vocab):
     none = kernels.sample_ids(ld, td, None, None, gd, nd).cpu()  # no filters at all: temperature alone
     full = kernels.sample_ids(ld, td, kd, torch.ones_like(pd), gd, nd).cpu()
     assert torch.equal(none, full)
+
+
+@pytest.mark.parametrize("vocab", [10240, 70000, 151936])
+def test_top_p_cut_of_rows_without_top_k(vocab):
+    """Where top-p alone cuts, to the resolution the masses are held in: values whose mass at or below
+    them, known in float64, lies just above 1 - p (kept) or just below it (dropped), each shown by a noise
+    that lets one of its entries win if it is kept. Logits are multiples of 2^-10, so every z - m is exact
+    in float32; what is left, relative to the row's total, is B = (entries at or below + 512 bins) masses
+    truncated to 2^-44 of the largest entry and 2^-22 of the mass itself (exp within an ulp on both
+    sides). Probes lie between B and 3 B off, the kept ones where masses in steps of 2^-40, which lose
+    2^-41 an entry on average, would drop them."""
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    probes, expect = [], []
+    for top in (12.0, 13.0, 14.0):
+        z = torch.round(torch.randn(vocab, generator=g, device=DEV) * 1024) / 1024
+        z[vocab // 3] = top
+        values, group, count = z.unique(return_inverse=True, return_counts=True)
+        mass = torch.exp(values.double() - top) * count
+        share, below = mass.cumsum(0) / mass.sum(), count.cumsum(0)
+        bound = (below + 512) * 2.0**-44 / mass.sum() + 2.0**-22 * share
+        for step in (-1, 0, 1):  # the float32 p nearest to 1 - share and its neighbours
+            p = (1 - share).float() + step * 2.0**-24
+            off = share - (1 - p.double())
+            usable = (share > 1e-5) & (share < 0.02) & (off.abs() > bound) & (off.abs() < 3 * bound)
+            usable &= (off < 0) | (off < 0.7 * below * 2.0**-41 / mass.sum())
+            for j in usable.nonzero().flatten().tolist()[::3][:30]:
+                probes.append((z, int((group == j).nonzero()[0]), float(p[j])))
+                expect.append(bool(off[j] > 0))
+    assert sum(expect) >= 3 and len(expect) - sum(expect) >= 3
+    want = torch.tensor(expect)
+    logits = torch.stack([z for z, _, _ in probes])
+    at = torch.tensor([i for _, i, _ in probes], device=DEV)
+    p = torch.tensor([q for _, _, q in probes], device=DEV)
+    noise = torch.ones_like(logits).scatter_(1, at[:, None], 1e-30)
+    greedy = torch.zeros(len(probes), dtype=torch.uint8, device=DEV)
+    got = kernels.sample_ids(logits, torch.ones_like(p), None, p, greedy, noise) == at
+    assert torch.equal(got.cpu(), want), (got.cpu() != want).nonzero().flatten().tolist()
