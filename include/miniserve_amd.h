@@ -368,18 +368,18 @@ int msa_sampling_probs(const float* logits, int64_t ld, int64_t rows, int64_t vo
  * greedy[r] != 0, else the exponential race argmax_i probs[r][i] / max(noise[r][i], FLT_MIN) with
  * probs as msa_sampling_probs and noise ~ Exp(1) [rows, ldn] drawn by the caller (the reference
  * draws it with torch's exponential_, per-row generators for seeded requests). With a workspace
- * of msa_sample_workspace_size(rows, vocab) bytes (rows <= 65535; 8-byte aligned, else rows without
- * top-k are not spread), greedy rows, rows with 0 < top_k <= 256 and rows without top-k are spread
- * over vocabulary chunks (four launches); a NULL workspace takes one workgroup per row. */
+ * of msa_sample_workspace_size(rows, vocab) bytes (rows <= 65535), greedy rows and rows with
+ * 0 < top_k <= 256 are spread over vocabulary chunks (two launches); a NULL workspace takes one
+ * workgroup per row. */
 size_t msa_sample_workspace_size(int64_t rows, int64_t vocab);
 int msa_sample(const float* logits, int64_t ld, int64_t rows, int64_t vocab, const float* temperature,
                const int32_t* top_k, const float* top_p, const uint8_t* greedy, const float* noise, int64_t ldn,
                int64_t* out_ids, void* workspace, size_t workspace_bytes, msa_stream_t stream);
-/* msa_sample for a batch whose rows are all greedy or have 0 < top_k <= 256: the two launches that
- * serve rows without top-k are left out (such a row, if there is one, takes one workgroup). */
-int msa_sample_ranked(const float* logits, int64_t ld, int64_t rows, int64_t vocab, const float* temperature,
-                      const int32_t* top_k, const float* top_p, const uint8_t* greedy, const float* noise, int64_t ldn,
-                      int64_t* out_ids, void* workspace, size_t workspace_bytes, msa_stream_t stream);
+/* msa_sample for a batch with rows without top-k: they are spread over the chunks too (four launches;
+ * the workspace 8-byte aligned, else one workgroup each as above). */
+int msa_sample_wide(const float* logits, int64_t ld, int64_t rows, int64_t vocab, const float* temperature,
+                    const int32_t* top_k, const float* top_p, const uint8_t* greedy, const float* noise, int64_t ldn,
+                    int64_t* out_ids, void* workspace, size_t workspace_bytes, msa_stream_t stream);
 
 /* ---- speculative-decoding verification (spec/rejection.py) ----------------------------------- */
 

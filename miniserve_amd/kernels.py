@@ -787,7 +787,10 @@ def lm_head_logits(
 
 # ---- sampling ---------------------------------------------------------------------------------------
 
-RANKED_MAX_TOP_K = 256  # largest top_k the sampling kernel takes from vocabulary chunks' candidates
+# Rows without top-k or top-p take the two launches that spread them over vocabulary chunks from this
+# vocabulary on (64 rows of 3072: 17.9 us by a workgroup each, 19.1 spread; of 4096: 20.5, 19.5); with
+# top-p from the smallest (1 x 64: 34, 24).
+SAMPLE_WIDE_MIN_VOCAB = 4096
 
 
 def _rows_f32(logits: Tensor, name: str) -> Tensor:
@@ -834,20 +837,22 @@ def sample_ids(
     top_p: Tensor | None,
     greedy: Tensor | None,
     noise: Tensor | None,
-    ranked: bool = False,
+    wide: bool | None = None,
 ) -> Tensor:
     """Token id per row: the greedy argmax where ``greedy``, else argmax(probs / noise) with the
     probabilities of ``sampling_probs`` (runner/sampler.py:55-69). ``noise`` [R, V] float32 ~ Exp(1);
-    it may be None only when every row is greedy. ``ranked``: the caller knows that every row is
-    greedy or has 0 < top_k <= 256, so the launches that serve other rows are left out (the same ids
-    either way: such a row would still be served, by one workgroup)."""
+    it may be None only when every row is greedy. ``wide``: spread the rows without top-k over vocabulary
+    chunks, in two more launches; else such a row is served by one workgroup (the same ids either way).
+    By default only where ``top_k`` is None, so that no row has it."""
     _on_gpu(logits)
     _rows_f32(logits, "sample_ids")
     r, v = logits.shape
     if noise is None:
         _check(greedy is not None, "sample_ids: noise is required for sampled rows")
         noise = logits  # never read: every row is greedy
-        ranked = True
+        wide = False
+    if wide is None:
+        wide = top_k is None and (top_p is not None or v >= SAMPLE_WIDE_MIN_VOCAB)
     _check(noise.dtype == torch.float32 and noise.dim() == 2 and noise.shape == (r, v) and noise.stride(-1) == 1,
            "sample_ids: noise [R, V] float32")
     out = torch.empty(r, dtype=torch.int64, device=logits.device)
@@ -855,13 +860,13 @@ def sample_ids(
     tk = _opt_param(top_k, torch.int32, r, "top_k")
     tp = _opt_param(top_p, torch.float32, r, "top_p")
     gr = _opt_param(greedy, torch.uint8, r, "greedy")
-    # Greedy rows, rows with 0 < top_k <= 256 and rows without top-k run over vocabulary chunks (the
-    # workspace holds each chunk's candidates); the others take a workgroup per row in the same call.
+    # Greedy rows, rows with 0 < top_k <= 256 and, with wide, rows without top-k run over vocabulary chunks
+    # (the workspace holds each chunk's candidates); the others take a workgroup per row in the same call.
     ws_bytes = _native.query("msa_sample_workspace_size", r, v)
     ws = workspaces.get("sample", logits.device, ws_bytes)
-    _native.call("msa_sample_ranked" if ranked else "msa_sample", _ptr(logits), logits.stride(0), r, v, _ptr(temps), _ptr(tk), _ptr(tp), _ptr(gr),
-                 _ptr(noise), noise.stride(0), _ptr(out), _ptr(ws), ws.numel() if ws is not None else 0,
-                 _stream(logits))
+    _native.call("msa_sample_wide" if wide else "msa_sample", _ptr(logits), logits.stride(0), r, v, _ptr(temps),
+                 _ptr(tk), _ptr(tp), _ptr(gr), _ptr(noise), noise.stride(0), _ptr(out), _ptr(ws),
+                 ws.numel() if ws is not None else 0, _stream(logits))
     return out
 
 

@@ -98,5 +98,6 @@ def sample(logits: Tensor, params: Sequence[Any], generators: Sequence[torch.Gen
     # The race clamps the noise it reads (to the smallest normal float32, as exponential_noise does), so
     # the pass over [R, V] that would clamp it in memory is left out.
     noise = _raw_noise((rows, vocab), generators, dev)
-    ranked = all(p.greedy or 0 < p.top_k <= kernels.RANKED_MAX_TOP_K for p in params)
-    return kernels.sample_ids(logits, temps, top_k, top_p, greedy, noise, ranked)
+    wide = any(not (p.greedy or 0 < p.top_k < vocab) and (p.top_p < 1.0 or vocab >= kernels.SAMPLE_WIDE_MIN_VOCAB)
+               for p in params)
+    return kernels.sample_ids(logits, temps, top_k, top_p, greedy, noise, wide)

@@ -241,8 +241,8 @@ def test_rows_without_top_k_over_chunks(vocab):
     noise = torch.empty(rows, vocab).exponential_(generator=g)
     ld = torch.empty(rows, vocab + 3, device=DEV)[:, :vocab].copy_(logits)
     td, kd, pd, gd, nd = (t.to(DEV) for t in (temps, k, p, greedy, noise))
-    got = kernels.sample_ids(ld, td, kd, pd, gd, nd).cpu()
-    assert torch.equal(got, kernels.sample_ids(ld, td, kd, pd, gd, nd).cpu())  # deterministic
+    got = kernels.sample_ids(ld, td, kd, pd, gd, nd, wide=True).cpu()
+    assert torch.equal(got, kernels.sample_ids(ld, td, kd, pd, gd, nd, wide=True).cpu())  # deterministic
     assert torch.equal(got[greedy.bool()], logits.argmax(-1)[greedy.bool()])
     whole = _whole_row_ids(ld, td, kd, pd, gd, nd).cpu()
     scores = (kernels.sampling_probs(ld, td, kd, pd) / nd.clamp_min(1.17549435e-38)).double()
@@ -253,8 +253,8 @@ def test_rows_without_top_k_over_chunks(vocab):
             assert int(got[r]) == int(whole[r]), r
             checked += 1
     assert checked >= rows - 2
-    none = kernels.sample_ids(ld, td, None, None, gd, nd).cpu()  # no filters at all: temperature alone
-    full = kernels.sample_ids(ld, td, kd, torch.ones_like(pd), gd, nd).cpu()
+    none = kernels.sample_ids(ld, td, None, None, gd, nd, wide=True).cpu()  # no filters at all: temperature alone
+    full = kernels.sample_ids(ld, td, kd, torch.ones_like(pd), gd, nd, wide=True).cpu()
     assert torch.equal(none, full)
 
 
@@ -293,3 +293,45 @@ def test_top_p_cut_of_rows_without_top_k(vocab):
     greedy = torch.zeros(len(probes), dtype=torch.uint8, device=DEV)
     got = kernels.sample_ids(logits, torch.ones_like(p), None, p, greedy, noise) == at
     assert torch.equal(got.cpu(), want), (got.cpu() != want).nonzero().flatten().tolist()
+
+
+def test_calls_spread_only_rows_without_top_k(monkeypatch):
+    """The two launches that spread rows without top-k are made where some row gains by them: not for calls
+    with a top_k tensor that do not ask for them, nor for batches whose rows are greedy, have top-k
+    (of any size), or are short and without top-p; one workgroup a row gives the same ids."""
+    from miniserve_amd import _native
+
+    calls, real = [], _native.call
+
+    def record(name, *args):
+        calls.append(name)
+        real(name, *args)
+
+    monkeypatch.setattr(_native, "call", record)
+    small, large = kernels.SAMPLE_WIDE_MIN_VOCAB - 1, kernels.SAMPLE_WIDE_MIN_VOCAB
+    for params, vocab, want in [
+        ([Params(top_k=20, top_p=0.9), Params(temperature=0.0)], large, "msa_sample"),
+        ([Params(top_k=1000), Params(top_k=5)], large, "msa_sample"),
+        ([Params()], small, "msa_sample"),
+        ([Params(), Params(top_k=20, top_p=0.9)], small, "msa_sample"),
+        ([Params(top_k=5), Params()], large, "msa_sample_wide"),
+        ([Params(top_p=0.9), Params(top_k=5)], small, "msa_sample_wide"),
+        ([Params(temperature=0.0)] * 2, large, "msa_sample"),
+    ]:
+        x = torch.randn(len(params), vocab, generator=torch.Generator().manual_seed(vocab)).to(DEV)
+        torch.cuda.manual_seed(3)
+        ids = hs.sample(x, params, [None] * len(params))
+        assert calls.pop() == want, (params, vocab)
+        if all(p.greedy for p in params):
+            continue
+        torch.cuda.manual_seed(3)
+        noise = torch.empty_like(x).exponential_()
+        temps = torch.tensor([max(p.temperature, 1e-5) for p in params], device=DEV)
+        k = torch.tensor([p.top_k for p in params], dtype=torch.int32, device=DEV)
+        p = torch.tensor([p.top_p for p in params], device=DEV)
+        greedy = torch.tensor([p.greedy for p in params], dtype=torch.uint8, device=DEV)
+        assert torch.equal(ids, kernels.sample_ids(x, temps, k, p, greedy, noise)) and calls.pop() == "msa_sample"
+    noise = torch.empty_like(x).exponential_()
+    kernels.sample_ids(x[:, :small], temps, None, p, greedy, noise[:, :small])
+    kernels.sample_ids(x[:, :small], temps, None, None, greedy, noise[:, :small])
+    assert calls[-2:] == ["msa_sample_wide", "msa_sample"]
