@@ -52,6 +52,13 @@ enum {
 /* Bytes of float32 workspace msa_int8_linear may use for this shape (0 if none). With less (or no)
  * workspace the call still succeeds, without splitting K across workgroups. */
 size_t msa_int8_linear_workspace_size(int64_t m, int64_t n, int64_t k);
+/* The same of msa_int8_linear_add_rmsnorm and of msa_int8_gemm_qk_norm_rope_cache (n its qkv columns). */
+size_t msa_int8_linear_add_rmsnorm_workspace_size(int64_t m, int64_t n, int64_t k);
+size_t msa_int8_gemm_qk_norm_rope_cache_workspace_size(int64_t m, int64_t n, int64_t k);
+/* What a caller should hold for any of the three before it captures them in a graph (0 if nothing):
+ * without it a call leaves much of the chip idle. The sizes above can be larger, or nonzero where this is 0;
+ * a call without the difference is served by another kernel at a smaller loss. */
+size_t msa_int8_linear_min_workspace_size(int64_t m, int64_t n, int64_t k);
 
 /* Int8Linear.forward (quant/int8.py:35-37) without materializing W: y[m, :] from x [m, k] (row
  * stride ldx), qweight [n, k] int8, scale [n] bf16. Each weight is dequantized in registers to
@@ -61,11 +68,11 @@ size_t msa_int8_linear_workspace_size(int64_t m, int64_t n, int64_t k);
  * ldr) is read only for MSA_EPI_RESIDUAL and may alias y. When K is split across workgroups the
  * splits meet in the workspace and a second kernel sums them in a fixed order (deterministic).
  * Batches of 128 or more rows with k % 64 == 0 run msa_int8_gemm (its split-K partials in the
- * workspace). Over weights of n * k >= 12 MiB with k % 64 == 0, batches of 65 or more rows do too, and
- * smaller ones read the weights once for all their rows (split-K partials in the workspace from 17 rows
- * and k >= 8192 on). Other batches with k in {1024, 2048, 3072, 4096} run msa_int8_linear_dec (no norm
- * prologue), and those whose activation tile fits in LDS (k % 64 == 0, k <= 4416) msa_int8_linear_rows;
- * neither uses the workspace. Without a workspace nothing is split. */
+ * workspace). Smaller ones with k in {1024, 2048, 3072, 4096} run msa_int8_linear_dec (no norm prologue),
+ * those whose activation tile fits in LDS (k % 64 == 0, k <= 4544) msa_int8_linear_rows (neither uses
+ * the workspace), the rest a split-K kernel. Over weights of n * k >= 12 MiB with k % 64 == 0,
+ * 65 or more rows run the GEMM and fewer a kernel that reads the weights once for all of them
+ * (with a long k in splits whose partials meet in the workspace). Without a workspace nothing is split. */
 int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                     const uint16_t* scale, int64_t n, uint16_t* y, int64_t ldy, int epilogue,
                     const uint16_t* residual, int64_t ldr, void* workspace, size_t workspace_bytes,

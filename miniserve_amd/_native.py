@@ -16,7 +16,7 @@ from pathlib import Path
 import torch  # noqa: F401  -- must be imported before the HIP library is loaded
 
 LIB_PATH = Path(__file__).resolve().parent / "libminiserve_amd.so"
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 # name -> (restype, argtypes); mirrors include/miniserve_amd.h.
 SIGNATURES: dict[str, tuple[object, list[object]]] = {
@@ -24,6 +24,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "msa_abi_version": (c_int, []),
     "msa_int8_quantize": (c_int, [c_void_p, c_int, c_int64, c_int64, c_void_p, c_void_p, c_void_p]),
     "msa_int8_linear_workspace_size": (c_size_t, [c_int64, c_int64, c_int64]),
+    "msa_int8_linear_add_rmsnorm_workspace_size": (c_size_t, [c_int64, c_int64, c_int64]),
+    "msa_int8_gemm_qk_norm_rope_cache_workspace_size": (c_size_t, [c_int64, c_int64, c_int64]),
+    "msa_int8_linear_min_workspace_size": (c_size_t, [c_int64, c_int64, c_int64]),
     "msa_int8_linear": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int,

@@ -337,6 +337,22 @@ size_t gemm_workspace_size(int64_t m, int64_t n, int64_t k, int epilogue) {
   return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
 }
 
+// The middle shapes' two splits pay without a fused consumer of the partials only over a long K (0.6B o /
+// down at 4096 tokens, K = 2048 / 3072: 33 / 47 us unsplit, 42 / 53 split; with the norm 39 / 51 and 38 / 48).
+static int plain_splits(int64_t m, int64_t n, int64_t k, int epilogue) {
+  const int splits = gemm_splits(m, n, k, epilogue);
+  return splits > 1 && splits128(m, n, k, epilogue) <= 1 && k < 4096 ? 1 : splits;
+}
+
+size_t gemm_plain_workspace_size(int64_t m, int64_t n, int64_t k) {
+  return plain_splits(m, n, k, MSA_EPI_NONE) > 1 ? gemm_workspace_size(m, n, k, MSA_EPI_NONE) : 0;
+}
+
+// The part without which the GEMM leaves much of the chip idle: the 128-token tiles' splits.
+size_t gemm_min_workspace_size(int64_t m, int64_t n, int64_t k) {
+  return splits128(m, n, k, MSA_EPI_NONE) > 1 ? gemm_workspace_size(m, n, k, MSA_EPI_NONE) : 0;
+}
+
 // The 256-token tilings (gemm_big.hip): the best-filling one and its tile count, and the GEMM on it.
 int gemm256_pick(int64_t m, int64_t n, int64_t k, int epilogue, int64_t* tiles);
 int gemm256_run(int t, const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
@@ -386,10 +402,7 @@ int gemm_run(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t*
   a.m = (int)m; a.n = (int)n; a.k = (int)k;
   a.n_blocks = (int)(epilogue == MSA_EPI_SILU_MUL ? (n / 2 + 63) / 64 : (n + kGBN - 1) / kGBN);
   a.m_blocks = (int)((m + kGBM - 1) / kGBM);
-  int splits = gemm_splits(m, n, k, epilogue);
-  // The middle shapes' two splits pay without the fused norm only over a long K (0.6B o / down at 4096
-  // tokens, K = 2048 / 3072: 33 / 47 us unsplit, 42 / 53 split; with the norm 39 / 51 and 38 / 48).
-  if (splits > 1 && splits128(m, n, k, epilogue) <= 1 && k < 4096) splits = 1;
+  int splits = plain_splits(m, n, k, epilogue);
   const bool unsplit_plan = splits == 1 || splits128(m, n, k, epilogue) <= 1;  // planned unsplit but for splits_mid
   if (splits > 1 && (!workspace || workspace_bytes < gemm_workspace_size(m, n, k, epilogue) || !aligned16(workspace)))
     splits = 1;
@@ -690,6 +703,10 @@ int launch_lm_gemm(const uint16_t* hidden, int64_t ld_hidden, int64_t hidden_row
 }  // namespace msa
 
 using namespace msa;
+
+extern "C" size_t msa_int8_gemm_qk_norm_rope_cache_workspace_size(int64_t m, int64_t n, int64_t k) {
+  return m > 0 && n > 0 && k > 0 && k % kGBK == 0 ? gemm_workspace_size(m, n, k, MSA_EPI_NONE) : 0;
+}
 
 extern "C" int msa_int8_gemm_qk_norm_rope_cache(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
                                                const int8_t* qweight, const uint16_t* scale, int heads, int kv_heads,

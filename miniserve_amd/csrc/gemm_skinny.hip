@@ -269,16 +269,6 @@ static int check_linear_args(const char* fn, const uint16_t* x, int64_t m, int64
 
 }  // namespace msa
 
-// Batches of at least this many rows (with k % 64 == 0) go to the LDS-tiled GEMM (gemm_int8.hip);
-// over weights of 12 MB and more already those past the wide decode kernel's 64: the kernels for
-// small batches read such weights once per 16 tokens (8B-shaped gate_up at 96 tokens 132 us, the GEMM
-// at 128 tokens 62).
-constexpr int64_t kGemmMinRows = 128;
-constexpr int64_t kGemmMinRowsWide = 65, kWideWeights = (int64_t)12 << 20;
-static bool takes_gemm(int64_t m, int64_t n, int64_t k) {
-  return k % 64 == 0 && (m >= kGemmMinRows || (m >= kGemmMinRowsWide && n * k >= kWideWeights));
-}
-
 namespace msa {
 bool dec_linear_supported(int64_t k);  // gemv_dec.hip: K in {1024, 2048, 3072, 4096}
 bool dec_stream_eligible(int64_t m, int64_t k, int64_t n, int epilogue);  // gemv_stream.hip
@@ -300,16 +290,6 @@ extern "C" int msa_int8_linear_rows(const uint16_t* x, int64_t ldx, int64_t m, i
                                     uint16_t* y, int64_t ldy, const uint16_t* residual, int64_t ldr,
                                     msa_stream_t stream);
 
-// msa_int8_linear_add_rmsnorm on the wide decode kernel: up to this many tokens the product and the
-// residual in one launch, then the norm; above, split-K partials that the norm's kernel merges (8B
-// down at 32 tokens: 22 us against 16.5, o 9.1 against 7.7; at 16 tokens 16.4 / 7.2 against 14.6 /
-// 6.7 with a dearer merge).
-constexpr int64_t kWideDirectTokens = 16;
-// msa_int8_linear there: a long K (8B down: 24.0 us at 32 tokens in one launch, 34.2 at 64) is split
-// too, merged by an epilogue kernel (about 20 and 23); o (K = 4096) takes 10.0 / 13.5 us in one
-// launch, which a merge would not beat.
-constexpr int64_t kWideSplitMinK = 8192;
-
 // Smaller batches whose activation tile fits in LDS go to the token-split kernels (gemv_rows.hip).
 static bool rows_fits(int64_t k) { return k % 64 == 0 && 16 * (k + 8) * 2 + 16 * 1024 <= 160 * 1024; }
 
@@ -317,7 +297,10 @@ namespace msa {  // the LDS-tiled GEMM route (gemm_int8.hip)
 int gemm_run(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight, const uint16_t* scale,
              int64_t n, uint16_t* y, int64_t ldy, int epilogue, const uint16_t* residual, int64_t ldr, void* workspace,
              size_t workspace_bytes, hipStream_t s);
+int gemm_splits(int64_t m, int64_t n, int64_t k, int epilogue);
 size_t gemm_workspace_size(int64_t m, int64_t n, int64_t k, int epilogue);
+size_t gemm_plain_workspace_size(int64_t m, int64_t n, int64_t k);
+size_t gemm_min_workspace_size(int64_t m, int64_t n, int64_t k);
 int gemm_run_partials(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                       const uint16_t* scale, int64_t n, float* part, size_t part_bytes, hipStream_t s);
 void launch_splitk_add_rmsnorm(const float* part, int k_split, int64_t rows, int dim, const uint16_t* resid_in,
@@ -326,21 +309,84 @@ void launch_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* w, uint16_t*
                     float eps, hipStream_t s);
 }  // namespace msa
 
-extern "C" size_t msa_int8_linear_workspace_size(int64_t m, int64_t n, int64_t k) {
-  if (m <= 0 || n <= 0 || k <= 0) return 0;
-  if (takes_gemm(m, n, k)) return msa::gemm_workspace_size(m, n, k, MSA_EPI_NONE);  // split-K partials
-  if (msa::dec_wide_eligible(m, k, n, k, n, n)) {  // the partials of msa_int8_linear_add_rmsnorm
-    const int sp = msa::dec_wide_splits(m, n, k);
-    return sp > 1 && m > kWideDirectTokens ? (size_t)sp * m * n * sizeof(float) : 0;
-  }
-  if (msa::dec_linear_supported(k) || rows_fits(k)) return 0;
+// ---- routes ---------------------------------------------------------------------------------------
+
+// What a linear runs on: the LDS-tiled GEMM from 128 rows on; smaller batches the decode kernel (K it
+// supports), the rows kernel (activation tile within LDS) or the skinny split-K kernel. Over weights of
+// 12 MB and more two kernels that read the weights once for all rows take their place: the wide decode kernel
+// up to 64 rows, the GEMM from 65 (the kernels for small batches read such weights once per 16 tokens:
+// 8B-shaped gate_up at 96 tokens 132 us, the GEMM at 128 tokens 62).
+constexpr int64_t kGemmMinRows = 128, kWideMaxRows = 64, kWideWeights = (int64_t)12 << 20;
+constexpr int kEpiNorm = -1;  // msa_int8_linear_add_rmsnorm: the residual, then the norm
+enum class Route { kGemm, kWide, kDec, kRows, kSkinny };
+
+static Route small_route(int64_t k) {
+  return msa::dec_linear_supported(k) ? Route::kDec : rows_fits(k) ? Route::kRows : Route::kSkinny;
+}
+
+static Route route(int64_t m, int64_t n, int64_t k, int64_t ldx, int64_t ldy, int64_t ldr, int epilogue) {
+  if (k % 64 == 0 && m >= kGemmMinRows) return Route::kGemm;
+  if (k % 64 != 0 || n * k < kWideWeights) return small_route(k);
+  if (m > kWideMaxRows) return Route::kGemm;
+  // (the streaming kernel, up to 16 rows at K of 2048 / 4096, is inside the decode entry point)
+  if (epilogue != kEpiNorm && msa::dec_stream_eligible(m, k, n, epilogue)) return small_route(k);
+  return msa::dec_wide_eligible(m, k, n, ldx, ldy, ldr) ? Route::kWide : small_route(k);
+}
+
+// K splits on the wide kernel. With the norm: up to 16 rows the product and the residual in one launch, then
+// the norm; above, partials that the norm's kernel merges (8B down at 32 tokens: 22 us against 16.5, o 9.1
+// against 7.7; at 16 tokens 16.4 / 7.2 against 14.6 / 6.7 with a dearer merge). Without: a long K (8B down:
+// 24.0 us at 32 tokens in one launch, 34.2 at 64; about 20 and 23 with the merge's launch); o (K = 4096)
+// takes 10.0 / 13.5 us in one launch, which a merge would not beat.
+static int wide_splits(int64_t m, int64_t n, int64_t k, int epilogue) {
+  if (m <= 16 || epilogue == MSA_EPI_SILU_MUL) return 1;
+  if (epilogue != kEpiNorm && k < 8192) return 1;
+  return msa::dec_wide_splits(m, n, k);
+}
+
+static size_t partial_bytes(int splits, int64_t m, int64_t n) {
+  return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
+}
+
+static size_t skinny_workspace_size(int64_t m, int64_t n, int64_t k) {
   size_t best = 0;
   for (int epi = 0; epi < 3; ++epi) {
-    const msa::SkinnyPlan p = msa::plan_skinny(m, n, k, epi, 0);
-    const size_t b = p.k_split > 1 ? (size_t)p.k_split * m * n * sizeof(float) : 0;
+    const size_t b = partial_bytes(msa::plan_skinny(m, n, k, epi, 0).k_split, m, n);
     best = b > best ? b : best;
   }
   return best;
+}
+
+static size_t route_workspace_size(int64_t m, int64_t n, int64_t k, int epilogue) {
+  switch (route(m, n, k, k, n, n, epilogue)) {
+    case Route::kGemm:
+      return epilogue == kEpiNorm ? msa::gemm_workspace_size(m, n, k, MSA_EPI_NONE) : msa::gemm_plain_workspace_size(m, n, k);
+    case Route::kWide: return partial_bytes(wide_splits(m, n, k, epilogue), m, n);
+    case Route::kSkinny: return skinny_workspace_size(m, n, k);
+    default: return 0;
+  }
+}
+
+extern "C" size_t msa_int8_linear_workspace_size(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  size_t best = 0;
+  for (int epi = 0; epi < 3; ++epi) {
+    const size_t b = route_workspace_size(m, n, k, epi);
+    best = b > best ? b : best;
+  }
+  return best;
+}
+
+extern "C" size_t msa_int8_linear_add_rmsnorm_workspace_size(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  const size_t own = route_workspace_size(m, n, k, kEpiNorm), linear = route_workspace_size(m, n, k, MSA_EPI_RESIDUAL);
+  return own > linear ? own : linear;
+}
+
+extern "C" size_t msa_int8_linear_min_workspace_size(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  if (k % 64 == 0 && m >= kGemmMinRows) return msa::gemm_min_workspace_size(m, n, k);
+  return small_route(k) == Route::kSkinny ? skinny_workspace_size(m, n, k) : 0;
 }
 
 extern "C" int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
@@ -358,15 +404,14 @@ extern "C" int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t 
   if (ldy < out_cols) return fail(MSA_ERR_INVALID, "msa_int8_linear: ldy too small");
   if (epilogue == MSA_EPI_RESIDUAL && (!residual || ldr < n))
     return fail(MSA_ERR_INVALID, "msa_int8_linear: residual epilogue needs residual with ldr >= n");
-  if (takes_gemm(m, n, k))
+  const int64_t ldr_used = epilogue == MSA_EPI_RESIDUAL ? ldr : 0;
+  const Route r = route(m, n, k, ldx, ldy, ldr_used, epilogue);
+  if (r == Route::kGemm)
     return gemm_run(x, m, k, ldx, qweight, scale, n, y, ldy, epilogue, residual, ldr, workspace, workspace_bytes,
                     (hipStream_t)stream);
-  // Large weights: the streaming kernel (up to 16 tokens, K of 2048 / 4096, enough rows; inside the
-  // decode entry point below), else the wide kernel.
-  if (!dec_stream_eligible(m, k, n, epilogue) &&
-      dec_wide_eligible(m, k, n, ldx, ldy, epilogue == MSA_EPI_RESIDUAL ? ldr : 0)) {
-    const int splits = m > kWideDirectTokens && k >= kWideSplitMinK && epilogue != MSA_EPI_SILU_MUL ? dec_wide_splits(m, n, k) : 1;
-    if (splits > 1 && workspace && workspace_bytes >= (size_t)splits * m * n * sizeof(float) && aligned16(workspace)) {
+  if (r == Route::kWide) {
+    const int splits = wide_splits(m, n, k, epilogue);
+    if (splits > 1 && workspace && workspace_bytes >= partial_bytes(splits, m, n) && aligned16(workspace)) {
       rc = launch_dec_wide_partials(x, m, k, ldx, qweight, scale, n, splits, (float*)workspace, (hipStream_t)stream);
       if (rc != MSA_OK) return rc;
       return launch_splitk_epilogue((const float*)workspace, splits, m, n, y, ldy, epilogue, residual, ldr, (hipStream_t)stream);
@@ -375,10 +420,10 @@ extern "C" int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t 
   }
   // Decode-sized batches: the decode kernel (all of a workgroup's loads in flight at once, the same
   // rounding points); other K that fit the LDS activation tile: the token-split rows kernel.
-  if (dec_linear_supported(k))
+  if (r == Route::kDec)
     return msa_int8_linear_dec(x, ldx, m, nullptr, nullptr, 0, m, k, nullptr, 0.f, qweight, scale, n, epilogue, y, ldy,
                                residual, ldr, stream);
-  if (rows_fits(k))
+  if (r == Route::kRows)
     return msa_int8_linear_rows(x, ldx, m, k, nullptr, 0.f, qweight, scale, n, epilogue, y, ldy, residual, ldr, stream);
 
   SkinnyPlan p = plan_skinny(m, n, k, epilogue, 0);
@@ -440,7 +485,8 @@ extern "C" int msa_int8_linear_add_rmsnorm(const uint16_t* x, int64_t m, int64_t
     return fail(MSA_ERR_UNSUPPORTED,
                 "msa_int8_linear_add_rmsnorm: n must be a multiple of 8 and residual / norm_w / out 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  if (takes_gemm(m, n, k)) {
+  const Route r = route(m, n, k, ldx, n, n, kEpiNorm);
+  if (r == Route::kGemm) {
     const int splits = gemm_run_partials(x, m, k, ldx, qweight, scale, n, (float*)workspace, workspace_bytes, s);
     if (splits < 0) return MSA_ERR_LAUNCH;
     if (splits > 1) {
@@ -450,9 +496,9 @@ extern "C" int msa_int8_linear_add_rmsnorm(const uint16_t* x, int64_t m, int64_t
       return check_launch("msa_int8_linear_add_rmsnorm (merge + norm)");
     }
   }
-  if (m > kWideDirectTokens && dec_wide_eligible(m, k, n, ldx, n, n)) {
-    const int splits = dec_wide_splits(m, n, k);
-    if (splits > 1 && workspace && workspace_bytes >= (size_t)splits * m * n * sizeof(float) && aligned16(workspace)) {
+  if (r == Route::kWide) {
+    const int splits = wide_splits(m, n, k, kEpiNorm);
+    if (splits > 1 && workspace && workspace_bytes >= partial_bytes(splits, m, n) && aligned16(workspace)) {
       rc = launch_dec_wide_partials(x, m, k, ldx, qweight, scale, n, splits, (float*)workspace, s);
       if (rc != MSA_OK) return rc;
       launch_splitk_add_rmsnorm((const float*)workspace, splits, m, (int)n, residual, residual, norm_w, out, eps, s);

@@ -56,16 +56,21 @@ class _Workspaces:
         self._bufs: dict[tuple[str, int, int], Tensor] = {}
 
     def get(
-        self, kind: str, device: torch.device, nbytes: int, stream: torch.cuda.Stream | None = None
+        self, kind: str, device: torch.device, nbytes: int, stream: torch.cuda.Stream | None = None,
+        need: int | None = None,
     ) -> Tensor | None:
         """The buffer of ``kind`` for the device's current stream (or for ``stream``: allocated on
-        it, so that the allocator recycles it only behind that stream's work)."""
+        it, so that the allocator recycles it only behind that stream's work). ``need``: during a graph
+        capture what is already there will do if it holds that many bytes (None if 0 and nothing is)."""
         if nbytes == 0:
             return None
         idx = device.index if device.index is not None else torch.cuda.current_device()
         key = (kind, idx, stream.cuda_stream if stream is not None else _raw_stream(idx))
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
+            if need is not None and (buf.numel() if buf is not None else 0) >= need:
+                if torch.cuda.is_current_stream_capturing():
+                    return buf
             _check(
                 not torch.cuda.is_current_stream_capturing(),
                 f"workspace '{kind}' must be reserved before graph capture (need {nbytes} bytes)",
@@ -78,6 +83,14 @@ class _Workspaces:
 
     def reserve(self, kind: str, device: torch.device, nbytes: int) -> None:
         self.get(kind, device, nbytes)
+
+    def linear(self, call: str, device: torch.device, m: int, n: int, k: int) -> tuple[int | None, int]:
+        """(pointer, bytes) of the linears' scratch for ``call`` on an [m, k] x [n, k] product."""
+        nbytes = _native.query(call + "_workspace_size", m, n, k)
+        if not nbytes:
+            return None, 0
+        ws = self.get("linear", device, nbytes, None, _native.query("msa_int8_linear_min_workspace_size", m, n, k))
+        return (ws.data_ptr(), ws.numel()) if ws is not None else (None, 0)
 
 
 workspaces = _Workspaces()
@@ -147,10 +160,8 @@ def int8_linear(
         _check(r2.stride(-1) == 1 and r2.dtype == torch.bfloat16, "int8_linear: residual must be row-major bf16")
         pr, ldr = r2.data_ptr(), r2.stride(0)
     pw, nw = None, 0
-    ws_bytes = _native.query("msa_int8_linear_workspace_size", m, n, k) if m else 0
-    if ws_bytes:
-        ws = workspaces.get("linear", x.device, ws_bytes)
-        pw, nw = ws.data_ptr(), ws.numel()
+    if _native.query("msa_int8_linear_workspace_size", m, n, k):
+        pw, nw = workspaces.linear("msa_int8_linear", x.device, m, n, k)
     _native.call("msa_int8_linear", px, m, k, ldx, qweight.data_ptr(), scale.data_ptr(), n, out.data_ptr(), cols,
                  epilogue, pr, ldr, pw, nw, _raw_stream(dev))
     return out
@@ -175,11 +186,10 @@ def int8_linear_add_rmsnorm(
     if out is None:
         out = torch.empty_like(residual)
     _check(out.shape == (m, n) and out.is_contiguous(), "int8_linear_add_rmsnorm: bad out")
-    ws_bytes = _native.query("msa_int8_linear_workspace_size", m, n, k) if m else 0
-    ws = workspaces.get("linear", x.device, ws_bytes)
+    pw, nw = workspaces.linear("msa_int8_linear_add_rmsnorm", x.device, m, n, k)
     _native.call(
         "msa_int8_linear_add_rmsnorm", _ptr(x), m, k, x.stride(0), _ptr(qweight), _ptr(scale), n, _ptr(residual),
-        _ptr(norm_w), float(eps), _ptr(out), _ptr(ws), ws.numel() if ws is not None else 0, _stream(x),
+        _ptr(norm_w), float(eps), _ptr(out), pw, nw, _stream(x),
     )
     return out
 
@@ -362,12 +372,11 @@ def int8_linear_qk_norm_rope_cache(
     _check(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.shape == v_cache.shape, "caches")
     _check(k_cache.shape[-2:] == (kv_heads, head_dim), "cache layout [slots, KVH, D]")
     q = torch.empty(t, heads, head_dim, dtype=torch.bfloat16, device=x.device)
-    ws_bytes = _native.query("msa_int8_linear_workspace_size", t, qweight.shape[0], k) if t else 0
-    ws = workspaces.get("linear", x.device, ws_bytes)
+    pw, nw = workspaces.linear("msa_int8_gemm_qk_norm_rope_cache", x.device, t, qweight.shape[0], k)
     _native.call(
         "msa_int8_gemm_qk_norm_rope_cache", _ptr(x), t, k, x.stride(0), _ptr(qweight), _ptr(scale), heads, kv_heads,
         head_dim, _ptr(q_norm_w), _ptr(k_norm_w), float(eps), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(q),
-        _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], _ptr(ws), ws.numel() if ws is not None else 0, _stream(x),
+        _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], pw, nw, _stream(x),
     )
     return q
 

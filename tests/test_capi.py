@@ -110,3 +110,23 @@ def test_workspace_sizes():
     assert _native.query("msa_paged_attention_decode_workspace_size", 64, 16, 128, 1) == 0
     ws = _native.query("msa_paged_attention_decode_workspace_size", 64, 16, 128, 8)
     assert ws >= 64 * 16 * 8 * (128 + 2) * 4
+
+
+def test_linear_workspaces_follow_each_route():
+    """Each linear asks for the partials of its own route: the plain one for none where only the fused ones
+    split, and a capture has to hold no more than the splits without which the chip stays idle."""
+
+    def sizes(m, n, k):
+        return tuple(_native.query(f"msa_{c}_workspace_size", m, n, k)
+                     for c in ("int8_linear", "int8_linear_add_rmsnorm", "int8_linear_min"))
+
+    for m, n, k in [(27, 4096, 4096), (27, 6144, 4096), (64, 24576, 4096), (16, 4096, 12288), (768, 4096, 2048)]:
+        assert sizes(m, n, k)[0] == 0 == sizes(m, n, k)[2], (m, n, k)
+    assert sizes(27, 4096, 4096)[1] == 4 * 27 * 4096 * 4 and sizes(768, 4096, 2048)[1] == 2 * 768 * 4096 * 4
+    plain, normed, least = sizes(96, 4096, 4096)  # the GEMM's splits, which no call had to hold before 128 rows
+    assert plain == normed == 8 * 96 * 4096 * 4 and least == 0
+    assert sizes(256, 4096, 4096) == (4 * 256 * 4096 * 4,) * 3
+    assert sizes(27, 4096, 12288)[0] == 4 * 27 * 4096 * 4  # a long K
+    assert sizes(17, 512, 24576)[2] > 0  # (and few outputs)
+    qk = _native.query("msa_int8_gemm_qk_norm_rope_cache_workspace_size", 448, 6144, 4096)
+    assert qk == 2 * 448 * 6144 * 4 and _native.query("msa_int8_linear_min_workspace_size", 448, 6144, 4096) == 0

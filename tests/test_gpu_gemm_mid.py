@@ -34,7 +34,7 @@ def test_gemm_mid_splits(m, n, k, split):
     q, s = oi.quantize_int8(_bf16((n, k), seed=n + k, std=0.02))
     x, r, w = _bf16((m, k), seed=m), _bf16((m, n), seed=m + 1), _bf16((n,), seed=3, std=0.1) + 1
     xd, qd, sd = x.to(DEV), q.to(DEV), s.to(DEV)
-    assert (_native.query("msa_int8_linear_workspace_size", m, n, k) == 2 * m * n * 4) is split
+    assert (_native.query("msa_int8_linear_add_rmsnorm_workspace_size", m, n, k) == 2 * m * n * 4) is split
     y = kernels.int8_linear(xd, qd, sd)
     assert torch.equal(y, kernels.int8_linear(xd, qd, sd))
     exact = x.double() @ oi.dequantize(q, s, torch.bfloat16).double().T

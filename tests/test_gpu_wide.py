@@ -215,3 +215,51 @@ def test_small_model_rows_that_share_a_slot(monkeypatch):
     assert [r[0] for r in runner.execute(shared)] == runner.forward_greedy(runner.prepare(shared)).tolist()
     slots = runner.prepare(shared).attn.slot_mapping.cpu()
     assert rel_l2(runner.kv_caches[0][0].cpu()[slots], okv[0][0][slots]) < 1e-2
+
+
+@pytest.mark.parametrize("m,n,k,fused", [
+    (27, 4096, 4096, False),  # needs nothing
+    (27, 4096, 4096, True),  # partials where there is room for them
+    (96, 4096, 4096, False),
+    (96, 4096, 4096, True),
+])
+def test_capture_without_a_reserved_workspace(m, n, k, fused, monkeypatch):
+    """Linears whose splits are a gain and no need are captured on a stream that holds no workspace, and then
+    run unsplit: replayed three times with eager work between, within one bf16 rounding of float64."""
+    monkeypatch.setattr(kernels, "workspaces", kernels._Workspaces())
+    q, s = oi.quantize_int8(_bf16((n, k), seed=n + k, std=0.02))
+    x, r = _bf16((m, k), seed=m), _bf16((m, n), seed=m + 1)
+    xd, qd, sd, rd, res = x.to(DEV), q.to(DEV), s.to(DEV), r.to(DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    w = torch.ones(n, dtype=torch.bfloat16, device=DEV)
+
+    def run():
+        if not fused:
+            return kernels.int8_linear(xd, qd, sd)
+        res.copy_(rd)
+        kernels.int8_linear_add_rmsnorm(xd, qd, sd, res, w, 1e-6)
+        return res
+
+    eager = run().clone()  # (also loads the kernels)
+    exact = x.double() @ oi.dequantize(q, s, torch.bfloat16).double().T + (r.double() if fused else 0.0)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        out = run()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu(), exact) < 4e-3
+        xd.mul_(1.0)
+    assert rel_l2(out.cpu(), eager.cpu()) < 4e-3
+
+
+def test_capture_still_wants_the_needed_workspace(monkeypatch):
+    """Splits without which most of the chip is idle are still to be reserved: refused during a capture."""
+    q, s = oi.quantize_int8(_bf16((4096, 4096), seed=1, std=0.02))
+    x, qd, sd = _bf16((256, 4096), seed=2).to(DEV), q.to(DEV), s.to(DEV)
+    monkeypatch.setattr(kernels, "workspaces", kernels._Workspaces())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="must be reserved before graph capture"):
+        kernels.int8_linear(x, qd, sd)
+    kernels.workspaces._bufs["linear", 0, torch.cuda.current_stream().cuda_stream] = torch.empty(16 << 20, dtype=torch.uint8, device=DEV)
+    kernels.int8_linear(x, qd, sd)
