@@ -70,8 +70,8 @@ size_t msa_int8_linear_min_workspace_size(int64_t m, int64_t n, int64_t k);
  * Batches of 128 or more rows with k % 64 == 0 run msa_int8_gemm (its split-K partials in the
  * workspace). Smaller ones with k in {1024, 2048, 3072, 4096} run msa_int8_linear_dec (no norm prologue),
  * those whose activation tile fits in LDS (k % 64 == 0, k <= 4544) msa_int8_linear_rows (neither uses
- * the workspace), the rest a split-K kernel. Over weights of n * k >= 12 MiB with k % 64 == 0,
- * 65 or more rows run the GEMM and fewer a kernel that reads the weights once for all of them
+ * the workspace), the rest a split-K kernel. Over weights of n * k >= 12 MiB with k % 64 == 0, where it is
+ * faster, 65 or more rows run the GEMM and fewer a kernel that reads the weights once for all of them
  * (with a long k in splits whose partials meet in the workspace). Without a workspace nothing is split. */
 int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                     const uint16_t* scale, int64_t n, uint16_t* y, int64_t ldy, int epilogue,

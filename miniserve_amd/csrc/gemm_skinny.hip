@@ -313,12 +313,53 @@ void launch_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* w, uint16_t*
 
 // What a linear runs on: the LDS-tiled GEMM from 128 rows on; smaller batches the decode kernel (K it
 // supports), the rows kernel (activation tile within LDS) or the skinny split-K kernel. Over weights of
-// 12 MB and more two kernels that read the weights once for all rows take their place: the wide decode kernel
-// up to 64 rows, the GEMM from 65 (the kernels for small batches read such weights once per 16 tokens:
-// 8B-shaped gate_up at 96 tokens 132 us, the GEMM at 128 tokens 62).
+// 12 MB and more two kernels that read the weights once for all rows take their place where they measure
+// faster: the wide decode kernel up to 64 rows, the GEMM from 65. The lines below were drawn over widths of
+// 64 to 49152, weights of 12 to 200 MB and 1 to 127 rows, with each epilogue (us, the smaller kernel, then the
+// one that reads the weights once):
 constexpr int64_t kGemmMinRows = 128, kWideMaxRows = 64, kWideWeights = (int64_t)12 << 20;
 constexpr int kEpiNorm = -1;  // msa_int8_linear_add_rmsnorm: the residual, then the norm
 enum class Route { kGemm, kWide, kDec, kRows, kSkinny };
+
+// Up to 64 rows (one wavefront's 16-row tiles of the matrix, K dealt to eight wavefronts).
+static bool wide_pays(int64_t m, int64_t n, int64_t k, int epilogue) {
+  const bool silu = epilogue == MSA_EPI_SILU_MUL;
+  if (!msa::dec_linear_supported(k) && !rows_fits(k)) {
+    // Against split-K: enough row tiles that most CUs stream (1024 x 12288 at 16 rows 12.3, 15.4; 2048 x 12288
+    // 16.7, 16.2; 2368 x 28672 33.5, 35.5); with its own K splits nearly always (512 x 49152 at 17-64 rows
+    // 0.79-1.0 of the time, 256 x 49152 0.96-1.12).
+    if (!silu && m > 16) return n >= 512;
+    if (m > 16) return n >= 2560;  // (2048 x 6144 at 64 rows 14.9, 18.0)
+    return n >= 2560 || (n >= 2048 && k <= 16384);
+  }
+  // Against the decode and rows kernels.
+  if (silu) {
+    if (k < 512 || (k < 1024 && m > 16)) return false;  // short chains: 65536 x 256 at 16 rows 11.0, 12.7
+    if (k == 1024 && m <= 32) return n >= 20480;         // 16384 x 1024 at 16 rows 7.1, 9.2; 24576 11.8, 9.0
+    if (k == 2048 && m <= 32) return n <= 12288;         // 16384 x 2048 at 32 rows 11.3, 13.4; 8192 9.9, 8.2
+    if (k == 3072 && m <= 16) return n > 16384;          // 8192 x 3072 at 16 rows 9.2, 10.7; 21888 23.0, 21.4
+    return k > 2048 || n <= 40960;                       // 51200 x 2048 at 64 rows 59, 74
+  }
+  if (epilogue == MSA_EPI_NONE && k == 2048 && m > 16 && m <= 32) return n >= 10240 && n <= 40960;  // 6144: 7.0, 7.7
+  // The smallest weights in whole rounds of the smaller kernels: 4096 x 3072 at 1 / 16 rows 5.4 / 6.2, 5.9 / 6.9
+  // (3072 x 4096 with the residual 1.06 of the time, 8192 x 1536 1.05-1.10).
+  if (m <= 16 && (k == 3072 || k == 4096)) return n * k >= (int64_t)16 << 20;
+  if (m <= 16 && n % 4096 == 0 && !msa::dec_linear_supported(k)) return n * k >= (int64_t)14 << 20;
+  return true;
+}
+
+// 65 to 127 rows.
+static bool gemm_pays(int64_t m, int64_t n, int64_t k, int epilogue) {
+  const int64_t tiles = (n + 127) / 128;
+  if (epilogue == MSA_EPI_SILU_MUL)  // never split: 64 tiles 1.1-1.6 of the time, 67 and more at most equal
+    return tiles >= 66 && (k != 2048 || n >= 24576);  // (16384 x 2048 at 96 rows 25.3, 29.3)
+  // Too few workgroups: 1024 x 12288 (64) at 65 rows 20.2, 25.2; 1408 x 12288 (88) 0.83 of the time.
+  if (tiles * msa::gemm_splits(m, n, k, MSA_EPI_NONE) < 68) return false;
+  // A plain product of one pass of the decode kernel: 6144 / 8192 x 2048 at 96 rows 16.2 / 16.7, 20.2 / 22.2;
+  // 12288 x 1024 18.1, 20.0; 4096 x 4096 23.1, 20.8.
+  if (epilogue == MSA_EPI_NONE && msa::dec_linear_supported(k)) return n * k >= (int64_t)(k == 2048 ? 24 : 16) << 20;
+  return true;
+}
 
 static Route small_route(int64_t k) {
   return msa::dec_linear_supported(k) ? Route::kDec : rows_fits(k) ? Route::kRows : Route::kSkinny;
@@ -327,10 +368,10 @@ static Route small_route(int64_t k) {
 static Route route(int64_t m, int64_t n, int64_t k, int64_t ldx, int64_t ldy, int64_t ldr, int epilogue) {
   if (k % 64 == 0 && m >= kGemmMinRows) return Route::kGemm;
   if (k % 64 != 0 || n * k < kWideWeights) return small_route(k);
-  if (m > kWideMaxRows) return Route::kGemm;
+  if (m > kWideMaxRows) return gemm_pays(m, n, k, epilogue) ? Route::kGemm : small_route(k);
   // (the streaming kernel, up to 16 rows at K of 2048 / 4096, is inside the decode entry point)
   if (epilogue != kEpiNorm && msa::dec_stream_eligible(m, k, n, epilogue)) return small_route(k);
-  return msa::dec_wide_eligible(m, k, n, ldx, ldy, ldr) ? Route::kWide : small_route(k);
+  return msa::dec_wide_eligible(m, k, n, ldx, ldy, ldr) && wide_pays(m, n, k, epilogue) ? Route::kWide : small_route(k);
 }
 
 // K splits on the wide kernel. With the norm: up to 16 rows the product and the residual in one launch, then
@@ -340,7 +381,7 @@ static Route route(int64_t m, int64_t n, int64_t k, int64_t ldx, int64_t ldy, in
 // takes 10.0 / 13.5 us in one launch, which a merge would not beat.
 static int wide_splits(int64_t m, int64_t n, int64_t k, int epilogue) {
   if (m <= 16 || epilogue == MSA_EPI_SILU_MUL) return 1;
-  if (epilogue != kEpiNorm && k < 8192) return 1;
+  if (epilogue != kEpiNorm && k < 8192 && (k <= 4416 || n >= 2560)) return 1;
   return msa::dec_wide_splits(m, n, k);
 }
 

@@ -280,17 +280,25 @@ static int wide_launch(WideArgs a, int tiles, int splits, hipStream_t s) {
   return MSA_OK;
 }
 
-// Tiles per unit: the fewest 16-row tiles on the busiest CU, then the most tiles per unit (their
-// activations are read once per unit). Wide units need registers: six tiles up to 32 tokens (8B
-// gate_up at 32 tokens: 27.5 us with six, 30 with three, 33 with two), three otherwise.
-static int wide_nt(int tiles, int mt) {
-  const int widest = mt == 2 ? 6 : 3;
-  int best = 1, cost = 1 << 30;
-  for (int nt : {1, 2, 3, 6}) {
-    if (nt > widest) break;
-    const int units = (tiles + nt - 1) / nt, c = (units + kWideCUs - 1) / kWideCUs * nt;
-    if (c <= cost) {
-      best = nt;
+// Tiles per unit: rounds of units x tiles x the time of a tile in a unit of that width, which falls with the
+// width (a unit's activations are read, and its partial tiles summed, once). Measured per tile and round in
+// tenths of the widest unit's, K = 512 to 12288: one token tile 14, 12, 10 for 1, 2, 3 tiles (up to four
+// tokens 12, 12, 10, and over a long K three tiles gain nothing by themselves: 17088 x 6144 at one token
+// 28.2 us in ones, 30.2 in threes); two token tiles 13, 13, 12 for 1, 2, 3 and 10 for 6; three and four 13,
+// 12, 10. Over 800 shapes the pick is 0.3% from the best width (5% with equal times: 65536 x 256 at one
+// token 20.3 us in twos, 11.8 in threes). Wide units need registers: six tiles up to 32 tokens, three
+// otherwise.
+static int wide_nt(int tiles, int tokens, int k) {
+  constexpr int kTime[5][4] = {{12, 12, 10, 0}, {14, 12, 10, 0}, {13, 13, 12, 10}, {13, 12, 10, 0}, {13, 12, 10, 0}};
+  constexpr int kWidth[4] = {1, 2, 3, 6};
+  const int mt = (tokens + 15) / 16, row = tokens <= 4 ? 0 : mt;
+  int best = 1;
+  int64_t cost = (int64_t)1 << 62;
+  for (int i = 0; i < (mt == 2 ? 4 : 3); ++i) {
+    const int units = (tiles + kWidth[i] - 1) / kWidth[i];
+    const int64_t c = (int64_t)((units + kWideCUs - 1) / kWideCUs) * kWidth[i] * kTime[row][i];
+    if (c < cost || (c == cost && !(row == 0 && k >= 4096 && kWidth[i] == 3))) {
+      best = kWidth[i];
       cost = c;
     }
   }
@@ -301,7 +309,7 @@ static int wide_nt(int tiles, int mt) {
 // gained nothing: 8B gate_up at 32 tokens, six tiles, 27.5 us with one chunk in flight, 28.1 with two).
 template <int EPI>
 static int wide_dispatch(const WideArgs& a, int tiles, hipStream_t s) {
-  const int mt = (a.t + 15) / 16, nt = wide_nt(tiles, mt);
+  const int mt = (a.t + 15) / 16, nt = wide_nt(tiles, a.t, a.k);
   switch (mt) {
     case 1:
       if (nt == 1) return wide_launch<1, 1, 4, 2, EPI>(a, tiles, 1, s);

@@ -127,6 +127,6 @@ def test_linear_workspaces_follow_each_route():
     assert plain == normed == 8 * 96 * 4096 * 4 and least == 0
     assert sizes(256, 4096, 4096) == (4 * 256 * 4096 * 4,) * 3
     assert sizes(27, 4096, 12288)[0] == 4 * 27 * 4096 * 4  # a long K
-    assert sizes(17, 512, 24576)[2] > 0  # (and few outputs)
+    assert sizes(17, 512, 24576)[2] > 0  # (and few outputs: split before, too)
     qk = _native.query("msa_int8_gemm_qk_norm_rope_cache_workspace_size", 448, 6144, 4096)
     assert qk == 2 * 448 * 6144 * 4 and _native.query("msa_int8_linear_min_workspace_size", 448, 6144, 4096) == 0

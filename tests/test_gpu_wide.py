@@ -6,7 +6,8 @@ layers against the general layer loop.
 Same operands and rounding points as the oracle's bf16 product, float32 accumulation in another
 order: within rel-L2 2e-3 of the oracle and within one bf16 rounding (4e-3) of float64, as the other
 decode linears. Shapes take every unit width (1, 2, 3, 6 tiles) and token-tile count, ragged last
-units, K whose chunks do not deal evenly to the eight wavefronts, 1 and 64 tokens."""
+units, K whose chunks do not deal evenly to the eight wavefronts, 1 and 64 tokens. The kernel is taken
+where it is the faster one: shapes to either side of those lines, on whatever serves them."""
 
 from __future__ import annotations
 
@@ -35,7 +36,9 @@ WIDE_SHAPES = [  # (m, n, k)
     (1, 4090, 4160),  # one tile per unit, ragged n, 65 chunks
     (16, 3072, 4160),
     (5, 6150, 3136),  # two tiles, 49 chunks
-    (13, 12290, 1088),  # three tiles, 17 chunks
+    (13, 12290, 1088),  # 769 tiles in twos, 17 chunks
+    (3, 12280, 1088),  # three tiles
+    (13, 12280, 1088),
     (17, 4096, 3136),
     (32, 6144, 3136),
     (20, 12280, 1088),
@@ -46,8 +49,11 @@ WIDE_SHAPES = [  # (m, n, k)
     (49, 4090, 3136),
     (64, 6144, 3136),
     (63, 12290, 1088),
+    (40, 12280, 1088),  # three tiles
+    (60, 12280, 1088),
     (32, 2048, 8256),  # split K, merged by the epilogue kernel
     (64, 1600, 8256),
+    (40, 2048, 6208),
 ]
 
 
@@ -77,6 +83,28 @@ def test_wide_linear(m, n, k):
     gate, up = exact.to(torch.bfloat16).chunk(2, dim=-1)
     act = kernels.int8_linear(xd, qd, sd, kernels.EPI_SILU_MUL)
     assert rel_l2(act.cpu(), torch.nn.functional.silu(gate) * up) < 8e-3
+
+
+@pytest.mark.parametrize("m,n,k", [  # to either side of the rules that choose the kernel for large weights
+    (16, 1024, 12352), (16, 2560, 4992), (20, 448, 28160), (9, 4096, 3072), (24, 6144, 2048), (8, 8192, 1536),
+    (70, 1024, 12288), (70, 2048, 6144), (100, 8192, 2048), (127, 4096, 4096), (65, 8448, 1536),
+])
+def test_large_weight_routes(m, n, k):
+    """Every epilogue, whichever kernel it takes (they need not agree): within one bf16 rounding of float64
+    (two with the residual's own sum, three with silu(gate) * up)."""
+    q, s = oi.quantize_int8(_bf16((n, k), seed=n + k, std=0.02))
+    x, r, w = _bf16((m, k), seed=m), _bf16((m, n), seed=m + 1), _bf16((n,), seed=3, std=0.1) + 1
+    xd, qd, sd, rd = (t.to(DEV) for t in (x, q, s, r))
+    exact = x.double() @ oi.dequantize(q, s, torch.bfloat16).double().T
+    assert rel_l2(kernels.int8_linear(xd, qd, sd).cpu(), exact) < 4e-3
+    assert rel_l2(kernels.int8_linear(xd, qd, sd, kernels.EPI_RESIDUAL, residual=rd).cpu(), exact + r.double()) < 8e-3
+    gate, up = exact.chunk(2, dim=-1)
+    act = kernels.int8_linear(xd, qd, sd, kernels.EPI_SILU_MUL).cpu()
+    assert rel_l2(act, gate * torch.sigmoid(gate) * up) < 1.2e-2
+    res = rd.clone()
+    out = kernels.int8_linear_add_rmsnorm(xd, qd, sd, res, w.to(DEV), 1e-6)
+    assert rel_l2(res.cpu(), exact + r.double()) < 8e-3
+    assert rel_l2(out.cpu(), ol.rms_norm(res.cpu(), w, 1e-6)) < 2e-3
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 4096, 4160), (16, 2048, 8256), (17, 4096, 3136), (40, 2048, 8256), (64, 2568, 4992)])
