@@ -335,9 +335,14 @@ static bool wide_pays(int64_t m, int64_t n, int64_t k, int epilogue) {
   // Against the decode and rows kernels.
   if (silu) {
     if (k < 512 || (k < 1024 && m > 16)) return false;  // short chains: 65536 x 256 at 16 rows 11.0, 12.7
-    if (k == 1024 && m <= 32) return n >= 20480;         // 16384 x 1024 at 16 rows 7.1, 9.2; 24576 11.8, 9.0
-    if (k == 2048 && m <= 32) return n <= 12288;         // 16384 x 2048 at 32 rows 11.3, 13.4; 8192 9.9, 8.2
-    if (k == 3072 && m <= 16) return n > 16384;          // 8192 x 3072 at 16 rows 9.2, 10.7; 21888 23.0, 21.4
+    // The decode kernel's rounds of 16384 rows (8192 at K = 3072) against a time that falls evenly: it keeps
+    // the shapes that fill its last one. K = 1024 at 16 rows: 12288 6.6, 5.8; 16384 7.1, 8.7; 24576 11.8, 9.0;
+    // 49152 18.3, 14.8. K = 2048 at 32: 8192 9.9, 8.2; 16384 11.3, 13.4; 24576 19.5, 15.6; 32768 20.9, 23.4.
+    // K = 3072 at 16: 4096 8.0, 7.3; 8192 9.2, 10.7; 10944 15.4, 11.9; 16384 16.8, 17.5; 21888 23.0, 20.7.
+    const int64_t round = k == 3072 ? 8192 : 16384, rounds = (n + round - 1) / round;
+    if (k == 1024 && m <= 32) return n >= 40960 || 4 * n <= 3 * rounds * round;
+    if (k == 2048 && m <= 32) return n <= 40960 && 4 * n <= 3 * rounds * round;
+    if (k == 3072 && m <= 16) return n <= 4608 || (n > round && 10 * n <= 9 * rounds * round);
     return k > 2048 || n <= 40960;                       // 51200 x 2048 at 64 rows 59, 74
   }
   if (epilogue == MSA_EPI_NONE && k == 2048 && m > 16 && m <= 32) return n >= 10240 && n <= 40960;  // 6144: 7.0, 7.7

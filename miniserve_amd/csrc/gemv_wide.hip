@@ -283,21 +283,20 @@ static int wide_launch(WideArgs a, int tiles, int splits, hipStream_t s) {
 // Tiles per unit: rounds of units x tiles x the time of a tile in a unit of that width, which falls with the
 // width (a unit's activations are read, and its partial tiles summed, once). Measured per tile and round in
 // tenths of the widest unit's, K = 512 to 12288: one token tile 14, 12, 10 for 1, 2, 3 tiles (up to four
-// tokens 12, 12, 10, and over a long K three tiles gain nothing by themselves: 17088 x 6144 at one token
-// 28.2 us in ones, 30.2 in threes); two token tiles 13, 13, 12 for 1, 2, 3 and 10 for 6; three and four 13,
-// 12, 10. Over 800 shapes the pick is 0.3% from the best width (5% with equal times: 65536 x 256 at one
+// tokens 12, 12, 10, and over a long K, where HBM sets the pace, the same: 17088 x 6144 at one token 28.2
+// us in ones, 30.2 in threes); two token tiles 13, 13, 12 for 1, 2, 3 and 10 for 6; three and four 13, 12, 10. Over 800 shapes the pick is 0.3% from the best width (5% with equal times: 65536 x 256 at one
 // token 20.3 us in twos, 11.8 in threes). Wide units need registers: six tiles up to 32 tokens, three
 // otherwise.
 static int wide_nt(int tiles, int tokens, int k) {
-  constexpr int kTime[5][4] = {{12, 12, 10, 0}, {14, 12, 10, 0}, {13, 13, 12, 10}, {13, 12, 10, 0}, {13, 12, 10, 0}};
+  constexpr int kTime[6][4] = {{12, 12, 10, 0}, {14, 12, 10, 0}, {13, 13, 12, 10}, {13, 12, 10, 0}, {13, 12, 10, 0}, {10, 10, 10, 0}};
   constexpr int kWidth[4] = {1, 2, 3, 6};
-  const int mt = (tokens + 15) / 16, row = tokens <= 4 ? 0 : mt;
+  const int mt = (tokens + 15) / 16, row = tokens > 4 ? mt : k >= 4096 ? 5 : 0;
   int best = 1;
   int64_t cost = (int64_t)1 << 62;
   for (int i = 0; i < (mt == 2 ? 4 : 3); ++i) {
     const int units = (tiles + kWidth[i] - 1) / kWidth[i];
     const int64_t c = (int64_t)((units + kWideCUs - 1) / kWideCUs) * kWidth[i] * kTime[row][i];
-    if (c < cost || (c == cost && !(row == 0 && k >= 4096 && kWidth[i] == 3))) {
+    if (c <= cost) {
       best = kWidth[i];
       cost = c;
     }

@@ -51,21 +51,11 @@ class RotaryEmbedding(nn.Module):
         t = torch.arange(self.max_positions, dtype=torch.float32)
         freqs = torch.outer(t, inv_freq)
         emb = torch.cat((freqs, freqs), dim=-1)
-        both = torch.stack((emb.cos(), emb.sin())).to(device)
-        self.cos, self.sin = both[0], both[1]
+        self.cos = emb.cos().to(device)
+        self.sin = emb.sin().to(device)
 
     def forward(self, positions: Tensor) -> tuple[Tensor, Tensor]:
-        cos, sin = self.cos, self.sin
-        if (
-            cos.data_ptr() + cos.nbytes == sin.data_ptr()
-            and cos.untyped_storage().data_ptr() == sin.untyped_storage().data_ptr()
-            and cos.shape == sin.shape
-            and cos.is_contiguous()
-            and sin.is_contiguous()
-        ):  # as build() lays them out: one gather launch instead of two (3 us of a captured step)
-            rows = cos.as_strided((2, *cos.shape), (cos.numel(), *cos.stride()))[:, positions]
-            return rows[0], rows[1]
-        return cos[positions], sin[positions]
+        return self.cos[positions], self.sin[positions]
 
 
 class SwiGLU(nn.Module):
