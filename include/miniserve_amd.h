@@ -175,6 +175,14 @@ int msa_lm_head_logits(const uint16_t* hidden, int64_t ld_hidden, int64_t hidden
 
 /* ---- norms, RoPE and the KV-cache write (model/layers.py, model/qwen3.py) -------------------- */
 
+/* The embedding rows embed[ids[t]] (bf16 [vocab, hidden]) into x [tokens, hidden] and the rotary rows of
+ * positions[t] (float32 tables [max_positions, 128]; a negative position counts from the end, as in an
+ * index) into cos_rows / sin_rows [tokens, 128]: model/qwen3.py:147-148 in one launch. An id or position
+ * out of range aborts, as torch's own kernels do. */
+int msa_embed_rope_rows(const int64_t* ids, const int64_t* positions, int64_t tokens, const uint16_t* embed,
+                        int64_t vocab, int64_t hidden, const float* cos_table, const float* sin_table,
+                        int64_t max_positions, uint16_t* x, float* cos_rows, float* sin_rows, msa_stream_t stream);
+
 /* RMSNorm.forward (model/layers.py:18-22): out = bf16(w * bf16(x * rsqrt(mean(x^2) + eps))). */
 int msa_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* weight, uint16_t* out, int64_t ldo,
                 int64_t rows, int64_t dim, float eps, msa_stream_t stream);

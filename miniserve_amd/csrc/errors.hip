@@ -40,4 +40,4 @@ int allow_dynamic_lds(const void* kernel, int bytes, const char* what) {
 
 extern "C" const char* msa_last_error(void) { return msa::g_last_error.c_str(); }
 
-extern "C" int msa_abi_version(void) { return 21; }
+extern "C" int msa_abi_version(void) { return 22; }

@@ -97,6 +97,30 @@ __global__ __launch_bounds__(256) void rmsnorm_row_kernel(const uint16_t* __rest
   }
 }
 
+// The head of a decode step over gathered rows, one workgroup per token: its embedding row and the rotary
+// rows of its position (128 dims), as torch's embedding and indexing kernels give them, out-of-range
+// entries ending the process the same way. One launch where those take three (4 us each in a graph).
+__global__ __launch_bounds__(256) void embed_rope_rows_kernel(const int64_t* __restrict__ ids,
+                                                              const int64_t* __restrict__ positions,
+                                                              const uint16_t* __restrict__ embed, int64_t vocab, int hidden,
+                                                              const float* __restrict__ cos_t,
+                                                              const float* __restrict__ sin_t, int64_t max_pos,
+                                                              uint16_t* __restrict__ x, float* __restrict__ cos_r,
+                                                              float* __restrict__ sin_r) {
+  const int64_t t = blockIdx.x, id = ids[t];
+  int64_t pos = positions[t];
+  if (id < 0 || id >= vocab || pos < -max_pos || pos >= max_pos) __builtin_trap();
+  pos += pos < 0 ? max_pos : 0;
+  const int tid = threadIdx.x;
+  if (tid < 64) {  // 32 pieces of the cos row, then of the sin row
+    const float4* src = (const float4*)((tid < 32 ? cos_t : sin_t) + pos * 128);
+    ((float4*)((tid < 32 ? cos_r : sin_r) + t * 128))[tid & 31] = src[tid & 31];
+  }
+  const uint4* row = (const uint4*)(embed + id * hidden);
+  uint4* out = (uint4*)(x + t * hidden);
+  for (int i = tid; i < hidden / 8; i += 256) out[i] = row[i];
+}
+
 __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const uint16_t* resid_in, const uint16_t* __restrict__ delta,
                                                           uint16_t* resid_out, const uint16_t* __restrict__ w,
                                                           uint16_t* __restrict__ out, int64_t rows, int dim, float eps) {
@@ -449,6 +473,24 @@ __global__ __launch_bounds__(256) void reshape_and_cache_kernel(const uint16_t* 
 }
 
 }  // namespace msa
+
+extern "C" int msa_embed_rope_rows(const int64_t* ids, const int64_t* positions, int64_t tokens, const uint16_t* embed,
+                                   int64_t vocab, int64_t hidden, const float* cos_table, const float* sin_table,
+                                   int64_t max_positions, uint16_t* x, float* cos_rows, float* sin_rows,
+                                   msa_stream_t stream) {
+  using namespace msa;
+  if (tokens == 0) return MSA_OK;
+  if (!ids || !positions || !embed || !cos_table || !sin_table || !x || !cos_rows || !sin_rows)
+    return fail(MSA_ERR_INVALID, "msa_embed_rope_rows: null pointer");
+  if (tokens < 0 || tokens >= (1 << 24) || vocab <= 0 || hidden <= 0 || hidden > 0x7fffffff || max_positions <= 0)
+    return fail(MSA_ERR_INVALID, "msa_embed_rope_rows: bad shape");
+  if (hidden % 8 != 0 || !aligned16(embed) || !aligned16(cos_table) || !aligned16(sin_table) || !aligned16(x) ||
+      !aligned16(cos_rows) || !aligned16(sin_rows))
+    return fail(MSA_ERR_UNSUPPORTED, "msa_embed_rope_rows: hidden must be a multiple of 8, pointers 16-byte aligned");
+  hipLaunchKernelGGL(embed_rope_rows_kernel, dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream, ids, positions,
+                     embed, vocab, (int)hidden, cos_table, sin_table, max_positions, x, cos_rows, sin_rows);
+  return check_launch("msa_embed_rope_rows");
+}
 
 extern "C" int msa_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* weight, uint16_t* out, int64_t ldo,
                            int64_t rows, int64_t dim, float eps, msa_stream_t stream) {

@@ -271,6 +271,27 @@ def qk_norm_rope_cache_splitk(
 # ---- norms / RoPE / cache -------------------------------------------------------------------------
 
 
+def embed_rope_rows(
+    ids: Tensor, positions: Tensor, weight: Tensor, cos_table: Tensor, sin_table: Tensor
+) -> tuple[Tensor, Tensor, Tensor]:
+    """(weight[ids] [T, hidden], cos_table[positions], sin_table[positions] [T, 128]) in one launch
+    (model/qwen3.py:147-148); ids and positions out of range abort, as indexing on the GPU does."""
+    _on_gpu(ids, positions, weight, cos_table, sin_table)
+    for t in (ids, positions):
+        _check(t.dtype == torch.int64 and t.dim() == 1 and t.is_contiguous() and t.numel() == ids.numel(),
+               "embed_rope_rows: int64 [T] ids and positions")
+    _check(weight.dtype == torch.bfloat16 and weight.dim() == 2 and weight.is_contiguous(), "embed_rope_rows: weight bf16")
+    for c in (cos_table, sin_table):
+        _check(c.dtype == torch.float32 and c.is_contiguous() and c.shape == (cos_table.shape[0], 128),
+               "embed_rope_rows: float32 [positions, 128] tables")
+    t, (vocab, hidden) = ids.numel(), weight.shape
+    x = torch.empty(t, hidden, dtype=torch.bfloat16, device=ids.device)
+    rows = torch.empty(2, t, 128, dtype=torch.float32, device=ids.device)
+    _native.call("msa_embed_rope_rows", _ptr(ids), _ptr(positions), t, _ptr(weight), vocab, hidden, _ptr(cos_table),
+                 _ptr(sin_table), cos_table.shape[0], _ptr(x), rows.data_ptr(), rows[1].data_ptr(), _stream(ids))
+    return x, rows[0], rows[1]
+
+
 def rmsnorm(x: Tensor, weight: Tensor, eps: float, out: Tensor | None = None) -> Tensor:
     """RMSNorm over the last dim (model/layers.py:18-22)."""
     _on_gpu(x, weight)

@@ -291,3 +291,18 @@ def test_capture_still_wants_the_needed_workspace(monkeypatch):
         kernels.int8_linear(x, qd, sd)
     kernels.workspaces._bufs["linear", 0, torch.cuda.current_stream().cuda_stream] = torch.empty(16 << 20, dtype=torch.uint8, device=DEV)
     kernels.int8_linear(x, qd, sd)
+
+
+@pytest.mark.parametrize("t,hidden", [(1, 8), (3, 4096), (128, 8200)])
+def test_embed_rope_rows(t, hidden):
+    """The embedding and rotary gathers of the large-model decode step, bit for bit: one piece to several
+    pieces per thread, first and last entries, positions counted from the end."""
+    g = torch.Generator().manual_seed(hidden)
+    weight, cos, sin = _bf16((50, hidden), seed=t).to(DEV), torch.randn(70, 128, generator=g).to(DEV), torch.randn(70, 128, generator=g).to(DEV)
+    ids, pos = torch.randint(0, 50, (t,), generator=g), torch.randint(-70, 70, (t,), generator=g)
+    ids[0], pos[0], ids[-1], pos[-1] = 0, -70, 49, 69
+    ids, pos = ids.to(DEV), pos.to(DEV)
+    x, c, s = kernels.embed_rope_rows(ids, pos, weight, cos, sin)
+    assert torch.equal(x, weight[ids]) and torch.equal(c, cos[pos]) and torch.equal(s, sin[pos])
+    with pytest.raises(RuntimeError, match="ids and positions"):
+        kernels.embed_rope_rows(ids, pos[:-1] if t > 1 else torch.cat([pos, pos]), weight, cos, sin)
