@@ -47,7 +47,10 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict
   }
 }
 
-// RMSNorm of rows of 2048 to 2048 NV elements: a workgroup per row, the row in registers between the
+// A launch holds fewer than 2^32 work items: past 2^24 rows of 256 threads each, four rows share them.
+constexpr int64_t kRowNormMaxRows = (int64_t)1 << 24;
+
+// RMSNorm of rows of 2048 to 2048 NV elements, fewer than kRowNormMaxRows of them: a workgroup per row, the row in registers between the
 // sum of squares and the normalization, every load (row and norm weight) issued before the first
 // use. A wavefront per row (above) walks a 4096-wide row in eight dependent steps, twice: 5.8 us
 // after an 8B-shaped o projection of 1 to 27 rows, latency alone, against 2.4 here (2.1-2.3 back to
@@ -443,7 +446,7 @@ void launch_splitk_add_rmsnorm(const float* part, int k_split, int64_t rows, int
 void launch_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* w, uint16_t* out, int64_t ldo, int64_t rows, int dim,
                     float eps, hipStream_t s) {
   // (out may be x: a workgroup has read its row before it writes it)
-  if (dim >= 2048 && dim <= 8192) {
+  if (dim >= 2048 && dim <= 8192 && rows < kRowNormMaxRows) {
     const dim3 grid((unsigned)rows), block(256);
     if (dim == 2048) hipLaunchKernelGGL(rmsnorm_row_kernel<1>, grid, block, 0, s, x, ldx, w, out, ldo, dim, eps);
     else if (dim <= 4096) hipLaunchKernelGGL(rmsnorm_row_kernel<2>, grid, block, 0, s, x, ldx, w, out, ldo, dim, eps);

@@ -27,3 +27,23 @@ def test_rmsnorm_row_widths(rows, dim):
     out = kernels.rmsnorm(xd, w.to(DEV), 1e-6)
     assert rel_l2(out.cpu(), ol.rms_norm(x, w, 1e-6)) < 2e-3
     assert torch.equal(kernels.rmsnorm(xd, w.to(DEV), 1e-6, out=xd), out)  # in place
+
+
+def test_rmsnorm_more_rows_than_a_launch_of_row_workgroups_holds():
+    """2^24 + 3 rows of 2048 in place (69 GB): a workgroup of 256 per row would be past 2^32 work items. The
+    first, middle and last rows against the same rows alone."""
+    rows, dim = (1 << 24) + 3, 2048
+    if torch.cuda.mem_get_info()[0] < rows * dim * 2 + (4 << 30):
+        pytest.skip("needs 73 GB of free device memory")
+    w = (_bf16((dim,), seed=4, std=0.1) + 1).to(DEV)
+    sample = _bf16((64, dim), seed=6, std=2.0).to(DEV)
+    x = torch.full((rows, dim), 0.5, dtype=torch.bfloat16, device=DEV)
+    places = [0, 1 << 23, rows - 64]
+    for at in places:
+        x[at : at + 64] = sample
+    want = kernels.rmsnorm(sample, w, 1e-6)
+    kernels.rmsnorm(x, w, 1e-6, out=x)
+    for at in places:
+        assert rel_l2(x[at : at + 64].cpu(), want.cpu()) < 2e-3
+    del x
+    torch.cuda.empty_cache()
