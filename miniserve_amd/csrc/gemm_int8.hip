@@ -314,11 +314,17 @@ static int splits256(int64_t m, int64_t n, int64_t k, int64_t ldx) {
 // Splits on the 256 x 128 tiles where their number is past what splits128 would split but leaves
 // much of the chip idle in one unsplit round (96 to 128 tiles on 256 CUs): two splits fill 192 to 256
 // of them in one round. 8B-shaped o at 768 / 1024 tokens 52 / 57 us unsplit, 48 / 56 in two splits
-// and their merge (with the next norm 56 / 61 and 45 / 51); down 140 / 151, 106 / 123.
+// and their merge (with the next norm 56 / 61 and 45 / 51); down 140 / 151, 106 / 123; the 8B-shaped
+// qkv with its q/k norm at 385 to 512 tokens 50 / 42-44, at 40 query heads over K = 5120 60 / 54.
+// The kernel deals output-row blocks to the eight XCDs, so one round also needs the fullest XCD's
+// workgroups to fit its 32 CUs: rows of 20 blocks put three blocks, 36 workgroups at 1300 tokens, on
+// four of them, a second round (2560 x 9728: 103 us unsplit, 146 split; with the norm 112 and 145).
 static int splits_mid(int64_t m, int64_t n, int64_t k, int epilogue) {
   if (epilogue == MSA_EPI_SILU_MUL || m < 192) return 1;
-  const int64_t tiles = ((n + 127) / 128) * ((m + 255) / 256);
-  return tiles >= 96 && tiles <= 128 && gemm256_split_plan(m, n, k) == 2 ? 2 : 1;
+  const int64_t n_blocks = (n + 127) / 128, m_blocks = (m + 255) / 256;
+  const int64_t tiles = n_blocks * m_blocks;
+  if (tiles < 96 || tiles > 128 || (n_blocks + 7) / 8 * m_blocks * 2 > 32) return 1;
+  return gemm256_split_plan(m, n, k) == 2 ? 2 : 1;
 }
 
 // The split count of a GEMM that splits K (1: unsplit): the 256 x 128 tiles' plan where it applies

@@ -29,6 +29,8 @@ def _bf16(shape, seed, std=1.0):
     (1020, 3968, 2112, False),  # 124 tiles, K steps that do not halve
     (1025, 4096, 2048, False),  # 160 tiles
     (768, 4096, 1024, False),  # halves of 512
+    (1300, 2560, 2048, False),  # 120 tiles, of which four XCDs would take 36 workgroups
+    (1536, 2048, 2048, True),  # 96 tiles, 24 workgroups on each
 ])
 def test_gemm_mid_splits(m, n, k, split):
     q, s = oi.quantize_int8(_bf16((n, k), seed=n + k, std=0.02))
