@@ -421,11 +421,16 @@ int gemm256_run(int t, const uint16_t* x, int64_t m, int64_t k, int64_t ldx, con
     case 1: return launch_big_epi<192, 8, 2>(a, (int)blocks, epilogue, s);
     default:
       // One round of workgroups, and the residual epilogue: eight wavefronts (8B o at 1300 tokens 57.9 us,
-      // sixteen 60.1; at 2048 with the residual 71.8, 74.3; 0.6B gate_up-sized rows at 1000 tokens 19.0,
-      // 19.4). More rounds: sixteen (8B qkv at 1300 / 2048 tokens 80 / 97, eight 90 / 104).
+      // sixteen 60.1; at 2048 with the residual 71.8, 74.3). More rounds: sixteen (8B qkv at 1300 / 2048
+      // tokens 80 / 97, eight 90 / 104).
+      // silu * up: eight, but for a longer K on at most three quarters of the CUs (16384 x 5120 at 256 /
+      // 512 / 1300 / 4096 tokens, the first 128 tiles: eight 80 / 91 / 257 / 587, sixteen 70 / 95 / 268 / 581;
+      // 24576 x 4096 at 256, 192 tiles: 68, 66; 6144 x 1024 at 1000, 192 tiles: 19.5, 20.3).
       if (epilogue == MSA_EPI_RESIDUAL) return launch_big<128, 4, 2, MSA_EPI_RESIDUAL>(a, (int)blocks, s);
       if (epilogue == MSA_EPI_NONE && (int64_t)a.n_blocks * a.m_blocks <= 256)
         return launch_big<128, 4, 2, MSA_EPI_NONE>(a, (int)blocks, s);
+      if (epilogue == MSA_EPI_SILU_MUL && (a.k <= 2048 || (int64_t)a.n_blocks * a.m_blocks > 192))
+        return launch_big<128, 4, 2, MSA_EPI_SILU_MUL>(a, (int)blocks, s);
       return launch_big_epi<128, 4, 4>(a, (int)blocks, epilogue, s);
   }
 }

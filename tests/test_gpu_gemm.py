@@ -97,7 +97,11 @@ def test_gemm256_parity(m, n, k, ldx_pad):
     assert torch.equal(rd.cpu(), r + y.cpu())
 
 
-@pytest.mark.parametrize("m,half,k", [(2048, 3072, 1024), (2000, 2600, 128), (2304, 2560, 64)])
+@pytest.mark.parametrize("m,half,k", [
+    (2048, 3072, 1024), (2000, 2600, 128), (2304, 2560, 64),
+    (250, 8200, 2112),  # 129 tiles of 128 rows, a longer K: sixteen wavefronts
+    (1000, 3072, 1024), (1300, 8190, 64),  # eight: 192 tiles, 768
+])
 def test_gemm256_silu_mul(m, half, k):
     n = 2 * half
     q, s = oi.quantize_int8(_bf16((n, k), seed=m + half, std=0.02))
