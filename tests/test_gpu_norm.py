@@ -29,6 +29,19 @@ def test_rmsnorm_row_widths(rows, dim):
     assert torch.equal(kernels.rmsnorm(xd, w.to(DEV), 1e-6, out=xd), out)  # in place
 
 
+@pytest.mark.parametrize("dim", [1024, 2056, 4096, 8192, 8200])
+def test_rmsnorm_non_finite_rows(dim):
+    """An infinity (the row's factor is 0: NaN there, zeros elsewhere), a NaN, squares past float32, and
+    bf16's lowest values; the rows between as ever."""
+    x, w = _bf16((6, dim), seed=dim, std=2.0), _bf16((dim,), seed=4, std=0.1) + 1
+    x[0, dim - 1], x[2, 3], x[3, 0] = float("-inf"), float("nan"), 3e38
+    x[5] = torch.finfo(torch.bfloat16).min
+    out, want = kernels.rmsnorm(x.to(DEV), w.to(DEV), 1e-6).cpu(), ol.rms_norm(x, w, 1e-6)
+    assert torch.equal(out.isnan(), want.isnan()) and want[0].isnan().sum() == 1 and want[2].isnan().all()
+    assert torch.equal(out[[0, 3, 5]].nan_to_num(7.0), want[[0, 3, 5]].nan_to_num(7.0))
+    assert rel_l2(out[[1, 4]], want[[1, 4]]) < 2e-3
+
+
 def test_rmsnorm_more_rows_than_a_launch_of_row_workgroups_holds():
     """2^24 + 3 rows of 2048 in place (69 GB): a workgroup of 256 per row would be past 2^32 work items. The
     first, middle and last rows against the same rows alone."""

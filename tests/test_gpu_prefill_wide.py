@@ -84,3 +84,26 @@ def test_prefill_wide_rule(heads, kv_heads, seqs, wide):
     ref = torch.zeros_like(qd)
     kernels.paged_attention_prefill(qd, kd, vd, p.block_tables, p.seq_info, p.work[tile], 128**-0.5, ref, 16)
     assert rel_l2(out.cpu(), ref.cpu()) < 2e-3
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(8, 8), (16, 8), (32, 8)])
+def test_prefill_wide_past_4gb_of_cache(heads, kv_heads):
+    """A cache of 4 GB and more is addressed with 64-bit offsets: blocks at the end of such a pool give, bit
+    for bit, what the same blocks give in a small one. The rest of the large pool is not read."""
+    chunks, q, k, v, kc, vc = _case(heads, kv_heads, [(70, 150), (0, 40), (33, 129)], seed=heads)
+    slots = _slots(chunks)
+    kc[slots], vc[slots] = k, v
+    base = (1 << 32) // (16 * kv_heads * 128 * 2) + 4096 - kc.shape[0] // 16
+    tile, qd, outs = ab.PREFILL_TILE[heads // kv_heads], q.to(DEV), []
+    for at in (0, base):
+        big = [torch.empty(at * 16 + kc.shape[0], kv_heads, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        big[0][at * 16 :], big[1][at * 16 :] = kc.to(DEV), vc.to(DEV)
+        assert (big[0].numel() * 2 > 1 << 32) is (at > 0)
+        meta = ab.build_attention_metadata([ab.SeqChunk(f, n, c, [b + at for b in t]) for f, n, c, t in chunks],
+                                           (slots + at * 16).to(DEV), 16)
+        p, out = meta.prefill, torch.zeros_like(qd)
+        kernels.paged_attention_prefill(qd, *big, p.block_tables, p.seq_info, p.work[2 * tile], 128**-0.5, out, 16, True)
+        outs.append(out.cpu())
+        del big
+    assert torch.equal(*outs) and outs[0].abs().sum() > 0
+    torch.cuda.empty_cache()

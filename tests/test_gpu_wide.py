@@ -149,9 +149,44 @@ def test_wide_decode_layers_match_the_layer_loop(batch, monkeypatch):
     assert rel_l2(got[0][1].cpu(), got[1][1].cpu()) < 5e-3
 
 
+@pytest.mark.parametrize("m,n,k", [(5, 6150, 3136), (20, 12280, 1088), (64, 6144, 3136), (64, 1600, 8256)])
+def test_wide_non_finite_rows(m, n, k):
+    """Infinities and NaN in single rows: those rows as a float32 product has them (0 * inf is NaN), the
+    others bit for bit what they are without."""
+    q, s = oi.quantize_int8(_bf16((n, k), seed=n + k, std=0.02))
+    x = _bf16((m, k), seed=m)
+    clean = kernels.int8_linear(x.to(DEV), q.to(DEV), s.to(DEV)).cpu()
+    x[0, k - 1], x[2, 5], x[m - 1, 0] = float("inf"), float("nan"), float("-inf")
+    x[3, 7], x[3, 70] = float("inf"), float("-inf")
+    y = kernels.int8_linear(x.to(DEV), q.to(DEV), s.to(DEV)).cpu()
+    bad = sorted({0, 2, 3, m - 1})
+    want = (x[bad].float() @ oi.dequantize(q, s, torch.bfloat16).float().T).to(torch.bfloat16)
+    assert not want.isfinite().any() and (want == float("inf")).any() and want.isnan().any()
+    assert torch.equal(y[bad].nan_to_num(7.0), want.nan_to_num(7.0)) and torch.equal(y[bad].isnan(), want.isnan())
+    keep = [i for i in range(m) if i not in bad]
+    assert torch.equal(y[keep], clean[keep])
+
+
 # One layer whose linears all reach WIDE_MIN_WEIGHTS and whose down projection is past the token-split kernels.
 LARGE = {**workloads.QWEN3_8B, "num_hidden_layers": 1, "intermediate_size": 4608, "vocab_size": 512,
          "tie_word_embeddings": True}
+
+
+@pytest.mark.parametrize("batch", [3, 20])
+@pytest.mark.parametrize("hidden,heads,kv_heads", [(3584, 32, 32), (3584, 32, 16), (4096, 32, 4), (3584, 32, 8)])
+def test_wide_decode_layers_of_other_shapes(hidden, heads, kv_heads, batch, monkeypatch):
+    """Every group size, and hidden sizes that the decode kernel does not take (3584: the norms then run
+    with the o and down projections for few tokens too), against the general loop at the bars above."""
+    cfg = {**LARGE, "hidden_size": hidden, "num_attention_heads": heads, "num_key_value_heads": kv_heads}
+    runner, sched = _decode_step(cfg, batch)
+    inp = runner.prepare(sched)
+    assert not runner.model._token_split_ok(batch) and runner.model._wide_decode_ok(batch, inp.attn)
+    got = _forward(runner, inp, 4 * batch)
+    monkeypatch.setattr(type(runner.model), "_wide_decode_ok", lambda self, tokens, meta: False)
+    want = _forward(runner, inp, 4 * batch)
+    assert rel_l2(got[0], want[0]) < 2e-2 and rel_l2(got[1], want[1]) < 5e-3
+    slots = inp.attn.slot_mapping.cpu()
+    assert rel_l2(got[1][0, :, slots], want[1][0, :, slots]) < 1e-2
 
 
 def _decode_step(cfg, batch, blocks_each=4, seed=5):
