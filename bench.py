@@ -232,7 +232,7 @@ def time_layer_attention(runner, sched, cfg, fused: bool = True) -> tuple[float,
     d = inp.attn.decode
     dev = runner.device
     heads, kvh, dim = cfg["num_attention_heads"], cfg["num_key_value_heads"], cfg["head_dim"]
-    ptok, parts = kernels.decode_splits(d.num_seqs, kvh, d.block_tables.shape[1], heads // kvh, d.split_context)
+    ptok, parts = kernels.decode_plan(d.num_seqs, kvh, d.block_tables.shape[1], heads // kvh, d.split_context)
     g = torch.Generator(device=dev).manual_seed(5)
     out = torch.empty(len(sched), heads, dim, dtype=torch.bfloat16, device=dev)
     caches = runner.kv_caches
@@ -558,7 +558,7 @@ def time_config2(q, kv, meta, ctx) -> tuple[float, int, str]:
 
     heads, kvh, dim = q.shape[1], kv.shape[3], q.shape[2]
     d = meta.decode
-    ptok, parts = kernels.decode_splits(d.num_seqs, kvh, d.block_tables.shape[1], heads // kvh, d.split_context)
+    ptok, parts = kernels.decode_plan(d.num_seqs, kvh, d.block_tables.shape[1], heads // kvh, d.split_context)
     out_t = torch.empty_like(q)
 
     def kern(i):
@@ -635,7 +635,7 @@ def bench_long_context(args) -> dict:
                                                                             strict=True))]
         meta = hb.build_attention_metadata(chunks, slots, 16)
         d = meta.decode
-        ptok, parts = kernels.decode_splits(nseq, kvh, d.block_tables.shape[1], heads // kvh, 32768)
+        ptok, parts = kernels.decode_plan(nseq, kvh, d.block_tables.shape[1], heads // kvh, 32768)
         out_t = torch.empty_like(q)
 
         def kern(i, kv=kv, q=q, d=d, ptok=ptok, parts=parts, out_t=out_t):
