@@ -82,7 +82,7 @@ int msa_int8_linear(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const 
  * 128-token x 128-row tiles; each int8 weight tile is dequantized once per token tile to the same
  * bf16(q * s) value as the reference, float32 accumulation, then the epilogue of msa_int8_linear
  * (MSA_EPI_RESIDUAL may write y in place over residual). k % 64 == 0; x, qweight 16-byte aligned.
- * msa_int8_linear routes batches of 128 or more rows here (65 or more over large weights). */
+ * msa_int8_linear routes batches of 128 or more rows here (65 or more over large weights, where it is faster). */
 int msa_int8_gemm(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                   const uint16_t* scale, int64_t n, uint16_t* y, int64_t ldy, int epilogue,
                   const uint16_t* residual, int64_t ldr, msa_stream_t stream);
@@ -201,9 +201,9 @@ int msa_add_rmsnorm(const uint16_t* residual, const uint16_t* delta, uint16_t* r
  * model/layers.py:18-22): residual = bf16(residual + bf16(x @ bf16(q * s)^T)) in place, then
  * out = RMSNorm(residual) with norm_w, eps. x [m, k] (row stride ldx), qweight [n, k], residual and
  * out [m, n] contiguous, n % 8 == 0, 16-byte aligned. When the GEMM splits K (128+ rows, few
- * output tiles) the float32 partials go to workspace (msa_int8_linear_workspace_size bytes) and
- * one kernel merges them, adds the residual and normalizes -- the split-K merge and the norm
- * launch of the unfused sequence become one pass. */
+ * output tiles) the float32 partials go to workspace (msa_int8_linear_add_rmsnorm_workspace_size
+ * bytes) and one kernel merges them, adds the residual and normalizes -- the split-K merge and the
+ * norm launch of the unfused sequence become one pass. */
 int msa_int8_linear_add_rmsnorm(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                                 const uint16_t* scale, int64_t n, uint16_t* residual, const uint16_t* norm_w,
                                 float eps, uint16_t* out, void* workspace, size_t workspace_bytes,
@@ -334,7 +334,7 @@ int msa_paged_attention_decode_qkv_rows(const uint16_t* qkv, int64_t ldqkv, cons
  * slot_mapping[t] (slots outside [0, num_slots) are skipped). cos / sin are [m, 128] float32.
  * head_dim must be 128; x, the norm weights, cos / sin, q_out and the caches 16-byte aligned.
  * When the GEMM would split K (few output tiles) and the workspace holds
- * msa_int8_linear_workspace_size(m, n, k) bytes, the split-K partials go to the workspace and
+ * msa_int8_gemm_qk_norm_rope_cache_workspace_size(m, n, k) bytes, the split-K partials go there and
  * msa_qk_norm_rope_cache_splitk sums them (the same values); otherwise the epilogue does it. */
 int msa_int8_gemm_qk_norm_rope_cache(const uint16_t* x, int64_t m, int64_t k, int64_t ldx, const int8_t* qweight,
                                      const uint16_t* scale, int heads, int kv_heads, int head_dim,

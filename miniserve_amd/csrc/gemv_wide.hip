@@ -231,8 +231,8 @@ __global__ __launch_bounds__(64 * W, W / 4 * OCC) void dec_wide_kernel(WideArgs 
 
 // ---- host side ----------------------------------------------------------------------------------
 
-// Weight matrices of at least this many bytes come here: from there on a launch streams for longer
-// than it takes to start. 8B-shaped o [4096 x 4096] at 27 tokens: 12.0 us on the decode kernel (which
+// Weight matrices of at least this many bytes come here where wide_pays: from there on a launch streams
+// for longer than it takes to start. 8B-shaped o [4096 x 4096] at 27 tokens: 12.0 us on the decode kernel (which
 // reads the weights once per 16 tokens), 9.1 here; down [4096 x 12288] at 1 / 27 tokens 42.6 / 48.6
 // us on the split-K kernel for small batches, 13.1 / 22.2 here; gate_up [24576 x 4096] at 27 / 64
 // tokens 48 / 95 us, 27.5 / 38 here. Below (the 0.6B shapes, 1-6 MB) the decode kernel, which has
