@@ -260,9 +260,10 @@ class Qwen3ForCausalLM(nn.Module):
         cfg = self.cfg
         t = input_ids.numel()
         ids = input_ids if input_ids.dtype == torch.int64 and input_ids.is_contiguous() else input_ids.long().contiguous()
-        pos = positions if positions.dtype == torch.int64 and positions.is_contiguous() else positions.long().contiguous()
+        pos = positions.to(ids.device, torch.int64).contiguous()
         # x: the residual stream, updated in place
-        x, cos, sin = kernels.embed_rope_rows(ids, pos, self.embed_tokens.weight, self.rotary.cos, self.rotary.sin)
+        x, cos, sin = kernels.embed_rope_rows(ids, pos, self.embed_tokens.weight.contiguous(), self.rotary.cos,
+                                              self.rotary.sin)
         inside = t <= kernels.STREAM_MAX_TOKENS and kernels.dec_supported(cfg.hidden_size)
         first = self.layers[0].input_layernorm
         h = x if inside else kernels.rmsnorm(x, first.weight, first.eps)

@@ -220,6 +220,8 @@ def test_wide_decode_layers_rotate_by_the_given_positions(batch, monkeypatch):
     positions = (inp.positions * 3 + 41) % 256
     assert not runner.model._token_split_ok(batch) and runner.model._wide_decode_ok(batch, inp.attn)
     own, got = _forward(runner, inp, 4 * batch), _forward(runner, inp, 4 * batch, positions)
+    other = _forward(runner, inp, 4 * batch, positions.int().cpu())  # as indexing takes them
+    assert torch.equal(other[0], got[0]) and torch.equal(other[1], got[1])
     monkeypatch.setattr(type(runner.model), "_wide_decode_ok", lambda self, tokens, meta: False)
     want = _forward(runner, inp, 4 * batch, positions)
     assert rel_l2(got[0], want[0]) < 2e-2 and rel_l2(got[1], want[1]) < 5e-3
