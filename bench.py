@@ -113,7 +113,7 @@ def decode_kernel_name(group: int, partition_tokens: int, fused: bool) -> str:
     fused decode-step entry point always four wavefronts; the plain one eight for splits of 1024+
     keys when the group has at most two query heads."""
     waves = 8 if (not fused and group <= 2 and partition_tokens >= 1024) else 4
-    return f"paged_decode_kernel<{group}, {waves}, {'true' if fused else 'false'}>"
+    return f"paged_decode_kernel<{group}, {waves}, {'true' if fused else 'false'}, false>"
 
 
 def dec_linear_name(m: int, k: int, epilogue: int, norm: bool) -> str:
